@@ -42,9 +42,6 @@ Context::Context(const tt_params& p) : prm(p) {
     TT_HIP(hipEventCreateWithFlags(&look_ev, hipEventDisableTiming));
     g = make_grid(p.nelx, p.nely, p.nelz, p.xc[1] - p.xc[0], p.xc[3] - p.xc[2], p.xc[5] - p.xc[4]);
     const long nd = g.nd, nn = g.nn, nel = g.nel;
-    const long apply_blocks = 8 * (((long)((g.nx + 7) / 8) * ((g.ny + 7) / 8) * ((g.nz + 1) / 2) + 7) / 8);
-    red.init((int)std::max<long>({apply_blocks, (nel + 255) / 256, (nn + 255) / 256, 2048}));
-
     // Newmark constants (LinearElasticity.cc:185-207)
     dt = p.t1 / p.nsteps;
     if (p.ti == 0) {
@@ -63,23 +60,9 @@ Context::Context(const tt_params& p) : prm(p) {
 
     hex8_stiffness(g.hx, g.hy, g.hz, p.nu, KE);
     hex8_mass(g.hx, g.hy, g.hz, M8);
-    float ke32[576], m832[64];
-    for (int i = 0; i < 576; i++) ke32[i] = (float)KE[i];
-    for (int i = 0; i < 64; i++) m832[i] = (float)M8[i];
-    KE64d.alloc(576); M864d.alloc(64); KE32d.alloc(576); M832d.alloc(64);
+    KE64d.alloc(576); M864d.alloc(64);
     TT_HIP(hipMemcpy(KE64d.p, KE, sizeof(KE), hipMemcpyHostToDevice));
     TT_HIP(hipMemcpy(M864d.p, M8, sizeof(M8), hipMemcpyHostToDevice));
-    TT_HIP(hipMemcpy(KE32d.p, ke32, sizeof(ke32), hipMemcpyHostToDevice));
-    TT_HIP(hipMemcpy(M832d.p, m832, sizeof(m832), hipMemcpyHostToDevice));
-    {
-        double af64[18 * 64];
-        float af32[AF32_WORDS];
-        mfma_fragments(KE, M8, af64, af32, reinterpret_cast<uint32_t*>(af32 + 18 * 64), afh_scale);
-        AF64d.alloc(18 * 64);
-        AF32d.alloc(AF32_WORDS);
-        TT_HIP(hipMemcpy(AF64d.p, af64, sizeof(af64), hipMemcpyHostToDevice));
-        TT_HIP(hipMemcpy(AF32d.p, af32, sizeof(af32), hipMemcpyHostToDevice));
-    }
 
     // Dirichlet mask, load location, optimisation region (index form of the reference's
     // coordinate tests with tolerance 0.05 h, LinearElasticity.cc:222-335, 540-575, 616-675)
@@ -108,15 +91,10 @@ Context::Context(const tt_params& p) : prm(p) {
             }
     mask.alloc(nn);
     TT_HIP(hipMemcpy(mask.p, m.data(), nn, hipMemcpyHostToDevice));
-    {
-        std::vector<uint8_t> f;
-        tile_bc_flags(g, m, 4, f);
-        tbc4.alloc(f.size());
-        TT_HIP(hipMemcpy(tbc4.p, f.data(), f.size(), hipMemcpyHostToDevice));
-        tile_bc_flags(g, m, 2, f);
-        tbc2.alloc(f.size());
-        TT_HIP(hipMemcpy(tbc2.p, f.data(), f.size(), hipMemcpyHostToDevice));
-    }
+    split.build(g, m);
+    // (an apply writes one partial per block; coarser levels have fewer nodes and no more blocks)
+    const long apply_blocks = 8 * ((std::max(split.s32.plan.ntiles(), split.s64.plan.ntiles()) + 7) / 8);
+    red.init((int)std::max<long>({apply_blocks, (nel + 255) / 256, (nn + 255) / 256, 2048}));
     F.alloc(nd);
     TT_HIP(hipMemcpy(F.p, Fhost.data(), nd * 8, hipMemcpyHostToDevice));
     std::vector<double> Ph(nel);
@@ -151,19 +129,12 @@ Context::Context(const tt_params& p) : prm(p) {
     op_fine64.mf = mf.p;
     op_fine64.KE64 = KE64d.p;
     op_fine64.M864 = M864d.p;
-    op_fine64.KE32 = KE32d.p;
-    op_fine64.M832 = M832d.p;
-    op_fine64.AF64 = AF64d.p;
-    op_fine64.AF32 = AF32d.p;
-    op_fine64.AFH = reinterpret_cast<const uint32_t*>(AF32d.p + 18 * 64);
-    op_fine64.hs[0] = afh_scale[0];
-    op_fine64.hs[1] = afh_scale[1];
     op_fine64.mask = mask.p;
-    op_fine64.tbc4 = tbc4.p;
-    op_fine64.tbc2 = tbc2.p;
-    build_batch_tables(g, btab);
-    op_fine64.tab4 = btab.t4;
-    op_fine64.tab2 = btab.t2;
+    op_fine64.split32 = split.s32;
+    op_fine64.split64 = split.s64;
+    upload_modes(KE, M8, modes64, modes32);
+    op_fine64.modes64 = modes64.p;
+    op_fine64.modes32 = modes32.p;
 
     mg.build(this, p.nlvls, p.precision == TT_PREC_MIXED, p.cheb_degree);
 

@@ -1,0 +1,90 @@
+// Tile splits of the column kernels (tt_apply_cols.inc).  Host code, run once per grid.
+#include <algorithm>
+#include <cmath>
+
+#include "tt_internal.h"
+
+namespace tt {
+
+// Tile split of one grid.  A block's planes pass one after the other, so its time is (planes + 2) times the time of a
+// plane, which is bound by latency while few blocks share a CU and by issue beyond.  Measured on 128x64x64 (256 CUs;
+// us per plane with 1, 2, 3 blocks per CU): FP32 0.96, 1.19, 1.6; FP64 1.27, 1.87, and no third block (registers).  The
+// columns of a tile (cx x cy <= 256 threads, one halo row and column) and the planes per block trade halo work
+// against blocks in flight: the split with the least modelled time is taken.
+ColPlan make_col_plan(const Grid& g, bool fp64) {
+    constexpr double cus = 256.0;
+    const int resident = fp64 ? 2 : 3;                // blocks per CU
+    const double lat = fp64 ? 1.27 : 1.0, iss = fp64 ? 0.93 : 0.54;  // us per plane: alone; per block sharing the CU
+    auto plane = [&](int r) { return std::max(lat, iss * r); };
+    ColPlan best{};
+    double cost = 1e300;
+    for (int cx = std::min(3, g.nx + 1); cx <= std::min(64, g.nx + 1); cx++) {
+        const int bx = cx - 1, tx = (g.nx + bx - 1) / bx;
+        const int cymax = std::min({256 / cx, 1024 / (3 * (cx + 1)) - 1, g.ny + 1});
+        for (int cy = std::min(3, cymax); cy <= cymax; cy++) {
+            const int by = cy - 1, ty = (g.ny + by - 1) / by;
+            for (int nk = 1, last = 0; nk <= g.nz; nk++) {
+                const int tz = (g.nz + nk - 1) / nk;
+                if (tz == last) continue;
+                last = tz;
+                const double nt = (double)tx * ty * tz, per = nt / cus;
+                const int r = (int)std::ceil(per);
+                // (between splits of one modelled time, the one with fewer blocks)
+                const double c = 1e-4 * nt + (r <= resident ? (nk + 2) * plane(r)
+                                                            : (nk + 2) * plane(resident) * (0.5 + per / resident));
+                if (c < cost) {
+                    cost = c;
+                    best = ColPlan{cx, bx, by, tx, ty, tz};
+                }
+            }
+        }
+    }
+    return best;
+}
+
+void col_bc_flags(const Grid& g, const ColPlan& p, const std::vector<uint8_t>& mask, std::vector<uint8_t>& f) {
+    f.assign(p.ntiles(), 0);
+    // tile a (b nodes per tile) stages nodes a b - 1 .. (a + 1) b
+    auto range = [](int i, int b, int nt, int& lo, int& hi) {
+        lo = std::max(0, (i + b - 1) / b - 1);
+        hi = std::min(nt - 1, (i + 1) / b);
+    };
+    std::vector<int> zlo(g.nz, 0), zhi(g.nz, 0);
+    for (int k = 0; k < g.nz; k++) {
+        int lo = -1, hi = -1;
+        for (int c = 0; c < p.tz; c++) {
+            const int k0 = (int)((long)c * g.nz / p.tz), k1 = (int)((long)(c + 1) * g.nz / p.tz);
+            if (k >= k0 - 1 && k <= k1) {
+                if (lo < 0) lo = c;
+                hi = c;
+            }
+        }
+        zlo[k] = lo;
+        zhi[k] = hi;
+    }
+    for (int k = 0; k < g.nz; k++)
+        for (int j = 0; j < g.ny; j++)
+            for (int i = 0; i < g.nx; i++) {
+                if (!mask[i + (size_t)g.nx * (j + (size_t)g.ny * k)]) continue;
+                int a0, a1, b0, b1;
+                range(i, p.bx, p.tx, a0, a1);
+                range(j, p.by, p.ty, b0, b1);
+                for (int c = zlo[k]; c <= zhi[k]; c++)
+                    for (int b = b0; b <= b1; b++)
+                        for (int a = a0; a <= a1; a++) f[a + (size_t)p.tx * (b + (size_t)p.ty * c)] = 1;
+            }
+}
+
+void ColSplitStore::build(const Grid& g, const std::vector<uint8_t>& mask) {
+    for (int d = 0; d < 2; d++) {
+        ColSplit& s = d ? s64 : s32;
+        s.plan = make_col_plan(g, d != 0);
+        std::vector<uint8_t> f;
+        col_bc_flags(g, s.plan, mask, f);
+        flags[d].alloc(f.size());
+        TT_HIP(hipMemcpy(flags[d].p, f.data(), f.size(), hipMemcpyHostToDevice));
+        s.bc = flags[d].p;
+    }
+}
+
+}  // namespace tt

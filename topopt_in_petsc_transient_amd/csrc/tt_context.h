@@ -19,13 +19,14 @@ struct Context;
 struct MGLevel {
     Grid g;
     bool fp64 = true;                  // precision of this level's vectors and element matrices
-    DBuf<uint8_t> mask, tbc4, tbc2;    // node mask; per-tile flags of clamped nodes (8x8x4, 8x8x2 tiles)
-    BatchTabStore btab;                // element batch tables of the tiles (full and edge tiles)
+    DBuf<uint8_t> mask;                // node mask
+    ColSplitStore split;               // tile splits of the operator kernels
     DBuf<double> kf64, mf64;           // FP64 coefficients (coarse levels: averages of children)
     DBuf<float> kf32, mf32;            // mixed mode, finest level
     DBuf<bf16_t> kfbf, mfbf;           // mixed mode, coarse levels
-    DBuf<double> KE64, M864, AF64;
-    DBuf<float> KE32, M832, AF32;
+    DBuf<double> KE64, M864;
+    DBuf<ModeConst<double>> modes64;
+    DBuf<ModeConst<float>> modes32;
     OpLevel op{};
     DBuf<char> b, x, x2, r, d, d2, dinv;  // level vectors (element size = 8 or 4 bytes)
     double lmax = 1.0;
@@ -105,13 +106,13 @@ struct Context {
     DBuf<double> xphys, kf, mf, dkf, dmf, P, Pkf, Pmf;
     DBuf<double> rcnt;  // per node: sum of region indicators of the adjacent elements
     DBuf<double> F;     // load location vector (3 nn)
-    DBuf<uint8_t> mask, tbc4, tbc2;
-    BatchTabStore btab;
+    DBuf<uint8_t> mask;
+    ColSplitStore split;
     std::vector<double> Fhost;
     OpLevel op_fine64{};  // FP64 fine operator view (for FCG residuals)
-    DBuf<double> KE64d, M864d, AF64d;
-    DBuf<float> KE32d, M832d, AF32d;
-    float afh_scale[2];
+    DBuf<double> KE64d, M864d;
+    DBuf<ModeConst<double>> modes64;
+    DBuf<ModeConst<float>> modes32;
     DBuf<float> kf32, mf32;  // FP32 fine coefficients for the FP32 microbenchmark apply
     bool density_set = false;
     bool initial_done = false;

@@ -93,6 +93,59 @@ void hex8_mass(double hx, double hy, double hz, double* m8) {
             }
 }
 
+// K~ = H K H' / 64 and M~ = H M H' / 64 with the 8 x 8 sign matrix H (per component), so that K = H' K~ H.  Mode
+// m = a + 2 b + 4 c has sign (2 i - 1) along each direction whose bit is set.  Box elements are symmetric under
+// the three reflections: K~ has no entries besides the blocks kept here, and M~ is diagonal, with a third per
+// odd direction.  (Summed in extended precision: the constants carry the matrices' rounding only.)
+void hex8_modes(const double* ke, const double* m8, ModeConst<double>& mc) {
+    double H[8][8];
+    for (int m = 0; m < 8; m++)
+        for (int a = 0; a < 8; a++)
+            H[m][a] = ((m & 1) ? kSx[a] : 1) * ((m & 2) ? kSy[a] : 1) * ((m & 4) ? kSz[a] : 1);
+    auto K = [&](int ci, int mi, int cj, int mj) {
+        long double s = 0.0L;
+        for (int a = 0; a < 8; a++)
+            for (int b = 0; b < 8; b++) s += (long double)(H[mi][a] * H[mj][b]) * ke[(3 * a + ci) * 24 + 3 * b + cj];
+        return (double)(s / 64.0L);
+    };
+    struct CM {
+        int c, m;
+    };
+    auto block = [&](const CM* x, int n, double* out) {
+        for (int i = 0; i < n; i++)
+            for (int j = i; j < n; j++) *out++ = K(x[i].c, x[i].m, x[j].c, x[j].m);
+    };
+    const CM nn[3] = {{0, 1}, {1, 2}, {2, 4}}, tt[3] = {{0, 6}, {1, 5}, {2, 3}};
+    const CM qq[3][2] = {{{1, 3}, {2, 5}}, {{0, 3}, {2, 6}}, {{0, 5}, {1, 6}}};
+    const CM ss[3][2] = {{{0, 2}, {1, 1}}, {{0, 4}, {2, 1}}, {{1, 4}, {2, 2}}};
+    block(nn, 3, mc.n);
+    block(tt, 3, mc.t);
+    for (int k = 0; k < 3; k++) {
+        block(qq[k], 2, mc.q[k]);
+        block(ss[k], 2, mc.s[k]);
+        mc.d[k] = K(k, 7, k, 7);
+    }
+    const int of[4] = {0, 1, 3, 7};  // one mode of each number of odd directions
+    for (int k = 0; k < 4; k++) {
+        long double s = 0.0L;
+        for (int a = 0; a < 8; a++)
+            for (int b = 0; b < 8; b++) s += (long double)(H[of[k]][a] * H[of[k]][b]) * m8[8 * a + b];
+        mc.m[k] = (double)(s / 64.0L);
+    }
+}
+
+void upload_modes(const double* ke, const double* m8, DBuf<ModeConst<double>>& d64, DBuf<ModeConst<float>>& d32) {
+    ModeConst<double> mc;
+    hex8_modes(ke, m8, mc);
+    ModeConst<float> mf;
+    static_assert(sizeof(mc) == 37 * sizeof(double) && sizeof(mf) == 37 * sizeof(float), "37 constants");
+    for (int i = 0; i < 37; i++) reinterpret_cast<float*>(&mf)[i] = (float)reinterpret_cast<const double*>(&mc)[i];
+    d64.alloc(1);
+    d32.alloc(1);
+    TT_HIP(hipMemcpy(d64.p, &mc, sizeof(mc), hipMemcpyHostToDevice));
+    TT_HIP(hipMemcpy(d32.p, &mf, sizeof(mf), hipMemcpyHostToDevice));
+}
+
 void hex8_helmholtz(double hx, double hy, double hz, double R, double* kf) {
     std::memset(kf, 0, sizeof(double) * 64);
     const double q = 1.0 / std::sqrt(3.0);

@@ -94,6 +94,41 @@ void hex8_stiffness(double hx, double hy, double hz, double nu, double* ke);  //
 void hex8_mass(double hx, double hy, double hz, double* m8);                 // 8x8 scalar, density 1
 void hex8_helmholtz(double hx, double hy, double hz, double R, double* kf);  // 8x8, R^2 Lap + mass
 
+// The element matrices in the element's symmetry-adapted basis (mode bits x, y, z of the sums and differences of the
+// corner values; see tt_apply_cols.inc): the stiffness matrix's blocks, upper triangles, and the mass matrix's
+// diagonal by the number of odd directions.
+template <typename T>
+struct ModeConst {
+    T n[6];     // ux100, uy010, uz001
+    T q[3][3];  // (uy110, uz101), (ux110, uz011), (ux101, uy011)
+    T s[3][3];  // (ux010, uy100), (ux001, uz100), (uy001, uz010)
+    T t[6];     // ux011, uy101, uz110
+    T d[3];     // ux111, uy111, uz111
+    T m[4];
+};
+void hex8_modes(const double* ke, const double* m8, ModeConst<double>& mc);
+// the same in device memory, in both precisions
+void upload_modes(const double* ke, const double* m8, DBuf<ModeConst<double>>& d64, DBuf<ModeConst<float>>& d32);
+// The tile split of one grid for the column kernels (tt_apply_cols.inc): columns of elements per tile row
+// (bx + 1) and owned node columns per tile in x and y; tiles (the nz node planes are split evenly over tz).
+struct ColPlan {
+    int cx, bx, by;
+    int tx, ty, tz;
+    int ntiles() const { return tx * ty * tz; }
+};
+ColPlan make_col_plan(const Grid& g, bool fp64);
+// Per tile of a split: 1 if the tile's staged node box (one halo layer) holds a node with a nonzero mask.
+void col_bc_flags(const Grid& g, const ColPlan& p, const std::vector<uint8_t>& mask, std::vector<uint8_t>& f);
+struct ColSplit {
+    ColPlan plan;
+    const uint8_t* bc;  // the flags, in device memory
+};
+struct ColSplitStore {  // the splits of one grid, by precision, with their flags
+    ColSplit s32{}, s64{};
+    DBuf<uint8_t> flags[2];
+    void build(const Grid& g, const std::vector<uint8_t>& mask);
+};
+
 // ------------------------------------------------------------------ reductions
 // Deterministic device reductions without fences or atomics: a reducing kernel
 // writes one partial per block into a partial buffer; the next kernel on the
@@ -194,22 +229,11 @@ struct OpLevel {
     const void* mf;        // element mass factors (mfac)
     const double* KE64;    // 576
     const double* M864;    // 64
-    const float* KE32;
-    const float* M832;
     const uint8_t* mask;   // per node clamped bits
-    const double* AF64;    // MFMA A fragments of [KE; M8 (x) I3] in lane order (18 x 64)
-    const float* AF32;
-    const uint32_t* AFH;   // FP16-split fragments (3 x 2 x 64 x 4 words), K / M rows scaled by 1 / hs
-    float hs[2];
-    const uint8_t* tbc4;   // per 8x8x4 / 8x8x2 tile: 1 if its staged node box holds a clamped node
-    const uint8_t* tbc2;
-    BatchTab tab4, tab2;   // element batch tables of the 8x8x4 / 8x8x2 tiles
+    const ModeConst<double>* modes64;  // the element matrices in the symmetry-adapted basis (device)
+    const ModeConst<float>* modes32;
+    ColSplit split64, split32;  // tile splits of the column kernels, by the precision they compute in
 };
-// Per-tile flags of 8 x 8 x tz node tiles: 1 if the tile's node box (one halo layer) holds a node
-// with a nonzero mask.
-void tile_bc_flags(const Grid& g, const std::vector<uint8_t>& mask, int tz, std::vector<uint8_t>& f);
-
-// MFMA A fragments of the interleaved [KE; M8 (x) I3] matrix, lane order (see tt_kernels.hip)
 // Symmetric coarsest solve on the packed lower triangle (64 x 64 tiles): size of the packed array,
 // packing of a full symmetric matrix, and x = A b with per-tile partials (nt (nt + 1) / 2 x 64 each).
 long sym_packed_size(int n);
@@ -224,9 +248,6 @@ void launch_dense_coarse(const Grid& g, const double* kf, const double* mf, doub
 void launch_spd_inv_small(double* A, int m, int lda, int* info, hipStream_t s);
 // dst (cols x rows) = src (rows x cols) transposed, column-major with leading dimensions lds, ldd.
 void launch_transpose(const double* src, int rows, int cols, int lds, double* dst, int ldd, hipStream_t s);
-constexpr int AF32_WORDS = 18 * 64 + 3 * 2 * 64 * 4;  // FP32 fragments followed by the FP16-split ones
-void mfma_fragments(const double* KE, const double* M8, double* af64, float* af32, uint32_t* afh, float* hs);
-
 // y = N.(cK*K + cM*M)(N.u) on free dofs, identity on clamped dofs.  With red: partials of u.y in
 // partial region dot_slot (PB_*).  Reductions below likewise take a partial region.
 void launch_apply_bc(const OpLevel& L, double cK, double cM, const void* u, void* y, bool fp64, hipStream_t s,

@@ -33,6 +33,56 @@ __device__ __forceinline__ double coef_ld(const bf16_t* p, long i) {
     return (double)__uint_as_float(((uint32_t)p[i]) << 16);
 }
 
+// A uniform pointer as a scalar base in global memory: what is added to it per lane stays a 32-bit byte offset (the
+// compiler would otherwise hoist base + lane offset out of a loop over planes into 64-bit vector address pairs).
+template <typename T>
+using gptr = __attribute__((address_space(1))) T*;
+template <typename T>
+__device__ __forceinline__ gptr<T> sbase(T* p) {
+    gptr<T> g = (gptr<T>)p;
+    asm("" : "+s"(g));
+    return g;
+}
+// A lane's offset as byte offsets of 1, 2, 4 and 8 byte elements, opaque to the compiler (it would widen the scaling to
+// 64 bits); what a kernel does not use costs nothing.
+struct LaneOff {
+    unsigned o1, o2, o4, o8;
+    __device__ __forceinline__ explicit LaneOff(unsigned i = 0) : o1(i), o2(2 * i), o4(4 * i), o8(8 * i) {
+        asm("" : "+v"(o1));
+        asm("" : "+v"(o2));
+        asm("" : "+v"(o4));
+        asm("" : "+v"(o8));
+    }
+    template <typename T>
+    __device__ __forceinline__ unsigned of() const {
+        return sizeof(T) == 1 ? o1 : sizeof(T) == 2 ? o2 : sizeof(T) == 4 ? o4 : o8;
+    }
+};
+// element i (+ c, an immediate) of a uniform pointer
+template <typename T>
+__device__ __forceinline__ T ldu(const T* p, const LaneOff& i, int c = 0) {
+    typedef __attribute__((address_space(1))) const char* cp;
+    return ((gptr<const T>)((cp)sbase(p) + i.of<T>()))[c];
+}
+// The three consecutive values of one node at dofs b + i .. b + i + 2 (b uniform, i per lane).
+template <typename T>
+__device__ __forceinline__ void ld3(const T* p, size_t b, const LaneOff& i, T (&v)[3]) {
+    typedef __attribute__((address_space(1))) const char* cp;
+    const gptr<const T> q = (gptr<const T>)((cp)sbase(p + b) + i.of<T>());
+#pragma unroll
+    for (int c = 0; c < 3; c++) v[c] = q[c];
+}
+template <typename T>
+__device__ __forceinline__ void st3(T* p, size_t b, const LaneOff& i, const T (&v)[3]) {
+    typedef __attribute__((address_space(1))) char* cp;
+    const gptr<T> q = (gptr<T>)((cp)sbase(p + b) + i.of<T>());
+#pragma unroll
+    for (int c = 0; c < 3; c++) q[c] = v[c];
+}
+__device__ __forceinline__ double coef_val(double v) { return v; }
+__device__ __forceinline__ float coef_val(float v) { return v; }
+__device__ __forceinline__ float coef_val(bf16_t v) { return __uint_as_float((uint32_t)v << 16); }
+
 constexpr int BS = 256;  // threads per block for all 1-D kernels
 
 // ------------------------------------------------------------------ deterministic block reduction
@@ -150,364 +200,161 @@ static inline int red_blocks(long n) {
 }
 
 // ------------------------------------------------------------------ operator apply
-constexpr int TX = 8, TY = 8, TZ = 4, NT = TX * TY * TZ;
-constexpr int HX = TX + 2, HY = TY + 2, HZ = TZ + 2, HN = HX * HY * HZ;
-constexpr int EXs = TX + 1, EYs = TY + 1, EZs = TZ + 1, EN = EXs * EYs * EZs;
-static_assert(NT == BS, "tile must match block size");
-
 struct GridArgs {
     int nx, ny, nz, ex, ey, ez;
 };
 static inline GridArgs gargs(const Grid& g) { return GridArgs{g.nx, g.ny, g.nz, g.ex, g.ey, g.ez}; }
 
-// Per-node contraction of one input: yK = sum_e kfe * KE[a rows] u_e, yM = sum_e mfe * (M8 (x) I3)[a rows] u_e.
-// FENCE keeps each element's matrix rows from being hoisted across the node's 8 elements (the
-// compiler otherwise holds the 576 + 64 uniform values in scalar registers and spills them).  It is
-// applied where K and M results leave the kernel separately (the split K / M outputs); with one
-// summed output the same fence makes the code larger.
-template <typename T, bool FENCE>
-__device__ __forceinline__ void node_contract(const T* __restrict__ sU, const T* __restrict__ sk,
-                                              const T* __restrict__ sm,
-                                              const T* __restrict__ KE, const T* __restrict__ M8, int tx, int ty,
-                                              int tz, T (&yK)[3], T (&yM)[3]) {
-#pragma unroll
-    for (int ez = 0; ez < 2; ez++)
-#pragma unroll
-        for (int ey = 0; ey < 2; ey++)
-#pragma unroll
-            for (int ex = 0; ex < 2; ex++) {
-                if (FENCE) __asm__ __volatile__("" ::: "memory");
-                const int a = corner_id(1 - ex, 1 - ey, 1 - ez);
-                const int eidx = ((tz + ez) * EYs + (ty + ey)) * EXs + (tx + ex);
-                const T kfe = sk[eidx], mfe = sm[eidx];
-                T k0 = 0, k1 = 0, k2 = 0, m0 = 0, m1 = 0, m2 = 0;
-#pragma unroll
-                for (int b = 0; b < 8; b++) {
-                    const int nidx = ((tz + ez + cz_of(b)) * HY + (ty + ey + cy_of(b))) * HX + (tx + ex + cx_of(b));
-                    const T u0 = sU[3 * nidx], u1 = sU[3 * nidx + 1], u2 = sU[3 * nidx + 2];
-                    const T* kr = KE + (3 * a) * 24 + 3 * b;
-                    k0 = fma(kr[0], u0, fma(kr[1], u1, fma(kr[2], u2, k0)));
-                    k1 = fma(kr[24], u0, fma(kr[25], u1, fma(kr[26], u2, k1)));
-                    k2 = fma(kr[48], u0, fma(kr[49], u1, fma(kr[50], u2, k2)));
-                    const T mab = M8[a * 8 + b];
-                    m0 = fma(mab, u0, m0);
-                    m1 = fma(mab, u1, m1);
-                    m2 = fma(mab, u2, m2);
-                }
-                yK[0] = fma(kfe, k0, yK[0]);
-                yK[1] = fma(kfe, k1, yK[1]);
-                yK[2] = fma(kfe, k2, yK[2]);
-                yM[0] = fma(mfe, m0, yM[0]);
-                yM[1] = fma(mfe, m1, yM[1]);
-                yM[2] = fma(mfe, m2, yM[2]);
-            }
-}
-
-// Per-node contraction of two inputs, yK = sum_e kfe * KE[a rows] u_e and yM = sum_e mfe * (M8 (x) I3)[a rows]
-// w_e, in neighbour order: the node's 27 neighbours in the outer loop, the 1-8 elements that hold both
-// the node and the neighbour in the inner one.  Each neighbour's values are read from LDS once (162
-// reads per node instead of 384 in element order); the 8 element coefficients (element e at offset
-// (e & 1, (e >> 1) & 1, e >> 2) - 1 from the node) come in registers.  The fence per neighbour keeps
-// the uniform matrix entries from being hoisted into scalar registers and spilled.  On the 128 x 64 x 64
-// right-hand side this order takes 68 us against 74 us per launch.
-template <typename T>
-__device__ __forceinline__ void node_contract_nb(const T* __restrict__ sU, const T* __restrict__ sW,
-                                                 const T (&kfe)[8], const T (&mfe)[8],
-                                                 const T* __restrict__ KE, const T* __restrict__ M8, int tx, int ty,
-                                                 int tz, T (&yK)[3], T (&yM)[3]) {
-#pragma unroll
-    for (int dz = -1; dz <= 1; dz++)
-#pragma unroll
-        for (int dy = -1; dy <= 1; dy++)
-#pragma unroll
-            for (int dx = -1; dx <= 1; dx++) {
-                __asm__ __volatile__("" ::: "memory");
-                const int nidx = ((tz + 1 + dz) * HY + (ty + 1 + dy)) * HX + (tx + 1 + dx);
-                const T u0 = sU[3 * nidx], u1 = sU[3 * nidx + 1], u2 = sU[3 * nidx + 2];
-                const T w0 = sW[3 * nidx], w1 = sW[3 * nidx + 1], w2 = sW[3 * nidx + 2];
-#pragma unroll
-                for (int e = 0; e < 8; e++) {
-                    const int ex = e & 1, ey = (e >> 1) & 1, ez = e >> 2;
-                    const int bx = 1 + dx - ex, by = 1 + dy - ey, bz = 1 + dz - ez;  // b as a corner of e
-                    if (bx < 0 || bx > 1 || by < 0 || by > 1 || bz < 0 || bz > 1) continue;
-                    const int a = corner_id(1 - ex, 1 - ey, 1 - ez), b = corner_id(bx, by, bz);
-                    const T* kr = KE + (3 * a) * 24 + 3 * b;
-                    const T t0 = fma(kr[0], u0, fma(kr[1], u1, kr[2] * u2));
-                    const T t1 = fma(kr[24], u0, fma(kr[25], u1, kr[26] * u2));
-                    const T t2 = fma(kr[48], u0, fma(kr[49], u1, kr[50] * u2));
-                    yK[0] = fma(kfe[e], t0, yK[0]);
-                    yK[1] = fma(kfe[e], t1, yK[1]);
-                    yK[2] = fma(kfe[e], t2, yK[2]);
-                    const T cm = mfe[e] * M8[a * 8 + b];
-                    yM[0] = fma(cm, w0, yM[0]);
-                    yM[1] = fma(cm, w1, yM[1]);
-                    yM[2] = fma(cm, w2, yM[2]);
-                }
-            }
-}
-
-// Input staging policies: produce the (masked) value of dof (node n, comp c) for the K and M inputs
+// Input staging policies of the column kernels: raw() loads what the staged value of a dof (at b + i + c, b uniform) is
+// made of, value() makes it (two values where K and M act on different vectors).  depth: planes the loads run ahead (the
+// three-vector form holds too much in flight for two).
 template <typename T>
 struct StageOne {  // w = u
+    static constexpr int inputs = 1, depth = 2;
     const T* u;
-    __device__ __forceinline__ void prologue() {}
-    __device__ __forceinline__ T k(unsigned i) const { return ld(u, i); }
-    __device__ __forceinline__ T m(unsigned i) const { return ld(u, i); }
+    typedef T Raw;
+    __device__ __forceinline__ Raw raw(size_t b, const LaneOff& i, int c = 0) const { return ldu(u + b, i, c); }
+    __device__ __forceinline__ void value(const Raw& r, T (&x)[1]) const { x[0] = r; }
 };
 // First Chebyshev iterate x0 = c1 D^-1 b formed on the fly, with b = (T) r (FP64) on the finest level
 template <typename T, bool FROM64>
 struct StageChebFirst {
+    static constexpr int inputs = 1, depth = 2;
     const double* r64;
     const T* b;
     const T* dinv;
     T c1;
-    __device__ __forceinline__ void prologue() {}
-    __device__ __forceinline__ T bval(unsigned i) const { return FROM64 ? (T)ld(r64, i) : ld(b, i); }
-    __device__ __forceinline__ T k(unsigned i) const { return c1 * ld(dinv, i) * bval(i); }
-    __device__ __forceinline__ T m(unsigned i) const { return k(i); }
+    struct Raw {
+        typename std::conditional<FROM64, double, T>::type b;
+        T di;
+    };
+    __device__ __forceinline__ Raw raw(size_t base, const LaneOff& i, int c = 0) const {
+        Raw r;
+        if constexpr (FROM64) r.b = ldu(r64 + base, i, c);
+        else r.b = ldu(b + base, i, c);
+        r.di = ldu(dinv + base, i, c);
+        return r;
+    }
+    __device__ __forceinline__ void value(const Raw& r, T (&x)[1]) const { x[0] = c1 * r.di * (T)r.b; }
 };
 struct StageThree {  // wK = sum_i cK_i in_i, wM = sum_i cM_i in_i (FP64)
+    static constexpr int inputs = 2, depth = 1;
     const double *u, *v, *a;
     double k0, k1, k2, m0, m1, m2;
-    __device__ __forceinline__ void prologue() {}
-    __device__ __forceinline__ double k(unsigned i) const { return k0 * ld(u, i) + k1 * ld(v, i) + k2 * ld(a, i); }
-    __device__ __forceinline__ double m(unsigned i) const { return m0 * ld(u, i) + m1 * ld(v, i) + m2 * ld(a, i); }
+    struct Raw {
+        double u, v, a;
+    };
+    __device__ __forceinline__ Raw raw(size_t b, const LaneOff& i, int c = 0) const {
+        return Raw{ldu(u + b, i, c), ldu(v + b, i, c), ldu(a + b, i, c)};
+    }
+    __device__ __forceinline__ void value(const Raw& r, double (&x)[2]) const {
+        x[0] = k0 * r.u + k1 * r.v + k2 * r.a;
+        x[1] = m0 * r.u + m1 * r.v + m2 * r.a;
+    }
 };
 
-struct EpiSplit;
-// The two-input form (the right-hand side) reads each node's 8 element coefficients into registers
-// instead of staging them in LDS: 28.8 instead of 35.3 KB of LDS per block, and with at most 96 VGPRs
-// (5 waves per SIMD requested) 5 instead of 4 blocks per CU.
-template <typename T, typename CT, bool TWO, bool MASKIN, class Stage, class Epi>
-__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(TWO ? 5 : 1))) void k_apply(
-    GridArgs g, const T* __restrict__ KE, const T* __restrict__ M8, const CT* __restrict__ kf,
-    const CT* __restrict__ mf, T cK, T cM, const uint8_t* __restrict__ mask, Stage st_in, Epi epi) {
-    __shared__ T sU[HN * 3];
-    __shared__ T sW[TWO ? HN * 3 : 1];
-    __shared__ T sk[TWO ? 1 : EN], sm[TWO ? 1 : EN];
-    const int i0 = blockIdx.x * TX, j0 = blockIdx.y * TY, k0 = blockIdx.z * TZ;
-    const int tid = threadIdx.x;
-    // the thread's own node
-    const int tx = tid % TX, ty = (tid / TX) % TY, tz = tid / (TX * TY);
-    const int oi = i0 + tx, oj = j0 + ty, ok = k0 + tz;
-    const bool inside = oi < g.nx && oj < g.ny && ok < g.nz;
-    Stage st = st_in;
-    st.prologue();
-    // Stage the node box and element coefficients.  Every global load of the
-    // block is issued before the first LDS store, so the block waits for one
-    // memory latency instead of one per loop trip.
-    constexpr int NSV = (HN * 3 + NT - 1) / NT;
-    constexpr int NSE = TWO ? 1 : (EN + NT - 1) / NT;
-    T val[NSV], valw[TWO ? NSV : 1];
-    T ca[NSE], cb[NSE];
-    T kfe[TWO ? 8 : 1], mfe[TWO ? 8 : 1];
-    if constexpr (TWO) {
-#pragma unroll
-        for (int e = 0; e < 8; e++) {
-            const int ei = oi - 1 + (e & 1), ej = oj - 1 + ((e >> 1) & 1), ek = ok - 1 + (e >> 2);
-            const bool in = inside && ei >= 0 && ei < g.ex && ej >= 0 && ej < g.ey && ek >= 0 && ek < g.ez;
-            const long ge = in ? ei + (long)g.ex * (ej + (long)g.ey * ek) : 0;
-            kfe[e] = in ? cK * (T)coef_ld(kf, ge) : (T)0;
-            mfe[e] = in ? cM * (T)coef_ld(mf, ge) : (T)0;
-        }
-    }
-#pragma unroll
-    for (int q = 0; q < NSV; q++) {
-        const int v = tid + q * NT;
-        const int node = v / 3, c = v - 3 * node;
-        const int hx = node % HX, hy = (node / HX) % HY, hz = node / (HX * HY);
-        const int gi = i0 - 1 + hx, gj = j0 - 1 + hy, gk = k0 - 1 + hz;
-        const bool in = v < HN * 3 && gi >= 0 && gi < g.nx && gj >= 0 && gj < g.ny && gk >= 0 && gk < g.nz;
-        const long n = in ? gi + (long)g.nx * (gj + (long)g.ny * gk) : 0;
-        T x = in ? st.k(3 * n + c) : (T)0;
-        T w = 0;
-        if (TWO) w = in ? st.m(3 * n + c) : (T)0;
-        if (MASKIN) {
-            const uint8_t cl = in ? mask[n] : (uint8_t)0;
-            if ((cl >> c) & 1) {
-                x = 0;
-                w = 0;
-            }
-        }
-        val[q] = x;
-        if (TWO) valw[q] = w;
-    }
-#pragma unroll
-    for (int q = 0; q < (TWO ? 0 : NSE); q++) {
-        const int e = tid + q * NT;
-        const int hx = e % EXs, hy = (e / EXs) % EYs, hz = e / (EXs * EYs);
-        const int gi = i0 - 1 + hx, gj = j0 - 1 + hy, gk = k0 - 1 + hz;
-        const bool in = e < EN && gi >= 0 && gi < g.ex && gj >= 0 && gj < g.ey && gk >= 0 && gk < g.ez;
-        const long ge = in ? gi + (long)g.ex * (gj + (long)g.ey * gk) : 0;
-        ca[q] = in ? cK * (T)coef_ld(kf, ge) : (T)0;
-        cb[q] = in ? cM * (T)coef_ld(mf, ge) : (T)0;
-    }
-#pragma unroll
-    for (int q = 0; q < NSV; q++) {
-        const int v = tid + q * NT;
-        if (v < HN * 3) {
-            sU[v] = val[q];
-            if (TWO) sW[v] = valw[q];
-        }
-    }
-#pragma unroll
-    for (int q = 0; q < (TWO ? 0 : NSE); q++) {
-        const int e = tid + q * NT;
-        if (e < EN) {
-            sk[e] = ca[q];
-            sm[e] = cb[q];
-        }
-    }
-    __syncthreads();
-    T yK[3] = {0, 0, 0}, yM[3] = {0, 0, 0};
-    long n = 0;
-    uint8_t cl = 0;
-    if (inside) {
-        if constexpr (TWO)
-            node_contract_nb<T>(sU, sW, kfe, mfe, KE, M8, tx, ty, tz, yK, yM);
-        else
-            node_contract<T, std::is_same<Epi, EpiSplit>::value>(sU, sk, sm, KE, M8, tx, ty, tz, yK, yM);
-        n = oi + (long)g.nx * (oj + (long)g.ny * ok);
-        cl = mask[n];
-    }
-    epi(inside, n, cl, yK, yM, st);
-}
+#include "tt_apply_cols.inc"
 
-#include "tt_apply_mfma.inc"
-
-// ---- epilogues.  fetch() loads the per-node operands an epilogue reads (its Pre) for one owned
-// node; the tile kernels issue it together with the staging loads, so that those loads are in
-// flight while the element contraction runs.  put() then handles that node (inside the grid) and
-// may add to the thread's reduction share; done() is called once by every thread of the block at
-// the end (reducing epilogues write their block partial there).  operator() is the
-// one-node-per-thread form.
-#define TT_EPI_CALL                                                                                      \
-    template <class S, typename V>                                                                     \
-    __device__ void operator()(bool in, int n, uint8_t cl, const V (&yK)[3], const V (&yM)[3],          \
-                               const S& st) const {                                                     \
-        double acc[2] = {0.0, 0.0};                                                                    \
-        if (in) {                                                                                      \
-            Pre pre;                                                                                   \
-            fetch(n, st, pre);                                                                         \
-            const V uo[3] = {st.k(3 * n), st.k(3 * n + 1), st.k(3 * n + 2)};                           \
-            put(n, cl, yK, yM, st, uo, acc, pre);                                                      \
-        }                                                                                              \
-        done(acc);                                                                                     \
-    }
+// ---- epilogues.  A node's three dofs are b + i .. b + i + 2, b uniform over the block (its node plane's first dof, or
+// 0).  fetch() loads the per-node operands an epilogue reads (its Pre) for one owned node, ahead of the element
+// contraction.  put() then handles that node (inside the grid): cl are its clamped dofs, uo its input values (not
+// masked); it may add to the thread's reduction share.  done() is called once by every thread of the block at the end
+// (reducing epilogues write their block partial there).
+// outputs: 2 where K and M results are taken apart (yK, yM), else yK is their sum; uses_input: whether put() reads uo.
 #define TT_NO_PRE                                                     \
     struct Pre {};                                                    \
     template <class S>                                                \
-    __device__ __forceinline__ void fetch(int, const S&, Pre&) const {}
-
-// Input value of dof i for an epilogue: the staged value uo (free dofs), re-read through the stage
-// only on clamped dofs, where the staged copy is masked.
-template <class S, typename T>
-__device__ __forceinline__ T input_at(const S& st, uint8_t cl, int c, int i, const T (&uo)[3]) {
-    T x = uo[c];
-    if ((cl >> c) & 1) x = st.k(i);
-    return x;
-}
+    __device__ __forceinline__ void fetch(size_t, const LaneOff&, const S&, Pre&) const {}
 
 template <typename T>
 struct EpiBC {  // y = A u on free dofs, u on clamped
+    static constexpr int outputs = 1;
+    static constexpr bool uses_input = true;
     T* y;
     TT_NO_PRE
-    template <class S>
-    __device__ void put(int n, uint8_t cl, const T (&yK)[3], const T (&yM)[3], const S& st, const T (&)[3],
+    __device__ void put(size_t b, const LaneOff& i, uint8_t cl, const T (&yK)[3], const T (&)[3], const T (&uo)[3],
                         double (&)[2], const Pre&) const {
+        T v[3];
 #pragma unroll
-        for (int c = 0; c < 3; c++) {
-            T v = yK[c] + yM[c];
-            if ((cl >> c) & 1) v = st.k(3 * n + c);
-            y[3 * n + c] = v;
-        }
+        for (int c = 0; c < 3; c++) v[c] = ((cl >> c) & 1) ? uo[c] : yK[c];
+        st3(y, b, i, v);
     }
     __device__ void done(double (&)[2]) const {}
-    TT_EPI_CALL
 };
 
 template <typename T>
 struct EpiBCDot {  // y = A u (BC form) and partials of u.y
+    static constexpr int outputs = 1;
+    static constexpr bool uses_input = true;
     T* y;
     double* part;
     TT_NO_PRE
-    template <class S>
-    __device__ void put(int n, uint8_t cl, const T (&yK)[3], const T (&yM)[3], const S& st, const T (&uo)[3],
+    __device__ void put(size_t b, const LaneOff& i, uint8_t cl, const T (&yK)[3], const T (&)[3], const T (&uo)[3],
                         double (&acc)[2], const Pre&) const {
+        T v[3];
 #pragma unroll
         for (int c = 0; c < 3; c++) {
-            const T u = input_at(st, cl, c, 3 * n + c, uo);
-            const T v = ((cl >> c) & 1) ? u : yK[c] + yM[c];
-            y[3 * n + c] = v;
-            acc[0] += (double)u * (double)v;
+            v[c] = ((cl >> c) & 1) ? uo[c] : yK[c];
+            acc[0] += (double)uo[c] * (double)v[c];
         }
+        st3(y, b, i, v);
     }
     __device__ void done(double (&acc)[2]) const {
         double a[1] = {acc[0]};
         write_partials<1>(a, part);
     }
-    TT_EPI_CALL
 };
 
 template <typename T>
 struct EpiResid {  // r = b - A x
-    const T* b;
+    static constexpr int outputs = 1;
+    static constexpr bool uses_input = true;
+    const T* rhs;
     T* r;
     struct Pre {
         T b[3];
     };
     template <class S>
-    __device__ __forceinline__ void fetch(int n, const S&, Pre& p) const {
-#pragma unroll
-        for (int c = 0; c < 3; c++) p.b[c] = b[3 * n + c];
-    }
-    template <class S>
-    __device__ void put(int n, uint8_t cl, const T (&yK)[3], const T (&yM)[3], const S& st, const T (&)[3],
+    __device__ __forceinline__ void fetch(size_t b, const LaneOff& i, const S&, Pre& p) const { ld3(rhs, b, i, p.b); }
+    __device__ void put(size_t b, const LaneOff& i, uint8_t cl, const T (&yK)[3], const T (&)[3], const T (&uo)[3],
                         double (&)[2], const Pre& p) const {
+        T v[3];
 #pragma unroll
-        for (int c = 0; c < 3; c++) {
-            T ax = yK[c] + yM[c];
-            if ((cl >> c) & 1) ax = st.k(3 * n + c);
-            r[3 * n + c] = p.b[c] - ax;
-        }
+        for (int c = 0; c < 3; c++) v[c] = p.b[c] - (((cl >> c) & 1) ? uo[c] : yK[c]);
+        st3(r, b, i, v);
     }
     __device__ void done(double (&)[2]) const {}
-    TT_EPI_CALL
 };
 
 // One damped-Jacobi step from x = 0 and its residual in one pass (an intermediate multigrid level's
 // pre-smoothing): x = c1 D^-1 b is formed in staging (StageChebFirst) and written, with r = b - A x.
 template <typename T>
 struct EpiResidFirst {
+    static constexpr int outputs = 1;
+    static constexpr bool uses_input = true;
     T* x;
     T* r;
     struct Pre {
         T b[3];
     };
     template <class S>
-    __device__ __forceinline__ void fetch(int n, const S& st, Pre& p) const {
-#pragma unroll
-        for (int c = 0; c < 3; c++) p.b[c] = st.bval(3 * n + c);
-    }
-    template <class S>
-    __device__ void put(int n, uint8_t cl, const T (&yK)[3], const T (&yM)[3], const S& st, const T (&uo)[3],
+    __device__ __forceinline__ void fetch(size_t b, const LaneOff& i, const S& st, Pre& p) const { ld3(st.b, b, i, p.b); }
+    __device__ void put(size_t b, const LaneOff& i, uint8_t cl, const T (&yK)[3], const T (&)[3], const T (&uo)[3],
                         double (&)[2], const Pre& p) const {
+        T v[3];
 #pragma unroll
-        for (int c = 0; c < 3; c++) {
-            const int i = 3 * n + c;
-            const T xi = input_at(st, cl, c, i, uo);
-            const T ax = ((cl >> c) & 1) ? xi : yK[c] + yM[c];
-            x[i] = xi;
-            r[i] = p.b[c] - ax;
-        }
+        for (int c = 0; c < 3; c++) v[c] = p.b[c] - (((cl >> c) & 1) ? uo[c] : yK[c]);
+        st3(x, b, i, uo);
+        st3(r, b, i, v);
     }
     __device__ void done(double (&)[2]) const {}
-    TT_EPI_CALL
 };
 
 // r = b - A x (FP64) with the partials of b.b and r.r, one per block into each of two regions
 struct EpiResidDots {
-    const double* b;
+    static constexpr int outputs = 1;
+    static constexpr bool uses_input = true;
+    const double* rhs;
     double* r;
     double* pbb;
     double* prr;
@@ -515,22 +362,17 @@ struct EpiResidDots {
         double b[3];
     };
     template <class S>
-    __device__ __forceinline__ void fetch(int n, const S&, Pre& p) const {
-#pragma unroll
-        for (int c = 0; c < 3; c++) p.b[c] = b[3 * n + c];
-    }
-    template <class S>
-    __device__ void put(int n, uint8_t cl, const double (&yK)[3], const double (&yM)[3], const S& st,
-                        const double (&)[3], double (&acc)[2], const Pre& p) const {
+    __device__ __forceinline__ void fetch(size_t b, const LaneOff& i, const S&, Pre& p) const { ld3(rhs, b, i, p.b); }
+    __device__ void put(size_t b, const LaneOff& i, uint8_t cl, const double (&yK)[3], const double (&)[3],
+                        const double (&uo)[3], double (&acc)[2], const Pre& p) const {
+        double v[3];
 #pragma unroll
         for (int c = 0; c < 3; c++) {
-            double ax = yK[c] + yM[c];
-            if ((cl >> c) & 1) ax = st.k(3 * n + c);
-            const double bi = p.b[c], ri = bi - ax;
-            r[3 * n + c] = ri;
-            acc[0] = fma(bi, bi, acc[0]);
-            acc[1] = fma(ri, ri, acc[1]);
+            v[c] = p.b[c] - (((cl >> c) & 1) ? uo[c] : yK[c]);
+            acc[0] = fma(p.b[c], p.b[c], acc[0]);
+            acc[1] = fma(v[c], v[c], acc[1]);
         }
+        st3(r, b, i, v);
     }
     __device__ void done(double (&acc)[2]) const {
         __shared__ double sh[16 * 2];
@@ -541,12 +383,13 @@ struct EpiResidDots {
             prr[bid] = acc[1];
         }
     }
-    TT_EPI_CALL
 };
 
 template <typename T>
 struct EpiCheb {  // r = b - A x; dn = c0 d + c1 dinv r; xn = x + dn
-    const T* b;
+    static constexpr int outputs = 1;
+    static constexpr bool uses_input = true;
+    const T* rhs;
     const T* d;
     const T* dinv;
     T c0, c1;
@@ -556,79 +399,72 @@ struct EpiCheb {  // r = b - A x; dn = c0 d + c1 dinv r; xn = x + dn
         T b[3], d[3], di[3];
     };
     template <class S>
-    __device__ __forceinline__ void fetch(int n, const S&, Pre& p) const {
-#pragma unroll
-        for (int c = 0; c < 3; c++) {
-            const int i = 3 * n + c;
-            p.b[c] = b[i];
-            p.di[c] = dinv[i];
-            p.d[c] = d ? d[i] : (T)0;
-        }
+    __device__ __forceinline__ void fetch(size_t b, const LaneOff& i, const S&, Pre& p) const {
+        ld3(rhs, b, i, p.b);
+        ld3(dinv, b, i, p.di);
+        if (d) ld3(d, b, i, p.d);
     }
-    template <class S>
-    __device__ void put(int n, uint8_t cl, const T (&yK)[3], const T (&yM)[3], const S& st, const T (&uo)[3],
+    __device__ void put(size_t b, const LaneOff& i, uint8_t cl, const T (&yK)[3], const T (&)[3], const T (&uo)[3],
                         double (&)[2], const Pre& p) const {
+        T dd[3], v[3];
 #pragma unroll
         for (int c = 0; c < 3; c++) {
-            const int i = 3 * n + c;
-            const T x = input_at(st, cl, c, i, uo);
-            const T ax = ((cl >> c) & 1) ? x : yK[c] + yM[c];
-            const T r = p.b[c] - ax;
-            T dd = c1 * p.di[c] * r;
-            if (d) dd = fma(c0, p.d[c], dd);
-            xn[i] = x + dd;
-            if (dn) dn[i] = dd;
+            const T r = p.b[c] - (((cl >> c) & 1) ? uo[c] : yK[c]);
+            dd[c] = c1 * p.di[c] * r;
+            if (d) dd[c] = fma(c0, p.d[c], dd[c]);
+            v[c] = uo[c] + dd[c];
         }
+        st3(xn, b, i, v);
+        if (dn) st3(dn, b, i, dd);
     }
     __device__ void done(double (&)[2]) const {}
-    TT_EPI_CALL
 };
 
 // Second Chebyshev step from x0 = c1 D^-1 b (staged by StageChebFirst, so d = x0):
 // dn = c0 x0 + c1 D^-1 (b - A x0), xn = x0 + dn; on the finest level it also writes b = (T) r.
 template <typename T, bool FROM64>
 struct EpiChebFirst {
+    static constexpr int outputs = 1;
+    static constexpr bool uses_input = true;
     T* bout;
     const T* dinv;
     T c0, c1;
     T* xn;
     T* dn;
     struct Pre {
-        T b[3], di[3];
+        typename std::conditional<FROM64, double, T>::type b[3];
+        T di[3];
     };
     template <class S>
-    __device__ __forceinline__ void fetch(int n, const S& st, Pre& p) const {
-#pragma unroll
-        for (int c = 0; c < 3; c++) {
-            const int i = 3 * n + c;
-            p.b[c] = st.bval(i);
-            p.di[c] = dinv[i];
-        }
+    __device__ __forceinline__ void fetch(size_t b, const LaneOff& i, const S& st, Pre& p) const {
+        if constexpr (FROM64) ld3(st.r64, b, i, p.b);
+        else ld3(st.b, b, i, p.b);
+        ld3(dinv, b, i, p.di);
     }
-    template <class S>
-    __device__ void put(int n, uint8_t cl, const T (&yK)[3], const T (&yM)[3], const S& st, const T (&uo)[3],
+    __device__ void put(size_t b, const LaneOff& i, uint8_t cl, const T (&yK)[3], const T (&)[3], const T (&uo)[3],
                         double (&)[2], const Pre& p) const {
+        T bi[3], dd[3], v[3];
 #pragma unroll
         for (int c = 0; c < 3; c++) {
-            const int i = 3 * n + c;
-            const T bi = p.b[c];
-            if (FROM64) bout[i] = bi;
-            const T x = input_at(st, cl, c, i, uo);
-            const T ax = ((cl >> c) & 1) ? x : yK[c] + yM[c];
-            const T dd = fma(c0, x, c1 * p.di[c] * (bi - ax));
-            xn[i] = x + dd;
-            dn[i] = dd;
+            bi[c] = (T)p.b[c];
+            const T ax = ((cl >> c) & 1) ? uo[c] : yK[c];
+            dd[c] = fma(c0, uo[c], c1 * p.di[c] * (bi[c] - ax));
+            v[c] = uo[c] + dd[c];
         }
+        if (FROM64) st3(bout, b, i, bi);
+        st3(xn, b, i, v);
+        st3(dn, b, i, dd);
     }
     __device__ void done(double (&)[2]) const {}
-    TT_EPI_CALL
 };
 
 // Last post-smoothing step of the finest level: z = x + c0 d + c1 D^-1 (b - A x) written in FP64
 // as the preconditioned residual of flexible CG, with partials of z.r and z.r_prev.
 template <typename T>
 struct EpiChebOut {
-    const T* b;
+    static constexpr int outputs = 1;
+    static constexpr bool uses_input = true;
+    const T* rhs;
     const T* d;
     const T* dinv;
     T c0, c1;
@@ -642,69 +478,66 @@ struct EpiChebOut {
         double r[3], rp[3];
     };
     template <class S>
-    __device__ __forceinline__ void fetch(int n, const S&, Pre& p) const {
-#pragma unroll
-        for (int c = 0; c < 3; c++) {
-            const int i = 3 * n + c;
-            p.b[c] = b[i];
-            p.di[c] = dinv[i];
-            p.d[c] = d ? d[i] : (T)0;
-            p.r[c] = r[i];
-            p.rp[c] = first ? 0.0 : rp[i];
-        }
+    __device__ __forceinline__ void fetch(size_t b, const LaneOff& i, const S&, Pre& p) const {
+        ld3(rhs, b, i, p.b);
+        ld3(dinv, b, i, p.di);
+        if (d) ld3(d, b, i, p.d);
+        ld3(r, b, i, p.r);
+        if (!first) ld3(rp, b, i, p.rp);
     }
-    template <class S>
-    __device__ void put(int n, uint8_t cl, const T (&yK)[3], const T (&yM)[3], const S& st, const T (&uo)[3],
+    __device__ void put(size_t b, const LaneOff& i, uint8_t cl, const T (&yK)[3], const T (&)[3], const T (&uo)[3],
                         double (&acc)[2], const Pre& p) const {
+        double zi[3];
 #pragma unroll
         for (int c = 0; c < 3; c++) {
-            const int i = 3 * n + c;
-            const T x = input_at(st, cl, c, i, uo);
-            const T ax = ((cl >> c) & 1) ? x : yK[c] + yM[c];
+            const T ax = ((cl >> c) & 1) ? uo[c] : yK[c];
             T dd = c1 * p.di[c] * (p.b[c] - ax);
             if (d) dd = fma(c0, p.d[c], dd);
-            const double zi = (double)(x + dd);
-            z[i] = zi;
-            acc[0] = fma(zi, p.r[c], acc[0]);
-            if (!first) acc[1] = fma(zi, p.rp[c], acc[1]);
+            zi[c] = (double)(uo[c] + dd);
+            acc[0] = fma(zi[c], p.r[c], acc[0]);
+            if (!first) acc[1] = fma(zi[c], p.rp[c], acc[1]);
         }
+        st3(z, b, i, zi);
     }
     __device__ void done(double (&acc)[2]) const { write_partials<2>(acc, part); }
-    TT_EPI_CALL
 };
 
 struct EpiSplit {  // yk = N.K(N u), ym = N.M(N u)
+    static constexpr int outputs = 2;
+    static constexpr bool uses_input = false;
     double* yk;
     double* ym;
     TT_NO_PRE
-    template <class S>
-    __device__ void put(int n, uint8_t cl, const double (&yK)[3], const double (&yM)[3], const S&,
+    __device__ void put(size_t b, const LaneOff& i, uint8_t cl, const double (&yK)[3], const double (&yM)[3],
                         const double (&)[3], double (&)[2], const Pre&) const {
+        double k[3], m[3];
 #pragma unroll
         for (int c = 0; c < 3; c++) {
             const bool clamped = (cl >> c) & 1;
-            yk[3 * n + c] = clamped ? 0.0 : yK[c];
-            ym[3 * n + c] = clamped ? 0.0 : yM[c];
+            k[c] = clamped ? 0.0 : yK[c];
+            m[c] = clamped ? 0.0 : yM[c];
         }
+        st3(yk, b, i, k);
+        st3(ym, b, i, m);
     }
     __device__ void done(double (&)[2]) const {}
-    TT_EPI_CALL
 };
 
 struct EpiRaw {  // y = yK + yM, no BC
+    static constexpr int outputs = 1;
+    static constexpr bool uses_input = false;
     double* y;
     TT_NO_PRE
-    template <class S>
-    __device__ void put(int n, uint8_t, const double (&yK)[3], const double (&yM)[3], const S&, const double (&)[3],
+    __device__ void put(size_t b, const LaneOff& i, uint8_t, const double (&yK)[3], const double (&)[3], const double (&)[3],
                         double (&)[2], const Pre&) const {
-#pragma unroll
-        for (int c = 0; c < 3; c++) y[3 * n + c] = yK[c] + yM[c];
+        st3(y, b, i, yK);
     }
     __device__ void done(double (&)[2]) const {}
-    TT_EPI_CALL
 };
 
 struct EpiRHS {  // R = N.(fs F + yK + yM)
+    static constexpr int outputs = 1;
+    static constexpr bool uses_input = false;
     const double* F;
     double fs;
     double* R;
@@ -712,30 +545,25 @@ struct EpiRHS {  // R = N.(fs F + yK + yM)
         double F[3];
     };
     template <class S>
-    __device__ __forceinline__ void fetch(int n, const S&, Pre& p) const {
-#pragma unroll
-        for (int c = 0; c < 3; c++) p.F[c] = F[3 * n + c];
-    }
-    template <class S>
-    __device__ void put(int n, uint8_t cl, const double (&yK)[3], const double (&yM)[3], const S&, const double (&)[3],
-                        double (&)[2], const Pre& p) const {
+    __device__ __forceinline__ void fetch(size_t b, const LaneOff& i, const S&, Pre& p) const { ld3(F, b, i, p.F); }
+    __device__ void put(size_t b, const LaneOff& i, uint8_t cl, const double (&yK)[3], const double (&)[3],
+                        const double (&)[3], double (&)[2], const Pre& p) const {
+        double v[3];
 #pragma unroll
         for (int c = 0; c < 3; c++) {
-            const int i = 3 * n + c;
-            double r = fs * p.F[c];
-            r += yK[c];
-            r += yM[c];
-            R[i] = ((cl >> c) & 1) ? 0.0 : r;
+            v[c] = ((cl >> c) & 1) ? 0.0 : fma(fs, p.F[c], yK[c]);
         }
+        st3(R, b, i, v);
     }
     __device__ void done(double (&)[2]) const {}
-    TT_EPI_CALL
 };
 
 // Flexible-CG direction and its product, with z staged (A z from the contraction): p = z + beta p_old,
 // q = A p = A z + beta q_old (p_old, q_old read at the owned node), partials of p.q.  beta from k_fcg_beta
 // (0 on a (re)start).
 struct EpiFcg {
+    static constexpr int outputs = 1;
+    static constexpr bool uses_input = true;
     double* pnew;
     double* q;
     const double* pold;
@@ -744,157 +572,61 @@ struct EpiFcg {
     int first;
     double* part;
     struct Pre {
-        double p[3], q[3], beta;
+        double p[3], q[3];
     };
     template <class S>
-    __device__ __forceinline__ void fetch(int n, const S&, Pre& pr) const {
-        pr.beta = first ? 0.0 : scal[SC_BETA];
-#pragma unroll
-        for (int c = 0; c < 3; c++) {
-            pr.p[c] = first ? 0.0 : pold[3 * n + c];
-            pr.q[c] = first ? 0.0 : qold[3 * n + c];
+    __device__ __forceinline__ void fetch(size_t b, const LaneOff& i, const S&, Pre& pr) const {
+        if (!first) {
+            ld3(pold, b, i, pr.p);
+            ld3(qold, b, i, pr.q);
         }
     }
-    template <class S>
-    __device__ void put(int n, uint8_t cl, const double (&yK)[3], const double (&yM)[3], const S& st,
+    __device__ void put(size_t b, const LaneOff& i, uint8_t cl, const double (&yK)[3], const double (&)[3],
                         const double (&uo)[3], double (&acc)[2], const Pre& pr) const {
+        double p[3], v[3];
+        const double beta = first ? 0.0 : scal[SC_BETA];  // (uniform)
 #pragma unroll
         for (int c = 0; c < 3; c++) {
-            const int i = 3 * n + c;
-            const double z = input_at(st, cl, c, i, uo);
-            const double az = ((cl >> c) & 1) ? z : yK[c] + yM[c];
-            const double p = first ? z : fma(pr.beta, pr.p[c], z);
-            const double v = first ? az : fma(pr.beta, pr.q[c], az);
-            pnew[i] = p;
-            q[i] = v;
-            acc[0] = fma(p, v, acc[0]);
+            const double az = ((cl >> c) & 1) ? uo[c] : yK[c];
+            p[c] = first ? uo[c] : fma(beta, pr.p[c], uo[c]);
+            v[c] = first ? az : fma(beta, pr.q[c], az);
+            acc[0] = fma(p[c], v[c], acc[0]);
         }
+        st3(pnew, b, i, p);
+        st3(q, b, i, v);
     }
     __device__ void done(double (&acc)[2]) const {
         double a[1] = {acc[0]};
         write_partials<1>(a, part);
     }
-    TT_EPI_CALL
 };
-#undef TT_EPI_CALL
 #undef TT_NO_PRE
 
-static inline dim3 apply_grid(const Grid& g) {
-    return dim3((g.nx + TX - 1) / TX, (g.ny + TY - 1) / TY, (g.nz + TZ - 1) / TZ);
-}
-
-// operator kernel family: 1 = element GEMM on the matrix cores (default), 0 = per-node vector FMA
-static int apply_impl() {
-    static int v = -1;
-    if (v < 0) {
-        const char* e = getenv("TT_APPLY_IMPL");
-        v = e ? atoi(e) : 1;
-    }
-    return v;
-}
-
-static int device_cus() {
-    static int cus = 0;
-    if (!cus) {
-        int dev = 0;
-        TT_HIP(hipGetDevice(&dev));
-        TT_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
-        if (cus <= 0) cus = 256;
-    }
-    return cus;
-}
-
-void tile_bc_flags(const Grid& g, const std::vector<uint8_t>& mask, int tz, std::vector<uint8_t>& f) {
-    const int tx = (g.nx + 7) / 8, ty = (g.ny + 7) / 8, tzn = (g.nz + tz - 1) / tz;
-    f.assign((size_t)tx * ty * tzn, 0);
-    // tile a (extent e) stages nodes e a - 1 .. e a + e
-    auto range = [](int i, int e, int nt, int& lo, int& hi) {
-        lo = std::max(0, (i - e) / e - 1);
-        hi = std::min(nt - 1, (i + 1) / e);
-    };
-    for (int k = 0; k < g.nz; k++)
-        for (int j = 0; j < g.ny; j++)
-            for (int i = 0; i < g.nx; i++) {
-                if (!mask[i + (size_t)g.nx * (j + (size_t)g.ny * k)]) continue;
-                int a0, a1, b0, b1, c0, c1;
-                range(i, 8, tx, a0, a1);
-                range(j, 8, ty, b0, b1);
-                range(k, tz, tzn, c0, c1);
-                for (int c = c0; c <= c1; c++)
-                    for (int b = b0; b <= b1; b++)
-                        for (int a = a0; a <= a1; a++)
-                            if (i >= 8 * a - 1 && i <= 8 * a + 8 && j >= 8 * b - 1 && j <= 8 * b + 8 &&
-                                k >= tz * c - 1 && k <= tz * c + tz)
-                                f[a + (size_t)tx * (b + (size_t)ty * c)] = 1;
-            }
-}
-
-// Launch of k_apply_tiles: one block per tile, rounded up to a multiple of 8 for the XCD-aware
-// tile order; returns the block count (= number of reduction partials).
-template <typename T, typename CT, int TZ_, bool MASKIN, class Stage, class Epi>
-static int launch_tiles_ct(const OpLevel& L, const T* AF, int tx, int ty, int tz, T cK, T cM, const Stage& st,
-                           const Epi& epi, hipStream_t s) {
-    const int ntiles = tx * ty * tz;
-    const int nb = 8 * ((ntiles + 7) / 8);
-    hipLaunchKernelGGL((k_apply_tiles<T, CT, TZ_, MASKIN, Stage, Epi>), dim3(nb), dim3(PTile<TZ_>::NTH), 0, s,
-                       gargs(L.g), tx, ty, ntiles, AF, (const CT*)L.kf, (const CT*)L.mf, cK, cM, L.mask,
-                       TZ_ == 4 ? L.tbc4 : L.tbc2, TZ_ == 4 ? L.tab4 : L.tab2, st, epi);
+template <typename T, typename CT, bool MASKIN, class Stage, class Epi>
+static int launch_cols_ct(const OpLevel& L, double cK, double cM, const Stage& st, const Epi& epi, hipStream_t s) {
+    const ColSplit& cs = sizeof(T) == 8 ? L.split64 : L.split32;
+    const ColPlan& p = cs.plan;
+    const int nb = 8 * ((p.ntiles() + 7) / 8);
+    const ModeConst<T>* mc = std::is_same<T, double>::value ? (const ModeConst<T>*)L.modes64 : (const ModeConst<T>*)L.modes32;
+    hipLaunchKernelGGL((k_apply_cols<T, CT, MASKIN, Stage, Epi>), dim3(nb), dim3(256), 0, s, gargs(L.g), p, mc,
+                       (const CT*)L.kf, (const CT*)L.mf, (T)cK, (T)cM, L.mask, cs.bc, st, epi);
     TT_HIP(hipGetLastError());
     return nb;
 }
-template <typename T, int TZ_, bool MASKIN, class Stage, class Epi>
-static int launch_tiles(const OpLevel& L, const T* AF, int tx, int ty, int tz, T cK, T cM, const Stage& st,
-                        const Epi& epi, hipStream_t s) {
+// launch on the level's coefficient kind; returns the block count (= number of reduction partials)
+template <typename T, bool MASKIN, class Stage, class Epi>
+static int run_apply(const OpLevel& L, double cK, double cM, const Stage& st, const Epi& epi, hipStream_t s) {
     switch (L.coef_kind) {
-    case COEF_F64: return launch_tiles_ct<T, double, TZ_, MASKIN>(L, AF, tx, ty, tz, cK, cM, st, epi, s);
-    case COEF_F32: return launch_tiles_ct<T, float, TZ_, MASKIN>(L, AF, tx, ty, tz, cK, cM, st, epi, s);
-    default: return launch_tiles_ct<T, bf16_t, TZ_, MASKIN>(L, AF, tx, ty, tz, cK, cM, st, epi, s);
+    case COEF_F64: return launch_cols_ct<T, double, MASKIN>(L, cK, cM, st, epi, s);
+    case COEF_F32: return launch_cols_ct<T, float, MASKIN>(L, cK, cM, st, epi, s);
+    default: return launch_cols_ct<T, bf16_t, MASKIN>(L, cK, cM, st, epi, s);
     }
 }
 
-// dispatch on coefficient kind and precision
-template <typename T, bool TWO, bool MASKIN, class Stage, class Epi>
-static int run_apply(const OpLevel& L, double cK, double cM, const Stage& st, const Epi& epi, hipStream_t s,
-                     bool allow_mfma = true) {
-    const T* KE = std::is_same<T, double>::value ? (const T*)L.KE64 : (const T*)L.KE32;
-    const T* M8 = std::is_same<T, double>::value ? (const T*)L.M864 : (const T*)L.M832;
-    GridArgs ga = gargs(L.g);
-    if (!TWO && allow_mfma && apply_impl() == 1) {
-        // FP32 runs on the FP16-split fragments, whose K / M rows carry the scales hs
-        const bool f32 = std::is_same<T, float>::value;
-        const T* AF = f32 ? (const T*)L.AFH : (const T*)L.AF64;
-        if (f32) {
-            cK *= L.hs[0];
-            cM *= L.hs[1];
-        }
-        // 8x8x4 tiles on grids with enough of them to fill the chip, 8x8x2 on the coarse levels
-        const int tx = (L.g.nx + 7) / 8, ty = (L.g.ny + 7) / 8;
-        const bool deep = (long)tx * ty * ((L.g.nz + 3) / 4) >= 4L * device_cus();
-        if (deep) return launch_tiles<T, 4, MASKIN>(L, AF, tx, ty, (L.g.nz + 3) / 4, (T)cK, (T)cM, st, epi, s);
-        return launch_tiles<T, 2, MASKIN>(L, AF, tx, ty, (L.g.nz + 1) / 2, (T)cK, (T)cM, st, epi, s);
-    }
-    dim3 grid = apply_grid(L.g);
-    switch (L.coef_kind) {
-    case COEF_F64:
-        hipLaunchKernelGGL((k_apply<T, double, TWO, MASKIN, Stage, Epi>), grid, dim3(NT), 0, s, ga, KE, M8,
-                           (const double*)L.kf, (const double*)L.mf, (T)cK, (T)cM, L.mask, st, epi);
-        break;
-    case COEF_F32:
-        hipLaunchKernelGGL((k_apply<T, float, TWO, MASKIN, Stage, Epi>), grid, dim3(NT), 0, s, ga, KE, M8,
-                           (const float*)L.kf, (const float*)L.mf, (T)cK, (T)cM, L.mask, st, epi);
-        break;
-    default:
-        hipLaunchKernelGGL((k_apply<T, bf16_t, TWO, MASKIN, Stage, Epi>), grid, dim3(NT), 0, s, ga, KE, M8,
-                           (const bf16_t*)L.kf, (const bf16_t*)L.mf, (T)cK, (T)cM, L.mask, st, epi);
-        break;
-    }
-    TT_HIP(hipGetLastError());
-    return (int)(grid.x * grid.y * grid.z);
-}
-
-// upper bound of the blocks of any apply launch on grid g (8x8x2 tiles, rounded up to a multiple of 8)
-static inline int apply_nblocks(const Grid& g) {
-    return 8 * ((((g.nx + 7) / 8) * ((g.ny + 7) / 8) * ((g.nz + 1) / 2) + 7) / 8);
+// the blocks of an apply launch on this level must fit the reducer's partial regions
+static inline void check_partials(const OpLevel& L, const Reducer& red) {
+    const int nt = std::max(L.split64.plan.ntiles(), L.split32.plan.ntiles());
+    TT_CHECK(8 * ((nt + 7) / 8) <= red.maxblocks, -3, "reducer too small");
 }
 
 void launch_apply_bc(const OpLevel& L, double cK, double cM, const void* u, void* y, bool fp64, hipStream_t s,
@@ -902,22 +634,22 @@ void launch_apply_bc(const OpLevel& L, double cK, double cM, const void* u, void
     if (fp64) {
         StageOne<double> st{(const double*)u};
         if (red) {
-            TT_CHECK(apply_nblocks(L.g) <= red->maxblocks, -3, "reducer too small");
+            check_partials(L, *red);
             EpiBCDot<double> e{(double*)y, red->part(dot_slot)};
-            red->nblk[dot_slot] = run_apply<double, false, true>(L, cK, cM, st, e, s);
+            red->nblk[dot_slot] = run_apply<double, true>(L, cK, cM, st, e, s);
             red->nv[dot_slot] = 1;
         } else {
-            run_apply<double, false, true>(L, cK, cM, st, EpiBC<double>{(double*)y}, s);
+            run_apply<double, true>(L, cK, cM, st, EpiBC<double>{(double*)y}, s);
         }
     } else {
         StageOne<float> st{(const float*)u};
         if (red) {
-            TT_CHECK(apply_nblocks(L.g) <= red->maxblocks, -3, "reducer too small");
+            check_partials(L, *red);
             EpiBCDot<float> e{(float*)y, red->part(dot_slot)};
-            red->nblk[dot_slot] = run_apply<float, false, true>(L, cK, cM, st, e, s);
+            red->nblk[dot_slot] = run_apply<float, true>(L, cK, cM, st, e, s);
             red->nv[dot_slot] = 1;
         } else {
-            run_apply<float, false, true>(L, cK, cM, st, EpiBC<float>{(float*)y}, s);
+            run_apply<float, true>(L, cK, cM, st, EpiBC<float>{(float*)y}, s);
         }
     }
 }
@@ -925,30 +657,30 @@ void launch_apply_bc(const OpLevel& L, double cK, double cM, const void* u, void
 void launch_residual(const OpLevel& L, double cK, double cM, const void* b, const void* x, void* r, bool fp64,
                      hipStream_t s) {
     if (fp64)
-        run_apply<double, false, true>(L, cK, cM, StageOne<double>{(const double*)x},
+        run_apply<double, true>(L, cK, cM, StageOne<double>{(const double*)x},
                                        EpiResid<double>{(const double*)b, (double*)r}, s);
     else
-        run_apply<float, false, true>(L, cK, cM, StageOne<float>{(const float*)x},
+        run_apply<float, true>(L, cK, cM, StageOne<float>{(const float*)x},
                                       EpiResid<float>{(const float*)b, (float*)r}, s);
 }
 
 void launch_resid_first(const OpLevel& L, double cK, double cM, const void* b, const void* dinv, double c1, void* x,
                         void* r, bool fp64, hipStream_t s) {
     if (fp64)
-        run_apply<double, false, true>(
+        run_apply<double, true>(
             L, cK, cM, StageChebFirst<double, false>{nullptr, (const double*)b, (const double*)dinv, c1},
             EpiResidFirst<double>{(double*)x, (double*)r}, s);
     else
-        run_apply<float, false, true>(
+        run_apply<float, true>(
             L, cK, cM, StageChebFirst<float, false>{nullptr, (const float*)b, (const float*)dinv, (float)c1},
             EpiResidFirst<float>{(float*)x, (float*)r}, s);
 }
 
 void launch_residual_dots(const OpLevel& L, double cK, double cM, const double* b, const double* x, double* r,
                           Reducer& red, int bb_region, int rr_region, hipStream_t s) {
-    TT_CHECK(apply_nblocks(L.g) <= red.maxblocks, -3, "reducer too small");
+    check_partials(L, red);
     EpiResidDots e{b, r, red.part(bb_region), red.part(rr_region)};
-    const int nb = run_apply<double, false, true>(L, cK, cM, StageOne<double>{x}, e, s);
+    const int nb = run_apply<double, true>(L, cK, cM, StageOne<double>{x}, e, s);
     red.nblk[bb_region] = red.nblk[rr_region] = nb;
     red.nv[bb_region] = red.nv[rr_region] = 1;
 }
@@ -957,11 +689,11 @@ void launch_cheb_step(const OpLevel& L, double cK, double cM, const void* b, con
                       const void* dinv, double c0, double c1, void* xn, void* dn, bool fp64, hipStream_t s) {
     if (fp64) {
         EpiCheb<double> e{(const double*)b, (const double*)d, (const double*)dinv, c0, c1, (double*)xn, (double*)dn};
-        run_apply<double, false, true>(L, cK, cM, StageOne<double>{(const double*)x}, e, s);
+        run_apply<double, true>(L, cK, cM, StageOne<double>{(const double*)x}, e, s);
     } else {
         EpiCheb<float> e{(const float*)b,  (const float*)d, (const float*)dinv, (float)c0,
                          (float)c1,        (float*)xn,      (float*)dn};
-        run_apply<float, false, true>(L, cK, cM, StageOne<float>{(const float*)x}, e, s);
+        run_apply<float, true>(L, cK, cM, StageOne<float>{(const float*)x}, e, s);
     }
 }
 
@@ -970,22 +702,22 @@ void launch_cheb_first_step(const OpLevel& L, double cK, double cM, const double
     if (fp64) {
         const double* dv = (const double*)dinv;
         if (r64)
-            run_apply<double, false, true>(L, cK, cM, StageChebFirst<double, true>{r64, nullptr, dv, c1_first},
+            run_apply<double, true>(L, cK, cM, StageChebFirst<double, true>{r64, nullptr, dv, c1_first},
                                            EpiChebFirst<double, true>{(double*)b, dv, c0, c1, (double*)xn,
                                                                       (double*)dn}, s);
         else
-            run_apply<double, false, true>(L, cK, cM,
+            run_apply<double, true>(L, cK, cM,
                                            StageChebFirst<double, false>{nullptr, (const double*)b, dv, c1_first},
                                            EpiChebFirst<double, false>{nullptr, dv, c0, c1, (double*)xn,
                                                                        (double*)dn}, s);
     } else {
         const float* dv = (const float*)dinv;
         if (r64)
-            run_apply<float, false, true>(L, cK, cM, StageChebFirst<float, true>{r64, nullptr, dv, (float)c1_first},
+            run_apply<float, true>(L, cK, cM, StageChebFirst<float, true>{r64, nullptr, dv, (float)c1_first},
                                           EpiChebFirst<float, true>{(float*)b, dv, (float)c0, (float)c1,
                                                                     (float*)xn, (float*)dn}, s);
         else
-            run_apply<float, false, true>(L, cK, cM,
+            run_apply<float, true>(L, cK, cM,
                                           StageChebFirst<float, false>{nullptr, (const float*)b, dv, (float)c1_first},
                                           EpiChebFirst<float, false>{nullptr, dv, (float)c0, (float)c1, (float*)xn,
                                                                      (float*)dn}, s);
@@ -995,22 +727,22 @@ void launch_cheb_first_step(const OpLevel& L, double cK, double cM, const double
 void launch_cheb_last(const OpLevel& L, double cK, double cM, const void* b, const void* x, const void* d,
                       const void* dinv, double c0, double c1, double* z, const double* r, const double* rp, bool first,
                       bool fp64, Reducer& red, hipStream_t s) {
-    TT_CHECK(apply_nblocks(L.g) <= red.maxblocks, -3, "reducer too small");
+    check_partials(L, red);
     if (fp64) {
         EpiChebOut<double> e{(const double*)b, (const double*)d, (const double*)dinv, c0, c1, z, r, rp,
                              first ? 1 : 0, red.part(PB_DOTS)};
-        red.nblk[PB_DOTS] = run_apply<double, false, true>(L, cK, cM, StageOne<double>{(const double*)x}, e, s);
+        red.nblk[PB_DOTS] = run_apply<double, true>(L, cK, cM, StageOne<double>{(const double*)x}, e, s);
     } else {
         EpiChebOut<float> e{(const float*)b, (const float*)d, (const float*)dinv, (float)c0, (float)c1, z, r, rp,
                             first ? 1 : 0, red.part(PB_DOTS)};
-        red.nblk[PB_DOTS] = run_apply<float, false, true>(L, cK, cM, StageOne<float>{(const float*)x}, e, s);
+        red.nblk[PB_DOTS] = run_apply<float, true>(L, cK, cM, StageOne<float>{(const float*)x}, e, s);
     }
     red.nv[PB_DOTS] = 2;
 }
 
 void launch_apply_split(const OpLevel& L, double cK, double cM, const double* u, double* yk, double* ym,
                         hipStream_t s) {
-    run_apply<double, false, true>(L, cK, cM, StageOne<double>{u}, EpiSplit{yk, ym}, s, false);
+    run_apply<double, true>(L, cK, cM, StageOne<double>{u}, EpiSplit{yk, ym}, s);
 }
 
 void launch_apply_raw(const OpLevel& L, const double* kf, const double* mf, double cK, double cM, const double* u,
@@ -1019,13 +751,13 @@ void launch_apply_raw(const OpLevel& L, const double* kf, const double* mf, doub
     L2.kf = kf;
     L2.mf = mf;
     L2.coef_kind = COEF_F64;
-    run_apply<double, false, false>(L2, cK, cM, StageOne<double>{u}, EpiRaw{y}, s);
+    run_apply<double, false>(L2, cK, cM, StageOne<double>{u}, EpiRaw{y}, s);
 }
 
 void launch_newmark_rhs(const OpLevel& L, const double* u, const double* v, const double* a, const double* F,
                         double fs, const double wK[3], const double wM[3], double* R, hipStream_t s) {
     StageThree st{u, v, a, wK[0], wK[1], wK[2], wM[0], wM[1], wM[2]};
-    run_apply<double, true, true>(L, 1.0, 1.0, st, EpiRHS{F, fs, R}, s);
+    run_apply<double, true>(L, 1.0, 1.0, st, EpiRHS{F, fs, R}, s);
 }
 
 // single-block reductions of partials: 1024 threads, so each sums ~5 of the ~5000 partials of a
@@ -1035,14 +767,14 @@ __global__ __launch_bounds__(BSR) void k_fcg_beta(const double* __restrict__ dot
                                                   int first);
 void launch_fcg_apply(const OpLevel& L, double cK, double cM, const double* z, const double* p_old, double* p_new,
                       const double* q_old, double* q_new, Reducer& red, bool first, hipStream_t s, bool beta) {
-    TT_CHECK(apply_nblocks(L.g) <= red.maxblocks, -3, "reducer too small");
+    check_partials(L, red);
     if (beta) {
         hipLaunchKernelGGL(k_fcg_beta, dim3(1), dim3(BSR), 0, s, red.part(PB_DOTS), red.nblk[PB_DOTS], red.scal.p,
                            first ? 1 : 0);
         TT_HIP(hipGetLastError());
     }
     EpiFcg e{p_new, q_new, p_old, q_old, red.scal.p, first ? 1 : 0, red.part(PB_PQ)};
-    red.nblk[PB_PQ] = run_apply<double, false, true>(L, cK, cM, StageOne<double>{z}, e, s);
+    red.nblk[PB_PQ] = run_apply<double, true>(L, cK, cM, StageOne<double>{z}, e, s);
     red.nv[PB_PQ] = 1;
 }
 

@@ -71,38 +71,14 @@ void Multigrid::build(Context* c, int nlvls, bool mixed_prec, int deg) {
         build_mask(g, c->prm.boundaries, m);
         lev->mask.alloc(g.nn);
         TT_HIP(hipMemcpy(lev->mask.p, m.data(), g.nn, hipMemcpyHostToDevice));
-        {
-            std::vector<uint8_t> f;
-            tile_bc_flags(g, m, 4, f);
-            lev->tbc4.alloc(f.size());
-            TT_HIP(hipMemcpy(lev->tbc4.p, f.data(), f.size(), hipMemcpyHostToDevice));
-            tile_bc_flags(g, m, 2, f);
-            lev->tbc2.alloc(f.size());
-            TT_HIP(hipMemcpy(lev->tbc2.p, f.data(), f.size(), hipMemcpyHostToDevice));
-        }
+        lev->split.build(g, m);
         double ke[576], m8[64];
         hex8_stiffness(g.hx, g.hy, g.hz, c->prm.nu, ke);
         hex8_mass(g.hx, g.hy, g.hz, m8);
-        float ke32[576], m832[64];
-        for (int i = 0; i < 576; i++) ke32[i] = (float)ke[i];
-        for (int i = 0; i < 64; i++) m832[i] = (float)m8[i];
         lev->KE64.alloc(576);
         lev->M864.alloc(64);
-        lev->KE32.alloc(576);
-        lev->M832.alloc(64);
         TT_HIP(hipMemcpy(lev->KE64.p, ke, sizeof(ke), hipMemcpyHostToDevice));
         TT_HIP(hipMemcpy(lev->M864.p, m8, sizeof(m8), hipMemcpyHostToDevice));
-        TT_HIP(hipMemcpy(lev->KE32.p, ke32, sizeof(ke32), hipMemcpyHostToDevice));
-        TT_HIP(hipMemcpy(lev->M832.p, m832, sizeof(m832), hipMemcpyHostToDevice));
-        {
-            double af64[18 * 64];
-            float af32[AF32_WORDS];
-            mfma_fragments(ke, m8, af64, af32, reinterpret_cast<uint32_t*>(af32 + 18 * 64), lev->op.hs);
-            lev->AF64.alloc(18 * 64);
-            lev->AF32.alloc(AF32_WORDS);
-            TT_HIP(hipMemcpy(lev->AF64.p, af64, sizeof(af64), hipMemcpyHostToDevice));
-            TT_HIP(hipMemcpy(lev->AF32.p, af32, sizeof(af32), hipMemcpyHostToDevice));
-        }
         if (l > 0) {
             lev->kf64.alloc(g.nel);
             lev->mf64.alloc(g.nel);
@@ -119,18 +95,13 @@ void Multigrid::build(Context* c, int nlvls, bool mixed_prec, int deg) {
             b->alloc(g.nd * es);
         lev->op.g = g;
         lev->op.mask = lev->mask.p;
-        lev->op.tbc4 = lev->tbc4.p;
-        lev->op.tbc2 = lev->tbc2.p;
-        build_batch_tables(g, lev->btab);
-        lev->op.tab4 = lev->btab.t4;
-        lev->op.tab2 = lev->btab.t2;
+        lev->op.split32 = lev->split.s32;
+        lev->op.split64 = lev->split.s64;
+        upload_modes(ke, m8, lev->modes64, lev->modes32);
+        lev->op.modes64 = lev->modes64.p;
+        lev->op.modes32 = lev->modes32.p;
         lev->op.KE64 = lev->KE64.p;
         lev->op.M864 = lev->M864.p;
-        lev->op.KE32 = lev->KE32.p;
-        lev->op.M832 = lev->M832.p;
-        lev->op.AF64 = lev->AF64.p;
-        lev->op.AF32 = lev->AF32.p;
-        lev->op.AFH = reinterpret_cast<const uint32_t*>(lev->AF32.p + 18 * 64);
         L.push_back(std::move(lev));
     }
     const Grid& gc = L.back()->g;

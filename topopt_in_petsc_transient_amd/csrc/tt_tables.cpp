@@ -1,6 +1,7 @@
-// Batch tables of the tile kernels (k_apply_tiles, tt_apply_mfma.inc): for each tile position in the grid
-// (first / interior / last tile in each direction, 64 per tile depth), the tile's elements in batches of 16
-// that share no node, with the slot words the kernel reads.  Host code, built once per grid.
+// Batch tables of 8 x 8 node tiles: for each tile position in the grid (first / interior / last tile in each direction,
+// 64 per tile depth), the tile's elements in batches of 16 that share no node.  No kernel of the library reads them since
+// the operator runs column by column (tt_apply_cols.inc); the file is not part of the library and stays for the test of
+// its invariants.
 #include <algorithm>
 #include <cstdlib>
 #include <vector>
