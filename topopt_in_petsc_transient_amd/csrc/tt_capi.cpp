@@ -138,7 +138,7 @@ Context::Context(const tt_params& p) : prm(p) {
 
     mg.build(this, p.nlvls, p.precision == TT_PREC_MIXED, p.cheb_degree);
 
-    for (DBuf<double>* b : {&kr, &krp, &kz, &kp0, &kp1, &kq, &kq2, &dinvM, &kx, &lam, &lamh[0], &lamh[1], &lamh[2], &lamh[3], &lamh[4], &lamh[5], &lamh[6], &lamh[7], &lamT, &mu, &nu, &mun, &nun, &hdu,
+    for (DBuf<double>* b : {&kr, &kz, &kp0, &kp1, &kq, &kq2, &dinvM, &kx, &lam, &lamh[0], &lamh[1], &lamh[2], &lamh[3], &lamh[4], &lamh[5], &lamh[6], &lamh[7], &lamT, &mu, &nu, &mun, &nun, &hdu,
                             &hddu, &hdddu, &Kl, &Ml, &rhs, &nu0})
         b->alloc(nd);
     TT_HIP(hipMemsetAsync(lamT.p, 0, nd * 8, stream));
@@ -178,7 +178,7 @@ Context::Context(const tt_params& p) : prm(p) {
     // PDE filter (PDEFilter.cc:28-191) on the same node grid
     fg = g;
     KFd.alloc(64);
-    for (DBuf<double>* b : {&fdinv, &fU, &frhs, &fr, &frp, &fz, &fp, &fp2, &fq}) b->alloc(nn);
+    for (DBuf<double>* b : {&fdinv, &fU, &frhs, &fr, &fz, &fp, &fp2, &fq}) b->alloc(nn);
     set_filter_radius(p.rmin);
 }
 
@@ -234,10 +234,10 @@ void Context::pde_filter(const double* in, double* out) {
     for (;;) {
         while (it < next_look) {
             launch_jacobi(fdinv.p, fr.p, fz.p, nn, stream);
-            launch_fcg_dots(fz.p, fr.p, frp.p, nn, red, first, stream);
+            launch_fcg_dots(fz.p, fr.p, fq.p, nn, red, first, stream);
             launch_fcg_direction(fz.p, pold, pnew, nn, red, first, stream);
             launch_filter_apply(fg, KFd.p, pnew, fq.p, &red, PB_PQ, stream);
-            launch_fcg_update(fU.p, pnew, fr.p, frp.p, fq.p, nn, red, first, stream);
+            launch_fcg_update(fU.p, pnew, fr.p, fq.p, nn, red, first, pnew == fp.p, stream);
             std::swap(pold, pnew);
             first = false;
             it++;
@@ -245,7 +245,7 @@ void Context::pde_filter(const double* in, double* out) {
         wait_look();
         double rr = 0.0;
         const volatile double* lk = red.look;
-        const int nb = red.nblk[PB_RR];
+        const int nb = red.nblk[rr_region(pold == fp.p)];
         for (int i = 0; i < nb; i++) rr += lk[i];
         const double bb = lk[Reducer::kLookBB];
         if (!std::isfinite(rr) || !std::isfinite(bb)) throw Error{TT_ERR_NONFINITE, "non-finite PDE filter input or residual"};
@@ -257,8 +257,8 @@ void Context::pde_filter(const double* in, double* out) {
             // confirm with the true residual; restart the recursion if it drifted
             launch_filter_apply(fg, KFd.p, fU.p, fq.p, nullptr, 0, stream);
             launch_lincomb(1.0, frhs.p, -1.0, fq.p, fr.p, nn, stream);
-            launch_dot(fr.p, fr.p, nn, red, PB_RR, stream);
-            rel = std::sqrt(reduce1(PB_RR) / bb);
+            launch_dot(fr.p, fr.p, nn, red, PB_MISC2, stream);
+            rel = std::sqrt(reduce1(PB_MISC2) / bb);
             if (rel <= tol) break;
             start(false);
             first = true;
@@ -564,20 +564,27 @@ int tt_time_fcg_apply(tt_ctx* ctx, int nrep, double* ms) {
     TT_CHECK(ms && nrep > 0, TT_ERR_ARG, "bad tt_time_fcg_apply arguments");
     const long nd = C.g.nd;
     // the flexible-CG apply of a Krylov iteration on the context's own vectors: z, p_old and q_old from a
-    // deterministic hash, beta = 0.5, then nrep launches of the tile kernel (the beta kernel excluded)
+    // deterministic hash, dot partials that give beta = 0.5, then nrep launches
     tt::launch_fill_hash(C.kz.p, nd, 0x51ED270B27A1F00Dull, true, C.stream);
     tt::launch_fill_hash(C.kp0.p, nd, 0x2F1C3A5B4D6E7F81ull, true, C.stream);
-    tt::launch_fill(C.red.scal.p + tt::SC_BETA, 0.5, 1, true, C.stream);
     tt::launch_fill_hash(C.kq2.p, nd, 0x7C3B1A9E5D2F4681ull, true, C.stream);
-    tt::launch_fcg_apply(C.op_fine64, C.cK_A, C.cM_A, C.kz.p, C.kp0.p, C.kp1.p, C.kq2.p, C.kq.p, C.red, false, C.stream,
-                         false);
+    const int nparts = 8 * ((C.split.s64.plan.ntiles() + 7) / 8);
+    double* dots = C.red.part(tt::PB_DOTS);
+    tt::launch_fill(dots, 0.0, 2 * nparts, true, C.stream);
+    tt::launch_fill(dots, 1.0, 1, true, C.stream);
+    tt::launch_fill(dots + 1, -0.5, 1, true, C.stream);
+    C.red.nblk[tt::PB_DOTS] = nparts;
+    tt::launch_fill(C.red.scal.p + tt::SC_DONE, 0.0, 1, true, C.stream);
+    tt::launch_fill(C.red.scal.p + tt::SC_ALPHA, 1.0, 1, true, C.stream);
+    tt::launch_fill(C.red.scal.p + tt::SC_GAMMA_OLD, 1.0, 1, true, C.stream);
+    tt::launch_fcg_apply(C.op_fine64, C.cK_A, C.cM_A, C.kz.p, C.kp0.p, C.kp1.p, C.kq2.p, C.kq.p, C.red, false, C.stream);
     hipEvent_t e0, e1;
     TT_HIP(hipEventCreate(&e0));
     TT_HIP(hipEventCreate(&e1));
     TT_HIP(hipEventRecord(e0, C.stream));
     for (int i = 0; i < nrep; i++)
         tt::launch_fcg_apply(C.op_fine64, C.cK_A, C.cM_A, C.kz.p, C.kp0.p, C.kp1.p, C.kq2.p, C.kq.p, C.red, false,
-                             C.stream, false);
+                             C.stream);
     TT_HIP(hipEventRecord(e1, C.stream));
     TT_HIP(hipEventSynchronize(e1));
     float t = 0.0f;
@@ -594,15 +601,15 @@ int tt_time_vcycle(tt_ctx* ctx, int nrep, double* ms_gpu, double* ms_host) {
     TT_CHECK(ms_gpu && ms_host && nrep > 0, TT_ERR_ARG, "bad tt_time_vcycle arguments");
     const long nd = C.g.nd;
     tt::launch_fill_hash(C.kr.p, nd, 0x3C6EF372FE94F82Bull, true, C.stream);
-    tt::launch_fill_hash(C.krp.p, nd, 0x6A09E667F3BCC908ull, true, C.stream);
-    C.mg.apply_fcg(C.kr.p, C.krp.p, C.kz.p, true);
+    tt::launch_fill_hash(C.kq2.p, nd, 0x6A09E667F3BCC908ull, true, C.stream);
+    C.mg.apply_fcg(C.kr.p, C.kq2.p, C.kz.p, true);
     C.sync();
     hipEvent_t e0, e1;
     TT_HIP(hipEventCreate(&e0));
     TT_HIP(hipEventCreate(&e1));
     TT_HIP(hipEventRecord(e0, C.stream));
     const auto h0 = std::chrono::steady_clock::now();
-    for (int i = 0; i < nrep; i++) C.mg.apply_fcg(C.kr.p, C.krp.p, C.kz.p, i == 0);
+    for (int i = 0; i < nrep; i++) C.mg.apply_fcg(C.kr.p, C.kq2.p, C.kz.p, i == 0);
     const auto h1 = std::chrono::steady_clock::now();
     TT_HIP(hipEventRecord(e1, C.stream));
     TT_HIP(hipEventSynchronize(e1));

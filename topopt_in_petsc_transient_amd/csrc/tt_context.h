@@ -72,12 +72,12 @@ struct Multigrid {
     void setup_operator(double cK_, double cM_);
     // z = B r (FP64 in and out)
     void apply(const double* r, double* z);
-    // z = B r as the flexible-CG preconditioner, also leaving the partials of z.r and z.r_prev
-    // (r_prev ignored when first) in the reducer's PB_DOTS region
-    void apply_fcg(const double* r, const double* rp, double* z, bool first);
+    // z = B r as the flexible-CG preconditioner, also leaving the partials of z.r and z.q_old
+    // (q_old ignored when first) in the reducer's PB_DOTS region
+    void apply_fcg(const double* r, const double* q_old, double* z, bool first);
 
    private:
-    void vcycle(int l, const double* r64 = nullptr, double* z64 = nullptr, const double* rp64 = nullptr,
+    void vcycle(int l, const double* r64 = nullptr, double* z64 = nullptr, const double* q64 = nullptr,
                 bool first = false);
     void coarse_solve(bool direct64);
     double power_lmax(int l, int iters);
@@ -126,7 +126,7 @@ struct Context {
     Multigrid mg;
 
     // Krylov work vectors (FP64, nd); kx holds the solution of a graph-replayed solve
-    DBuf<double> kr, krp, kz, kp0, kp1, kq, kq2, dinvM, kx;
+    DBuf<double> kr, kz, kp0, kp1, kq, kq2, dinvM, kx;
 
     // One multigrid-preconditioned flexible-CG iteration captured as a HIP graph, keyed by everything
     // its launches bake in (pointers of the rotating buffers, first-iteration flag, operator scalars),
@@ -162,7 +162,7 @@ struct Context {
 
     // PDE filter
     double KF[64];
-    DBuf<double> KFd, fdinv, fU, frhs, fr, frp, fz, fp, fp2, fq, ftmp_e, ftmp_e2;
+    DBuf<double> KFd, fdinv, fU, frhs, fr, fz, fp, fp2, fq, ftmp_e, ftmp_e2;
     int filter_iters = 0;  // iterations of the last filter solve (when the host first reads the residual)
     Grid fg{};
 

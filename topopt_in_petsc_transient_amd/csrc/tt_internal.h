@@ -135,7 +135,7 @@ struct ColSplitStore {  // the splits of one grid, by precision, with their flag
 // stream (or the host) sums the partials in block order.  Kernel boundaries
 // give the visibility, so no block pays a device-scope fence (which on a
 // multi-XCD GPU means an L2 write-back).
-enum { PB_DOTS = 0, PB_PQ, PB_RR, PB_MISC, PB_MISC2, PB_COUNT };
+enum { PB_DOTS = 0, PB_PQ, PB_RR, PB_RR2, PB_MISC, PB_MISC2, PB_COUNT };
 struct Reducer {
     DBuf<double> partials;   // PB_COUNT regions of [maxblocks * 4]
     DBuf<double> scal;       // device scalars (see SC_* indices)
@@ -160,10 +160,7 @@ struct Reducer {
 enum {
     SC_GAMMA = 0,   // z.r of current iteration
     SC_GAMMA_OLD,   // z.r of previous iteration
-    SC_DELTA,       // z.r_prev
-    SC_BETA,
-    SC_PQ,
-    SC_ALPHA,
+    SC_ALPHA,       // step length of the last update
     SC_RR,          // r.r
     SC_TMP0,
     SC_TMP1,
@@ -276,11 +273,11 @@ void launch_newmark_rhs(const OpLevel& L, const double* u, const double* v, cons
 // diagonal of (cK K + cM M) with identity on clamped dofs, inverted
 void launch_diag_inv(const OpLevel& L, double cK, double cM, void* dinv, bool fp64, hipStream_t s);
 
-// FCG fused apply: p = z + beta p_old (beta from scal) and q = A p = A z + beta q_old, partial p.q ->
-// alpha = gamma / pq.  Only z is staged with its halo; p_old and q_old are read at the owned nodes.
-// beta = false: the tile kernel alone, with the beta already in scal (measurement)
+// FCG fused apply: p = z + beta p_old and q = A p = A z + beta q_old, partials of p.q.  Only z is staged with its halo;
+// p_old and q_old are read at the owned nodes.  Every block forms beta itself from the z.r and z.q_old partials
+// (PB_DOTS): with r = r_prev - alpha q_old, beta = (z.r - z.r_prev) / gamma_old = -alpha z.q_old / gamma_old.
 void launch_fcg_apply(const OpLevel& L, double cK, double cM, const double* z, const double* p_old, double* p_new,
-                      const double* q_old, double* q_new, Reducer& red, bool first, hipStream_t s, bool beta = true);
+                      const double* q_old, double* q_new, Reducer& red, bool first, hipStream_t s);
 
 // vector kernels
 void launch_fill(void* x, double v, long n, bool fp64, hipStream_t s);
@@ -293,9 +290,9 @@ void launch_cheb_first_from64(const double* r, void* b, const void* dinv, double
 // (b = (T) r64 written out when r64 is given), then dn = c0 x0 + c1 D^-1 (b - A x0), xn = x0 + dn
 void launch_cheb_first_step(const OpLevel& L, double cK, double cM, const double* r64, void* b, const void* dinv,
                             double c1_first, double c0, double c1, void* xn, void* dn, bool fp64, hipStream_t s);
-// last post-smoothing step of the finest level: z (FP64) = x + dn, partials of z.r and z.r_prev into PB_DOTS
+// last post-smoothing step of the finest level: z (FP64) = x + dn, partials of z.r and z.q_old into PB_DOTS
 void launch_cheb_last(const OpLevel& L, double cK, double cM, const void* b, const void* x, const void* d,
-                      const void* dinv, double c0, double c1, double* z, const double* r, const double* rp, bool first,
+                      const void* dinv, double c0, double c1, double* z, const double* r, const double* q, bool first,
                       bool fp64, Reducer& red, hipStream_t s);
 // bc = R rf (fine precision fp64; an FP32 fine level may write an FP64 coarse vector, out64)
 void launch_restrict(const Grid& fine, const Grid& coarse, const void* rf, const uint8_t* cmask, void* bc,
@@ -324,21 +321,24 @@ struct Expand3 {
     int nb, nout;
 };
 void launch_expand3(const Expand3& e, long n, hipStream_t s);
-void launch_fcg_dots(const double* z, const double* r, const double* rprev, long n, Reducer& red, bool first,
+// partials of z.r and z.q_old (PB_DOTS)
+void launch_fcg_dots(const double* z, const double* r, const double* q_old, long n, Reducer& red, bool first,
                      hipStream_t s);
 // Flexible-CG (re)start from the b.b and r.r partial regions: device tolerance (rtol ||b||)^2, the
 // b = 0 flag, and whether the current x already meets the tolerance.
-// reset_iters: a new solve (SC_ITERS = 0) rather than a restart of the same one.  After every
-// launch_fcg_update the PB_RR region holds nblk partials of r.r followed by SC_ITERS.
+// reset_iters: a new solve (SC_ITERS = 0) rather than a restart of the same one.
 void launch_fcg_init(Reducer& red, int bb_region, int rr_region, double rtol2, bool reset_iters, hipStream_t s);
 // x += alpha p, r -= alpha q with alpha = gamma / p.q, unless x already met the tolerance (set at the
 // (re)start, or by the previous update's r.r after its first iteration): then alpha = 0 from there on,
-// so the result does not depend on when the host looks at the residual.  x = 0 if b = 0.
-void launch_fcg_update(double* x, const double* p, double* r, double* rprev, const double* q, long n, Reducer& red,
-                       bool first, hipStream_t s);
+// so the result does not depend on when the host looks at the residual.  x = 0 if b = 0.  Every block forms alpha
+// itself from the p.q partials and the previous update's r.r; odd: the parity of the iteration (its r.r partials go to
+// region rr_region(odd), the previous update's are in the other one).
+inline int rr_region(bool odd) { return odd ? PB_RR2 : PB_RR; }
+void launch_fcg_update(double* x, const double* p, double* r, const double* q, long n, Reducer& red, bool first,
+                       bool odd, hipStream_t s);
 void launch_jacobi(const double* dinv, const double* r, double* z, long n, hipStream_t s);
-// Flexible-CG direction for a matrix without a fused apply kernel: beta from the z.r / z.r_prev partials
-// of launch_fcg_dots (0 on a (re)start), then p_new = z + beta p_old.
+// Flexible-CG direction for a matrix without a fused apply kernel: beta from the partials of launch_fcg_dots (0 on a
+// (re)start), then p_new = z + beta p_old.
 void launch_fcg_direction(const double* z, const double* p_old, double* p_new, long n, Reducer& red, bool first,
                           hipStream_t s);
 // power iteration: x = dinv.Ax with partials of ||x||^2 in PB_MISC; then x /= ||x||

@@ -258,7 +258,7 @@ struct StageThree {  // wK = sum_i cK_i in_i, wM = sum_i cM_i in_i (FP64)
 // ---- epilogues.  A node's three dofs are b + i .. b + i + 2, b uniform over the block (its node plane's first dof, or
 // 0).  fetch() loads the per-node operands an epilogue reads (its Pre) for one owned node, ahead of the element
 // contraction.  put() then handles that node (inside the grid): cl are its clamped dofs, uo its input values (not
-// masked); it may add to the thread's reduction share.  done() is called once by every thread of the block at the end
+// masked); it may add to the thread's reduction share.  prologue() runs first, on every thread of every block.  done() is called once by every thread of the block at the end
 // (reducing epilogues write their block partial there).
 // outputs: 2 where K and M results are taken apart (yK, yM), else yK is their sum; uses_input: whether put() reads uo.
 #define TT_NO_PRE                                                     \
@@ -279,6 +279,7 @@ struct EpiBC {  // y = A u on free dofs, u on clamped
         for (int c = 0; c < 3; c++) v[c] = ((cl >> c) & 1) ? uo[c] : yK[c];
         st3(y, b, i, v);
     }
+    __device__ void prologue() {}
     __device__ void done(double (&)[2]) const {}
 };
 
@@ -299,6 +300,7 @@ struct EpiBCDot {  // y = A u (BC form) and partials of u.y
         }
         st3(y, b, i, v);
     }
+    __device__ void prologue() {}
     __device__ void done(double (&acc)[2]) const {
         double a[1] = {acc[0]};
         write_partials<1>(a, part);
@@ -323,6 +325,7 @@ struct EpiResid {  // r = b - A x
         for (int c = 0; c < 3; c++) v[c] = p.b[c] - (((cl >> c) & 1) ? uo[c] : yK[c]);
         st3(r, b, i, v);
     }
+    __device__ void prologue() {}
     __device__ void done(double (&)[2]) const {}
 };
 
@@ -347,6 +350,7 @@ struct EpiResidFirst {
         st3(x, b, i, uo);
         st3(r, b, i, v);
     }
+    __device__ void prologue() {}
     __device__ void done(double (&)[2]) const {}
 };
 
@@ -374,6 +378,7 @@ struct EpiResidDots {
         }
         st3(r, b, i, v);
     }
+    __device__ void prologue() {}
     __device__ void done(double (&acc)[2]) const {
         __shared__ double sh[16 * 2];
         block_sum<2>(acc, sh);
@@ -417,6 +422,7 @@ struct EpiCheb {  // r = b - A x; dn = c0 d + c1 dinv r; xn = x + dn
         st3(xn, b, i, v);
         if (dn) st3(dn, b, i, dd);
     }
+    __device__ void prologue() {}
     __device__ void done(double (&)[2]) const {}
 };
 
@@ -455,11 +461,12 @@ struct EpiChebFirst {
         st3(xn, b, i, v);
         st3(dn, b, i, dd);
     }
+    __device__ void prologue() {}
     __device__ void done(double (&)[2]) const {}
 };
 
 // Last post-smoothing step of the finest level: z = x + c0 d + c1 D^-1 (b - A x) written in FP64
-// as the preconditioned residual of flexible CG, with partials of z.r and z.r_prev.
+// as the preconditioned residual of flexible CG, with partials of z.r and z.q_old.
 template <typename T>
 struct EpiChebOut {
     static constexpr int outputs = 1;
@@ -470,12 +477,12 @@ struct EpiChebOut {
     T c0, c1;
     double* z;
     const double* r;
-    const double* rp;
+    const double* q;
     int first;
     double* part;
     struct Pre {
         T b[3], d[3], di[3];
-        double r[3], rp[3];
+        double r[3], q[3];
     };
     template <class S>
     __device__ __forceinline__ void fetch(size_t b, const LaneOff& i, const S&, Pre& p) const {
@@ -483,7 +490,7 @@ struct EpiChebOut {
         ld3(dinv, b, i, p.di);
         if (d) ld3(d, b, i, p.d);
         ld3(r, b, i, p.r);
-        if (!first) ld3(rp, b, i, p.rp);
+        if (!first) ld3(q, b, i, p.q);
     }
     __device__ void put(size_t b, const LaneOff& i, uint8_t cl, const T (&yK)[3], const T (&)[3], const T (&uo)[3],
                         double (&acc)[2], const Pre& p) const {
@@ -495,10 +502,11 @@ struct EpiChebOut {
             if (d) dd = fma(c0, p.d[c], dd);
             zi[c] = (double)(uo[c] + dd);
             acc[0] = fma(zi[c], p.r[c], acc[0]);
-            if (!first) acc[1] = fma(zi[c], p.rp[c], acc[1]);
+            if (!first) acc[1] = fma(zi[c], p.q[c], acc[1]);
         }
         st3(z, b, i, zi);
     }
+    __device__ void prologue() {}
     __device__ void done(double (&acc)[2]) const { write_partials<2>(acc, part); }
 };
 
@@ -520,6 +528,7 @@ struct EpiSplit {  // yk = N.K(N u), ym = N.M(N u)
         st3(yk, b, i, k);
         st3(ym, b, i, m);
     }
+    __device__ void prologue() {}
     __device__ void done(double (&)[2]) const {}
 };
 
@@ -532,6 +541,7 @@ struct EpiRaw {  // y = yK + yM, no BC
                         double (&)[2], const Pre&) const {
         st3(y, b, i, yK);
     }
+    __device__ void prologue() {}
     __device__ void done(double (&)[2]) const {}
 };
 
@@ -555,12 +565,23 @@ struct EpiRHS {  // R = N.(fs F + yK + yM)
         }
         st3(R, b, i, v);
     }
+    __device__ void prologue() {}
     __device__ void done(double (&)[2]) const {}
 };
 
+// beta of the flexible CG (Polak-Ribiere form) from the z.r and z.q_old partials, formed by every block of a consumer
+// (fixed order: bit-identical); block 0 also keeps gamma = z.r for the update.  beta is 0 on a (re)start, and once
+// the solve is frozen, when gamma_old may be 0.  (One block for it alone took 4.4 us per iteration; summing ~500
+// partials in every block hides behind the other blocks' work.)
+__device__ __forceinline__ double fcg_beta(const double* part, int nblk, double* scal, int first) {
+    double d[2];
+    sum_partials<2>(part, nblk, d);
+    if (blockIdx.x == 0 && threadIdx.x == 0) scal[SC_GAMMA] = d[0];
+    return (first || scal[SC_DONE] != 0.0) ? 0.0 : -scal[SC_ALPHA] * d[1] / scal[SC_GAMMA_OLD];
+}
+
 // Flexible-CG direction and its product, with z staged (A z from the contraction): p = z + beta p_old,
-// q = A p = A z + beta q_old (p_old, q_old read at the owned node), partials of p.q.  beta from k_fcg_beta
-// (0 on a (re)start).
+// q = A p = A z + beta q_old (p_old, q_old read at the owned node), partials of p.q.
 struct EpiFcg {
     static constexpr int outputs = 1;
     static constexpr bool uses_input = true;
@@ -568,12 +589,16 @@ struct EpiFcg {
     double* q;
     const double* pold;
     const double* qold;
-    const double* scal;
+    double* scal;
+    const double* dots;
+    int dots_nblk;
     int first;
     double* part;
+    double beta;
     struct Pre {
         double p[3], q[3];
     };
+    __device__ __forceinline__ void prologue() { beta = fcg_beta(dots, dots_nblk, scal, first); }
     template <class S>
     __device__ __forceinline__ void fetch(size_t b, const LaneOff& i, const S&, Pre& pr) const {
         if (!first) {
@@ -584,7 +609,6 @@ struct EpiFcg {
     __device__ void put(size_t b, const LaneOff& i, uint8_t cl, const double (&yK)[3], const double (&)[3],
                         const double (&uo)[3], double (&acc)[2], const Pre& pr) const {
         double p[3], v[3];
-        const double beta = first ? 0.0 : scal[SC_BETA];  // (uniform)
 #pragma unroll
         for (int c = 0; c < 3; c++) {
             const double az = ((cl >> c) & 1) ? uo[c] : yK[c];
@@ -725,15 +749,15 @@ void launch_cheb_first_step(const OpLevel& L, double cK, double cM, const double
 }
 
 void launch_cheb_last(const OpLevel& L, double cK, double cM, const void* b, const void* x, const void* d,
-                      const void* dinv, double c0, double c1, double* z, const double* r, const double* rp, bool first,
+                      const void* dinv, double c0, double c1, double* z, const double* r, const double* q, bool first,
                       bool fp64, Reducer& red, hipStream_t s) {
     check_partials(L, red);
     if (fp64) {
-        EpiChebOut<double> e{(const double*)b, (const double*)d, (const double*)dinv, c0, c1, z, r, rp,
+        EpiChebOut<double> e{(const double*)b, (const double*)d, (const double*)dinv, c0, c1, z, r, q,
                              first ? 1 : 0, red.part(PB_DOTS)};
         red.nblk[PB_DOTS] = run_apply<double, true>(L, cK, cM, StageOne<double>{(const double*)x}, e, s);
     } else {
-        EpiChebOut<float> e{(const float*)b, (const float*)d, (const float*)dinv, (float)c0, (float)c1, z, r, rp,
+        EpiChebOut<float> e{(const float*)b, (const float*)d, (const float*)dinv, (float)c0, (float)c1, z, r, q,
                             first ? 1 : 0, red.part(PB_DOTS)};
         red.nblk[PB_DOTS] = run_apply<float, true>(L, cK, cM, StageOne<float>{(const float*)x}, e, s);
     }
@@ -763,17 +787,11 @@ void launch_newmark_rhs(const OpLevel& L, const double* u, const double* v, cons
 // single-block reductions of partials: 1024 threads, so each sums ~5 of the ~5000 partials of a
 // fine-grid launch (latency bound: 256 threads took ~4.6 us per call)
 constexpr int BSR = 1024;
-__global__ __launch_bounds__(BSR) void k_fcg_beta(const double* __restrict__ dots_part, int dots_nblk, double* scal,
-                                                  int first);
 void launch_fcg_apply(const OpLevel& L, double cK, double cM, const double* z, const double* p_old, double* p_new,
-                      const double* q_old, double* q_new, Reducer& red, bool first, hipStream_t s, bool beta) {
+                      const double* q_old, double* q_new, Reducer& red, bool first, hipStream_t s) {
     check_partials(L, red);
-    if (beta) {
-        hipLaunchKernelGGL(k_fcg_beta, dim3(1), dim3(BSR), 0, s, red.part(PB_DOTS), red.nblk[PB_DOTS], red.scal.p,
-                           first ? 1 : 0);
-        TT_HIP(hipGetLastError());
-    }
-    EpiFcg e{p_new, q_new, p_old, q_old, red.scal.p, first ? 1 : 0, red.part(PB_PQ)};
+    EpiFcg e{p_new, q_new,        p_old, q_old, red.scal.p, red.part(PB_DOTS), red.nblk[PB_DOTS], first ? 1 : 0,
+             red.part(PB_PQ), 0.0};
     red.nblk[PB_PQ] = run_apply<double, true>(L, cK, cM, StageOne<double>{z}, e, s);
     red.nv[PB_PQ] = 1;
 }
@@ -1398,30 +1416,20 @@ int launch_proj3(const double* Q, int k0, int nq, const double* a, const double*
     return nb;
 }
 
-// gamma = z.r, delta = z.r_prev (flexible CG, Polak-Ribiere form)
-__global__ void k_fcg_dots(const double* __restrict__ z, const double* __restrict__ r, const double* __restrict__ rp,
+// partials of z.r and z.q_old (flexible CG, Polak-Ribiere form; see fcg_beta)
+__global__ void k_fcg_dots(const double* __restrict__ z, const double* __restrict__ r, const double* __restrict__ q,
                            long n, double* part, int first) {
     double acc[2] = {0.0, 0.0};
     for (long i = blockIdx.x * (long)blockDim.x + threadIdx.x; i < n; i += (long)gridDim.x * blockDim.x) {
         acc[0] = fma(z[i], r[i], acc[0]);
-        if (!first) acc[1] = fma(z[i], rp[i], acc[1]);
+        if (!first) acc[1] = fma(z[i], q[i], acc[1]);
     }
     write_partials<2>(acc, part);
 }
-// gamma = z.r and beta = (z.r - z.r_prev) / gamma_old (0 on a (re)start, and once the solve is
-// frozen, when gamma_old may be 0) from the partials of k_fcg_dots
-__global__ __launch_bounds__(BSR) void k_fcg_beta(const double* __restrict__ dots_part, int dots_nblk, double* scal, int first) {
-    double d[2];
-    sum_partials<2>(dots_part, dots_nblk, d);
-    if (threadIdx.x == 0) {
-        scal[SC_GAMMA] = d[0];
-        scal[SC_BETA] = (first || scal[SC_DONE] != 0.0) ? 0.0 : (d[0] - d[1]) / scal[SC_GAMMA_OLD];
-    }
-}
-void launch_fcg_dots(const double* z, const double* r, const double* rprev, long n, Reducer& red, bool first,
+void launch_fcg_dots(const double* z, const double* r, const double* q_old, long n, Reducer& red, bool first,
                      hipStream_t s) {
     const int nb = rb_blocks(n);
-    hipLaunchKernelGGL(k_fcg_dots, dim3(nb), dim3(BS), 0, s, z, r, rprev, n, red.part(PB_DOTS), (int)first);
+    hipLaunchKernelGGL(k_fcg_dots, dim3(nb), dim3(BS), 0, s, z, r, q_old, n, red.part(PB_DOTS), (int)first);
     red.nblk[PB_DOTS] = nb;
     red.nv[PB_DOTS] = 2;
     TT_HIP(hipGetLastError());
@@ -1456,77 +1464,83 @@ void launch_fcg_init(Reducer& red, int bb_region, int rr_region, double rtol2, b
     red.nv[bb_region] = 1;
 }
 
-// alpha = gamma / (p.q) from the partials of the FCG apply (one block); gamma becomes gamma_old.
-// After the first iteration of a (re)start, the previous update's r.r (its partials) is checked
-// too: once it is <= (rtol ||b||)^2, SC_DONE stays set and alpha is 0 for the rest of the solve,
-// so x is frozen at the first iteration that met the tolerance.
-__global__ __launch_bounds__(BSR) void k_fcg_alpha(const double* __restrict__ pq_part, int pq_nblk, const double* __restrict__ rr_part,
-                            int rr_nblk, double* scal, int first) {
+// x += alpha p (x = 0 if b = 0); r -= alpha q; partials of r.r.  Every block forms alpha = gamma / (p.q) itself from the
+// p.q partials, and checks the previous update's r.r (not on the first iteration of a (re)start): once that is
+// <= (rtol ||b||)^2, SC_DONE is set and alpha is 0 for the rest of the solve, so x is frozen at the first iteration that
+// met the tolerance; a frozen solve keeps x and r as they are.  Block 0 writes the scalars: what other blocks read of
+// them gives the same decision before and after that write (SC_DONE is only ever set to what they find themselves).
+// HBM bound: 6 vectors, 14 us at 128x64x64 (with r_prev written as a 7th vector, which z.q_old makes unnecessary, and
+// a one-block kernel for alpha before it: 17 + 4.7 us).
+__global__ __launch_bounds__(BS) void k_fcg_update(double* __restrict__ x, const double* __restrict__ p,
+                                                   double* __restrict__ r, const double* __restrict__ q, long n,
+                                                   const double* __restrict__ pq_part, int pq_nblk,
+                                                   const double* __restrict__ rr_old, int rr_nblk, double* scal,
+                                                   double* part, double* look, int first) {
+    const long i0 = blockIdx.x * (long)blockDim.x + threadIdx.x, st = (long)gridDim.x * blockDim.x;
+    // the first values are in flight while the partials are summed
+    double x0 = 0.0, p0 = 0.0, r0 = 0.0, q0 = 0.0;
+    if (i0 < n) {
+        x0 = x[i0];
+        p0 = p[i0];
+        r0 = r[i0];
+        q0 = q[i0];
+    }
     double pq[1], rr[1] = {0.0};
     sum_partials<1>(pq_part, pq_nblk, pq);
-    if (!first) sum_partials<1>(rr_part, rr_nblk, rr);
-    if (threadIdx.x == 0) {
-        const bool done = scal[SC_DONE] != 0.0 || (!first && rr[0] <= scal[SC_TOL2]);
-        const double gam = scal[SC_GAMMA];
-        scal[SC_DONE] = done ? 1.0 : 0.0;
-        scal[SC_ALPHA] = done ? 0.0 : gam / pq[0];
-        scal[SC_GAMMA_OLD] = gam;
-        if (!done) scal[SC_ITERS] += 1.0;
-    }
-}
-
-// x += alpha p (x = 0 if b = 0); r_prev = r; r -= alpha q; partials of r.r.  A frozen solve keeps
-// x and r as they are.
-__global__ void k_fcg_update(double* __restrict__ x, const double* __restrict__ p, double* __restrict__ r,
-                             double* __restrict__ rp, const double* __restrict__ q, long n,
-                             const double* __restrict__ scal, double* part, double* look) {
-    const double al = scal[SC_ALPHA];
-    const bool zero = scal[SC_ZERO] != 0.0, done = scal[SC_DONE] != 0.0;
+    if (!first) sum_partials<1>(rr_old, rr_nblk, rr);
+    const bool zero = scal[SC_ZERO] != 0.0, done = scal[SC_DONE] != 0.0 || (!first && rr[0] <= scal[SC_TOL2]);
+    const double gam = scal[SC_GAMMA], al = done ? 0.0 : gam / pq[0];
     double acc[1] = {0.0};
-    for (long i = blockIdx.x * (long)blockDim.x + threadIdx.x; i < n; i += (long)gridDim.x * blockDim.x) {
+    for (long i = i0; i < n; i += st) {
+        if (i != i0) {
+            x0 = x[i];
+            p0 = p[i];
+            r0 = r[i];
+            q0 = q[i];
+        }
         if (zero) x[i] = 0.0;
-        else if (!done) x[i] = fma(al, p[i], x[i]);
-        const double ri = r[i];
-        rp[i] = ri;
-        const double rn = done ? ri : fma(-al, q[i], ri);
-        r[i] = rn;
+        else if (!done) x[i] = fma(al, p0, x0);
+        const double rn = done ? r0 : fma(-al, q0, r0);
+        if (!done) r[i] = rn;
         acc[0] = fma(rn, rn, acc[0]);
     }
     __shared__ double sh[16];
     block_sum<1>(acc, sh);
-    if (threadIdx.x == 0) {  // the partial for k_fcg_alpha, and its copy for the host's look
+    if (threadIdx.x == 0) {  // the partial for the next update, and its copy for the host's look
         part[blockIdx.x] = acc[0];
         look[blockIdx.x] = acc[0];
-        if (blockIdx.x == 0) look[gridDim.x] = scal[SC_ITERS];
+        if (blockIdx.x == 0) {
+            const double it = scal[SC_ITERS] + (done ? 0.0 : 1.0);
+            scal[SC_DONE] = done ? 1.0 : 0.0;
+            scal[SC_ALPHA] = al;
+            scal[SC_GAMMA_OLD] = gam;
+            scal[SC_ITERS] = it;
+            look[gridDim.x] = it;
+        }
     }
 }
-void launch_fcg_update(double* x, const double* p, double* r, double* rprev, const double* q, long n, Reducer& red,
-                       bool first, hipStream_t s) {
-    hipLaunchKernelGGL(k_fcg_alpha, dim3(1), dim3(BSR), 0, s, red.part(PB_PQ), red.nblk[PB_PQ], red.part(PB_RR),
-                       red.nblk[PB_RR], red.scal.p, first ? 1 : 0);
-    TT_HIP(hipGetLastError());
-    const int nb = rb_blocks(n);
+void launch_fcg_update(double* x, const double* p, double* r, const double* q, long n, Reducer& red, bool first,
+                       bool odd, hipStream_t s) {
+    const int nb = rb_blocks(n), now = rr_region(odd), old = rr_region(!odd);
     TT_CHECK(nb < Reducer::kLookBB, -3, "look buffer too small");
-    hipLaunchKernelGGL(k_fcg_update, dim3(nb), dim3(BS), 0, s, x, p, r, rprev, q, n, red.scal.p, red.part(PB_RR),
-                       red.look_dev);
-    red.nblk[PB_RR] = nb;
-    red.nv[PB_RR] = 1;
+    hipLaunchKernelGGL(k_fcg_update, dim3(nb), dim3(BS), 0, s, x, p, r, q, n, red.part(PB_PQ), red.nblk[PB_PQ],
+                       red.part(old), red.nblk[old], red.scal.p, red.part(now), red.look_dev, first ? 1 : 0);
+    red.nblk[now] = nb;
+    red.nv[now] = 1;
     TT_HIP(hipGetLastError());
 }
 
 __global__ void k_fcg_direction(const double* __restrict__ z, const double* __restrict__ pold,
-                                double* __restrict__ pnew, long n, const double* __restrict__ scal, int first) {
-    const double beta = first ? 0.0 : scal[SC_BETA];
+                                double* __restrict__ pnew, long n, const double* __restrict__ dots, int dots_nblk,
+                                double* scal, int first) {
+    const double beta = fcg_beta(dots, dots_nblk, scal, first);
     for (long i = blockIdx.x * (long)blockDim.x + threadIdx.x; i < n; i += (long)gridDim.x * blockDim.x)
         pnew[i] = first ? z[i] : fma(beta, pold[i], z[i]);
 }
 void launch_fcg_direction(const double* z, const double* p_old, double* p_new, long n, Reducer& red, bool first,
                           hipStream_t s) {
-    hipLaunchKernelGGL(k_fcg_beta, dim3(1), dim3(BSR), 0, s, red.part(PB_DOTS), red.nblk[PB_DOTS], red.scal.p,
-                       first ? 1 : 0);
-    TT_HIP(hipGetLastError());
-    hipLaunchKernelGGL(k_fcg_direction, dim3(nblocks(n)), dim3(BS), 0, s, z, p_old, p_new, n, red.scal.p,
-                       first ? 1 : 0);
+    hipLaunchKernelGGL(k_fcg_direction, dim3(rb_blocks(n)), dim3(BS), 0, s, z, p_old, p_new, n, red.part(PB_DOTS),
+                       red.nblk[PB_DOTS], red.scal.p, first ? 1 : 0);
     TT_HIP(hipGetLastError());
 }
 

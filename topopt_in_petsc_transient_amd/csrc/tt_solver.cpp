@@ -357,7 +357,7 @@ void Multigrid::coarse_solve(bool direct64) {
     if (!lc.fp64) launch_copy(x64, lc.x.p, nc, true, false, s);
 }
 
-void Multigrid::vcycle(int l, const double* r64, double* z64, const double* rp64, bool first) {
+void Multigrid::vcycle(int l, const double* r64, double* z64, const double* q64, bool first) {
     const int nl = (int)L.size();
     if (l == nl - 1) {
         coarse_solve(l > 0 && dense && !L[l]->fp64);  // as decided by the level above (direct64)
@@ -426,7 +426,7 @@ void Multigrid::vcycle(int l, const double* r64, double* z64, const double* rp64
         }
         if (z64 && k == npost - 1) {  // last step: z = x_new in FP64 plus the flexible-CG dots
             launch_cheb_last(lv.op, cK, cM, lv.b.p, lv.x.p, k > 0 ? lv.d.p : nullptr, lv.dinv.p, c0, c1, z64, r64,
-                             rp64, first, f64, ctx->red, s);
+                             q64, first, f64, ctx->red, s);
             break;
         }
         launch_cheb_step(lv.op, cK, cM, lv.b.p, lv.x.p, k > 0 ? lv.d.p : nullptr, lv.dinv.p, c0, c1, lv.x2.p,
@@ -436,14 +436,14 @@ void Multigrid::vcycle(int l, const double* r64, double* z64, const double* rp64
     }
 }
 
-void Multigrid::apply_fcg(const double* r, const double* rp, double* z, bool first) {
+void Multigrid::apply_fcg(const double* r, const double* q_old, double* z, bool first) {
     finish_inverse();
     if (L.size() == 1) {
         apply(r, z);
-        launch_fcg_dots(z, r, rp, L[0]->g.nd, ctx->red, first, ctx->stream);
+        launch_fcg_dots(z, r, q_old, L[0]->g.nd, ctx->red, first, ctx->stream);
         return;
     }
-    vcycle(0, r, z, rp, first);
+    vcycle(0, r, z, q_old, first);
 }
 
 void Multigrid::apply(const double* r, double* z) {
@@ -502,7 +502,7 @@ SolveResult Context::fcg(double cK, double cM, bool use_mg, SolveKind kind, cons
     // from one iteration before the fewest any of the last kHintLen solves of this kind took.  A look
     // that comes too late costs idle iterations instead (~0.4 ms each at 128x64x64), never a
     // different answer: the device freezes x at the first iteration whose recursive residual meets
-    // the tolerance (k_fcg_alpha).  Measured on the 128x64x64 forward sweep (2-3 iterations per
+    // the tolerance (k_fcg_update).  Measured on the 128x64x64 forward sweep (2-3 iterations per
     // solve, a few solves converging after one): looking first at the fewest instead of one before
     // it ran 3 % slower.
     int* hist = fcg_hist[kind];
@@ -528,13 +528,13 @@ SolveResult Context::fcg(double cK, double cM, bool use_mg, SolveKind kind, cons
     if (graphed) launch_copy(x, xs, nd, true, true, stream);
     auto iteration = [&]() {
         if (use_mg) {
-            mg.apply_fcg(kr.p, krp.p, kz.p, first);  // z = B r with the dots z.r, z.r_prev
+            mg.apply_fcg(kr.p, qold, kz.p, first);  // z = B r with the dots z.r, z.q_old
         } else {
             launch_jacobi(dinvM.p, kr.p, kz.p, nd, stream);
-            launch_fcg_dots(kz.p, kr.p, krp.p, nd, red, first, stream);
+            launch_fcg_dots(kz.p, kr.p, qold, nd, red, first, stream);
         }
         launch_fcg_apply(op, cK, cM, kz.p, pold, pnew, qold, qnew, red, first, stream);
-        launch_fcg_update(xs, pnew, kr.p, krp.p, qnew, nd, red, first, stream);
+        launch_fcg_update(xs, pnew, kr.p, qnew, nd, red, first, pnew == kp0.p, stream);
     };
     int it = 0;
     while (!conv && it < prm.maxit) {
@@ -589,7 +589,7 @@ SolveResult Context::fcg(double cK, double cM, bool use_mg, SolveKind kind, cons
         wait_look();
         {
             const volatile double* lk = red.look;
-            const int nb = red.nblk[PB_RR];
+            const int nb = red.nblk[rr_region(pold == kp0.p)];  // (p_new of the iteration just queued)
             for (int i = 0; i < nb; i++) rr += lk[i];
             moved = (int)lk[nb];
             bb = lk[Reducer::kLookBB];
