@@ -181,6 +181,7 @@ struct Context {
     void expand_state(int t, double* out);    // u, v, a of reduced state t on the full mesh
     void project3(const double* h0, const double* h1, const double* h2, double* out);  // out[3k+i] = Q_k.h_i
     DBuf<double> gmV, gmZ;  // flexible-GMRES Krylov and preconditioned vectors of the basis solves
+    DBuf<double> gmG, gmH, gmPart;  // Gram-Schmidt: dots within groups, coefficients, partials (launch_mgs)
     SolveResult fgmres(double cK, double cM, const double* b, double* x);
     void reduced_adjoint(const std::function<void(const double*)>& grad_state,
                          const std::function<void(int, const double*, const double*, const double*, int)>& sens);

@@ -313,6 +313,12 @@ void launch_dot(const double* a, const double* b, long n, Reducer& red, int slot
 // block partials into part[(k*1024 + block)*3 + i]; returns the number of blocks (at most 1024)
 int launch_proj3(const double* Q, int k0, int nq, const double* a, const double* b, const double* c, long n,
                  double* part, hipStream_t s);
+// Modified Gram-Schmidt of w against the k orthonormal vectors V_i = V + i*n, then w /= ||w||, on the device: h[0..k-1]
+// receive the coefficients and h[k] = ||w|| (w stays as it is if that is 0).  Groups of kMgsGroup vectors share a
+// pass over w; G (kMgsMax x kMgsMax, device, kept between calls while V grows) holds the dots of vectors of one
+// group, from which the group's coefficients follow one after the other.  part: 2 x kMgsBlocks x (kMgsGroup + 1).
+constexpr int kMgsGroup = 8, kMgsBlocks = 256, kMgsMax = 32;
+void launch_mgs(double* w, const double* V, int k, long n, double* G, double* h, double* part, hipStream_t s);
 // out[o] = sum_k c[o][k] Q_k for nout <= 3 outputs and nb <= 64 vectors Q_k = Q + k*n, one pass over Q
 struct Expand3 {
     const double* Q;
@@ -321,6 +327,8 @@ struct Expand3 {
     int nb, nout;
 };
 void launch_expand3(const Expand3& e, long n, hipStream_t s);
+// out[0] += sum_k c[0][k] Q_k
+void launch_axpy_multi(const Expand3& e, long n, hipStream_t s);
 // partials of z.r and z.q_old (PB_DOTS)
 void launch_fcg_dots(const double* z, const double* r, const double* q_old, long n, Reducer& red, bool first,
                      hipStream_t s);

@@ -1379,6 +1379,113 @@ void launch_expand3(const Expand3& e, long n, hipStream_t s) {
     TT_HIP(hipGetLastError());
 }
 
+__global__ void k_axpy_multi(Expand3 e, long n) {
+    const long i = blockIdx.x * (long)blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    double s0 = e.out[0][i];
+#pragma unroll 4
+    for (int k = 0; k < e.nb; k++) s0 = fma(e.c[0][k], e.Q[(size_t)k * n + i], s0);
+    e.out[0][i] = s0;
+}
+void launch_axpy_multi(const Expand3& e, long n, hipStream_t s) {
+    TT_CHECK(e.nb >= 1 && e.nb <= 64, -3, "launch_axpy_multi: 1..64 vectors");
+    hipLaunchKernelGGL(k_axpy_multi, dim3(nblocks(n)), dim3(BS), 0, s, e, n);
+    TT_HIP(hipGetLastError());
+}
+
+// Modified Gram-Schmidt in passes over groups of vectors.  One pass subtracts the current group (its coefficients from
+// the dots that the previous pass left) and forms the dots of the new w with the next group, or, after the last, with
+// its own group and itself.  With D_i = w.v_i at the group's start, the coefficients one after the other are
+// h_i = D_i - sum_{j < i} h_j (v_j.v_i): exactly those of subtracting v_0, v_1, ... in turn, with the stored dots
+// of the group's vectors.  HBM bound: (2 + group + next group) vectors a pass, against a dot product, a host round trip
+// and an update (5 vectors and ~28 us) per vector before: an Arnoldi step of 16 vectors at 128x64x64 takes 90
+// instead of 450 us.
+constexpr int MG = kMgsGroup, MB = kMgsBlocks, MT = 512;
+static_assert(MT / 64 == MG, "one wave sums one entry");
+// entry q of the MB partial rows, summed by wave q (fixed order), into d[q]; entry MG by wave 0
+__device__ __forceinline__ void mgs_sums(const double* __restrict__ part, double* d) {
+    const int q = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    for (int e = q; e <= MG; e += MG) {
+        double x = 0.0;
+#pragma unroll
+        for (int b = 0; b < MB / 64; b++) x += part[(size_t)(lane + 64 * b) * (MG + 1) + e];
+#pragma unroll
+        for (int off = 32; off > 0; off >>= 1) x += __shfl_xor(x, off, 64);
+        if (lane == 0) d[e] = x;
+    }
+    __syncthreads();
+}
+__global__ __launch_bounds__(MT) void k_mgs(double* __restrict__ w, const double* __restrict__ V, long n, int i0, int na,
+                                            int nnext, const double* __restrict__ part_in,
+                                            double* __restrict__ part_out, const double* __restrict__ G,
+                                            double* __restrict__ h) {
+    __shared__ double d[MG + 1], hs[MG], sh[16 * (MG + 1)];
+    if (threadIdx.x < MG) hs[threadIdx.x] = 0.0;
+    if (na > 0) {
+        mgs_sums(part_in, d);
+        if (threadIdx.x == 0)
+            for (int i = 0; i < na; i++) {
+                double x = d[i];
+                for (int j = 0; j < i; j++) x = fma(-hs[j], G[(i0 + j) * kMgsMax + i0 + i], x);
+                hs[i] = x;
+                if (blockIdx.x == 0) h[i0 + i] = x;
+            }
+    }
+    __syncthreads();
+    const double* Va = V + (size_t)i0 * n;
+    const double* Vb = Va + (size_t)na * n;
+    double hq[MG], acc[MG + 1];
+#pragma unroll
+    for (int q = 0; q < MG; q++) hq[q] = hs[q];
+#pragma unroll
+    for (int q = 0; q <= MG; q++) acc[q] = 0.0;
+    for (long i = blockIdx.x * (long)MT + threadIdx.x; i < n; i += (long)MB * MT) {
+        double va[MG], vb[MG];
+        double wi = w[i];
+#pragma unroll
+        for (int q = 0; q < MG; q++) va[q] = q < na ? Va[(size_t)q * n + i] : 0.0;
+#pragma unroll
+        for (int q = 0; q < MG; q++) vb[q] = q < nnext ? Vb[(size_t)q * n + i] : 0.0;
+#pragma unroll
+        for (int q = 0; q < MG; q++)
+            if (q < na) wi = fma(-hq[q], va[q], wi);
+        if (na > 0) w[i] = wi;
+#pragma unroll
+        for (int q = 0; q < MG; q++) acc[q] = fma(wi, nnext > 0 ? vb[q] : va[q], acc[q]);
+        acc[MG] = fma(wi, wi, acc[MG]);
+    }
+    block_sum<MG + 1>(acc, sh);
+    if (threadIdx.x == 0)
+#pragma unroll
+        for (int q = 0; q <= MG; q++) part_out[(size_t)blockIdx.x * (MG + 1) + q] = acc[q];
+}
+// w /= ||w||, h[k] = ||w||, and the dots of the new vector k with the earlier ones of its group (the last pass's)
+__global__ __launch_bounds__(MT) void k_mgs_scale(double* __restrict__ w, long n, int k, const double* __restrict__ part,
+                                                  double* __restrict__ G, double* __restrict__ h) {
+    __shared__ double d[MG + 1];
+    mgs_sums(part, d);
+    const double nrm = sqrt(d[MG]), inv = nrm > 0.0 ? 1.0 / nrm : 1.0;
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        h[k] = nrm;
+        const int g0 = k / MG * MG;
+        for (int i = g0; i < k; i++) G[i * kMgsMax + k] = d[i - g0] * inv;
+    }
+    for (long i = blockIdx.x * (long)MT + threadIdx.x; i < n; i += (long)MB * MT) w[i] *= inv;
+}
+void launch_mgs(double* w, const double* V, int k, long n, double* G, double* h, double* part, hipStream_t s) {
+    TT_CHECK(k >= 1 && k < kMgsMax, -3, "launch_mgs: 1..31 vectors");
+    double* pb[2] = {part, part + (size_t)MB * (MG + 1)};
+    int cur = 0;
+    hipLaunchKernelGGL(k_mgs, dim3(MB), dim3(MT), 0, s, w, V, n, 0, 0, std::min(MG, k), pb[1], pb[0], G, h);
+    for (int i0 = 0; i0 < k; i0 += MG) {
+        const int na = std::min(MG, k - i0), nn = std::min(MG, std::max(0, k - i0 - na));
+        hipLaunchKernelGGL(k_mgs, dim3(MB), dim3(MT), 0, s, w, V, n, i0, na, nn, pb[cur], pb[cur ^ 1], G, h);
+        cur ^= 1;
+    }
+    hipLaunchKernelGGL(k_mgs_scale, dim3(MB), dim3(MT), 0, s, w, n, k, pb[cur], G, h);
+    TT_HIP(hipGetLastError());
+}
+
 template <int NQ>
 __global__ void k_proj3(const double* __restrict__ Q, int k0, const double* __restrict__ a,
                         const double* __restrict__ b, const double* __restrict__ c, long n, double* part) {

@@ -114,12 +114,16 @@ void Context::project3(const double* h0, const double* h1, const double* h2, dou
 // (modified Gram-Schmidt Arnoldi, Givens rotations; the true residual is formed at every restart and
 // decides convergence: ||b - A x|| <= rtol ||b||).
 static constexpr int kRestart = 30;
+static_assert(kRestart < kMgsMax, "Gram-Schmidt work arrays");
 SolveResult Context::fgmres(double cK, double cM, const double* b, double* x) {
     const long nd = g.nd;
     const int m = kRestart;
     if (!gmV.p) {
         gmV.alloc((size_t)(m + 1) * nd);
         gmZ.alloc((size_t)m * nd);
+        gmG.alloc(kMgsMax * kMgsMax);
+        gmH.alloc(kMgsMax);
+        gmPart.alloc(2 * (size_t)kMgsBlocks * (kMgsGroup + 1));
     }
     auto V = [&](int i) { return gmV.p + (size_t)i * nd; };
     auto Z = [&](int i) { return gmZ.p + (size_t)i * nd; };
@@ -151,14 +155,13 @@ SolveResult Context::fgmres(double cK, double cM, const double* b, double* x) {
         for (; k < m && it < prm.maxit; k++) {
             mg.apply(V(k), Z(k));
             launch_apply_bc(op_fine64, cK, cM, Z(k), V(k + 1), true, stream);
-            for (int i = 0; i <= k; i++) {
-                const double h = dot(V(k + 1), V(i));
-                H[(size_t)i * m + k] = h;
-                launch_lincomb(1.0, V(k + 1), -h, V(i), V(k + 1), nd, stream);
-            }
-            const double hn = std::sqrt(dot(V(k + 1), V(k + 1)));
+            // column k of H (k + 1 coefficients and the norm): device work, one read-back
+            launch_mgs(V(k + 1), V(0), k + 1, nd, gmG.p, gmH.p, gmPart.p, stream);
+            TT_HIP(hipMemcpyAsync(projhost, gmH.p, sizeof(double) * (k + 2), hipMemcpyDeviceToHost, stream));
+            sync();
+            for (int i = 0; i <= k; i++) H[(size_t)i * m + k] = projhost[i];
+            const double hn = projhost[k + 1];
             H[(size_t)(k + 1) * m + k] = hn;
-            if (hn > 0.0) launch_scale(V(k + 1), nd, 1.0 / hn, stream);
             for (int i = 0; i < k; i++) {  // earlier rotations on the new column
                 const double a0 = H[(size_t)i * m + k], a1 = H[(size_t)(i + 1) * m + k];
                 H[(size_t)i * m + k] = cs[i] * a0 + sn[i] * a1;
@@ -184,7 +187,15 @@ SolveResult Context::fgmres(double cK, double cM, const double* b, double* x) {
             for (int j = i + 1; j < k; j++) s -= H[(size_t)i * m + j] * y[j];
             y[i] = s / H[(size_t)i * m + i];
         }
-        for (int i = 0; i < k; i++) launch_lincomb(1.0, x, y[i], Z(i), x, nd, stream);
+        if (k > 0) {
+            Expand3 e{};
+            e.Q = gmZ.p;
+            e.nb = k;
+            e.nout = 1;
+            e.out[0] = x;
+            for (int i = 0; i < k; i++) e.c[0][i] = y[i];
+            launch_axpy_multi(e, nd, stream);
+        }
     }
     stats.krylov_iters += it;
     stats.last_iters = it;
