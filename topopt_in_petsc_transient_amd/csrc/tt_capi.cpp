@@ -178,7 +178,7 @@ Context::Context(const tt_params& p) : prm(p) {
     // PDE filter (PDEFilter.cc:28-191) on the same node grid
     fg = g;
     KFd.alloc(64);
-    for (DBuf<double>* b : {&fdinv, &fU, &frhs, &fr, &fz, &fp, &fp2, &fq}) b->alloc(nn);
+    for (DBuf<double>* b : {&fdinv, &fU, &frhs, &fr, &fp, &fp2, &fq}) b->alloc(nn);
     set_filter_radius(p.rmin);
 }
 
@@ -186,6 +186,7 @@ Context::Context(const tt_params& p) : prm(p) {
 void Context::set_filter_radius(double rmin) {
     prm.rmin = rmin;
     const double R = rmin / 2.0 / std::sqrt(3.0);
+    filter_R = R;
     hex8_helmholtz(g.hx, g.hy, g.hz, R, KF);
     TT_HIP(hipMemcpyAsync(KFd.p, KF, sizeof(KF), hipMemcpyHostToDevice, stream));
     launch_filter_diag(fg, KFd.p, fdinv.p, stream);
@@ -217,14 +218,9 @@ void Context::pde_filter(const double* in, double* out) {
     // residual meets it, so late looks cost idle iterations, never a different answer).  The host reads
     // the residual from one iteration before the last solve's count, then every 4 iterations, and
     // confirms the true residual once the recursive one has converged.
-    auto start = [&](bool reset) {
-        launch_filter_apply(fg, KFd.p, fU.p, fq.p, nullptr, 0, stream);
-        launch_lincomb(1.0, frhs.p, -1.0, fq.p, fr.p, nn, stream);
-        if (reset) launch_dot(frhs.p, frhs.p, nn, red, PB_MISC, stream);
-        launch_dot(fr.p, fr.p, nn, red, PB_MISC2, stream);
-        launch_fcg_init(red, PB_MISC, PB_MISC2, tol * tol, reset, stream);
-    };
-    start(true);
+    const FilterOp op{{fg.hx, fg.hy, fg.hz}, filter_R * filter_R};
+    launch_filter_residual(fg, op, fU.p, frhs.p, fdinv.p, fr.p, red, true, stream);
+    launch_fcg_init(red, PB_MISC, PB_MISC2, tol * tol, true, stream);
     const int maxit = 20000;
     int it = 0, next_look = std::max(filter_iters - 1, 1);
     bool first = true;
@@ -233,11 +229,8 @@ void Context::pde_filter(const double* in, double* out) {
     double rel = 0.0;
     for (;;) {
         while (it < next_look) {
-            launch_jacobi(fdinv.p, fr.p, fz.p, nn, stream);
-            launch_fcg_dots(fz.p, fr.p, fq.p, nn, red, first, stream);
-            launch_fcg_direction(fz.p, pold, pnew, nn, red, first, stream);
-            launch_filter_apply(fg, KFd.p, pnew, fq.p, &red, PB_PQ, stream);
-            launch_fcg_update(fU.p, pnew, fr.p, fq.p, nn, red, first, pnew == fp.p, stream);
+            launch_filter_direction(fg, op, fr.p, fdinv.p, pold, pnew, fq.p, red, first, stream);
+            launch_fcg_update(fU.p, pnew, fr.p, fq.p, nn, red, first, pnew == fp.p, stream, fdinv.p);
             std::swap(pold, pnew);
             first = false;
             it++;
@@ -255,12 +248,10 @@ void Context::pde_filter(const double* in, double* out) {
         }
         if (rr <= tol * tol * bb * (1.0 + 1e-10)) {
             // confirm with the true residual; restart the recursion if it drifted
-            launch_filter_apply(fg, KFd.p, fU.p, fq.p, nullptr, 0, stream);
-            launch_lincomb(1.0, frhs.p, -1.0, fq.p, fr.p, nn, stream);
-            launch_dot(fr.p, fr.p, nn, red, PB_MISC2, stream);
+            launch_filter_residual(fg, op, fU.p, frhs.p, fdinv.p, fr.p, red, false, stream);
             rel = std::sqrt(reduce1(PB_MISC2) / bb);
             if (rel <= tol) break;
-            start(false);
+            launch_fcg_init(red, PB_MISC, PB_MISC2, tol * tol, false, stream);
             first = true;
         }
         if (it >= maxit) throw Error{TT_ERR_NOT_CONVERGED, "PDE filter solve did not converge"};

@@ -161,8 +161,8 @@ struct Context {
         mu, nu, mun, nun, hdu, hddu, hdddu, Kl, Ml, rhs, df, fxs, nu0;
 
     // PDE filter
-    double KF[64];
-    DBuf<double> KFd, fdinv, fU, frhs, fr, fz, fp, fp2, fq, ftmp_e, ftmp_e2;
+    double KF[64], filter_R = 0.0;
+    DBuf<double> KFd, fdinv, fU, frhs, fr, fp, fp2, fq, ftmp_e, ftmp_e2;
     int filter_iters = 0;  // iterations of the last filter solve (when the host first reads the residual)
     Grid fg{};
 

@@ -342,13 +342,11 @@ void launch_fcg_init(Reducer& red, int bb_region, int rr_region, double rtol2, b
 // itself from the p.q partials and the previous update's r.r; odd: the parity of the iteration (its r.r partials go to
 // region rr_region(odd), the previous update's are in the other one).
 inline int rr_region(bool odd) { return odd ? PB_RR2 : PB_RR; }
+// With dinv, the partials of z.r and z.q for the next direction (z = D^-1 r of the new r) go to PB_DOTS: the Jacobi
+// preconditioner needs no kernel of its own.
 void launch_fcg_update(double* x, const double* p, double* r, const double* q, long n, Reducer& red, bool first,
-                       bool odd, hipStream_t s);
+                       bool odd, hipStream_t s, const double* dinv = nullptr);
 void launch_jacobi(const double* dinv, const double* r, double* z, long n, hipStream_t s);
-// Flexible-CG direction for a matrix without a fused apply kernel: beta from the partials of launch_fcg_dots (0 on a
-// (re)start), then p_new = z + beta p_old.
-void launch_fcg_direction(const double* z, const double* p_old, double* p_new, long n, Reducer& red, bool first,
-                          hipStream_t s);
 // power iteration: x = dinv.Ax with partials of ||x||^2 in PB_MISC; then x /= ||x||
 void launch_norm_power(const void* Ax, const void* dinv, void* x, long n, Reducer& red, bool fp64, hipStream_t s);
 void launch_scale_by_norm(void* x, long n, Reducer& red, bool fp64, hipStream_t s);
@@ -391,8 +389,16 @@ struct SensArgs {
 void launch_sens(const SensArgs& a, Reducer& red, double* fx_out, hipStream_t s);
 
 // PDE filter (scalar Helmholtz on nodes)
-void launch_filter_apply(const Grid& g, const double* kf, const double* u, double* y, Reducer* red, int dot_slot,
-                         hipStream_t s);
+// The filter's operator R^2 (Kx My Mz + Mx Ky Mz + Mx My Kz) + Mx My Mz by its 1-D factors.
+struct FilterOp {
+    double h[3], R2;
+};
+// r = rhs - A U, partials of r.r (PB_MISC2), of z.r with z = D^-1 r (PB_DOTS) and, with bb, of rhs.rhs (PB_MISC)
+void launch_filter_residual(const Grid& g, const FilterOp& f, const double* U, const double* rhs, const double* dinv,
+                            double* r, Reducer& red, bool bb, hipStream_t s);
+// Jacobi-preconditioned CG direction and product: p = z + beta p_old with z = D^-1 r, q = A p, partials of p.q
+void launch_filter_direction(const Grid& g, const FilterOp& f, const double* r, const double* dinv, const double* p_old,
+                             double* p_new, double* q, Reducer& red, bool first, hipStream_t s);
 void launch_filter_T(const Grid& g, const double* x, double scale, double* rhs, hipStream_t s);
 void launch_filter_Tt(const Grid& g, const double* U, double* out, hipStream_t s);
 void launch_filter_diag(const Grid& g, const double* kf, double* dinv, hipStream_t s);

@@ -1578,11 +1578,13 @@ void launch_fcg_init(Reducer& red, int bb_region, int rr_region, double rtol2, b
 // them gives the same decision before and after that write (SC_DONE is only ever set to what they find themselves).
 // HBM bound: 6 vectors, 14 us at 128x64x64 (with r_prev written as a 7th vector, which z.q_old makes unnecessary, and
 // a one-block kernel for alpha before it: 17 + 4.7 us).
+template <bool JAC>
 __global__ __launch_bounds__(BS) void k_fcg_update(double* __restrict__ x, const double* __restrict__ p,
                                                    double* __restrict__ r, const double* __restrict__ q, long n,
                                                    const double* __restrict__ pq_part, int pq_nblk,
                                                    const double* __restrict__ rr_old, int rr_nblk, double* scal,
-                                                   double* part, double* look, int first) {
+                                                   double* part, double* look, int first,
+                                                   const double* __restrict__ dinv, double* dots) {
     const long i0 = blockIdx.x * (long)blockDim.x + threadIdx.x, st = (long)gridDim.x * blockDim.x;
     // the first values are in flight while the partials are summed
     double x0 = 0.0, p0 = 0.0, r0 = 0.0, q0 = 0.0;
@@ -1597,7 +1599,10 @@ __global__ __launch_bounds__(BS) void k_fcg_update(double* __restrict__ x, const
     if (!first) sum_partials<1>(rr_old, rr_nblk, rr);
     const bool zero = scal[SC_ZERO] != 0.0, done = scal[SC_DONE] != 0.0 || (!first && rr[0] <= scal[SC_TOL2]);
     const double gam = scal[SC_GAMMA], al = done ? 0.0 : gam / pq[0];
-    double acc[1] = {0.0};
+    constexpr int NA = JAC ? 3 : 1;
+    double acc[NA];
+#pragma unroll
+    for (int k = 0; k < NA; k++) acc[k] = 0.0;
     for (long i = i0; i < n; i += st) {
         if (i != i0) {
             x0 = x[i];
@@ -1610,12 +1615,21 @@ __global__ __launch_bounds__(BS) void k_fcg_update(double* __restrict__ x, const
         const double rn = done ? r0 : fma(-al, q0, r0);
         if (!done) r[i] = rn;
         acc[0] = fma(rn, rn, acc[0]);
+        if constexpr (JAC) {  // (q0 is the next direction's q_old)
+            const double z = dinv[i] * rn;
+            acc[1] = fma(z, rn, acc[1]);
+            acc[2] = fma(z, q0, acc[2]);
+        }
     }
-    __shared__ double sh[16];
-    block_sum<1>(acc, sh);
+    __shared__ double sh[16 * NA];
+    block_sum<NA>(acc, sh);
     if (threadIdx.x == 0) {  // the partial for the next update, and its copy for the host's look
         part[blockIdx.x] = acc[0];
         look[blockIdx.x] = acc[0];
+        if constexpr (JAC) {
+            dots[2 * blockIdx.x] = acc[1];
+            dots[2 * blockIdx.x + 1] = acc[2];
+        }
         if (blockIdx.x == 0) {
             const double it = scal[SC_ITERS] + (done ? 0.0 : 1.0);
             scal[SC_DONE] = done ? 1.0 : 0.0;
@@ -1627,28 +1641,178 @@ __global__ __launch_bounds__(BS) void k_fcg_update(double* __restrict__ x, const
     }
 }
 void launch_fcg_update(double* x, const double* p, double* r, const double* q, long n, Reducer& red, bool first,
-                       bool odd, hipStream_t s) {
+                       bool odd, hipStream_t s, const double* dinv) {
     const int nb = rb_blocks(n), now = rr_region(odd), old = rr_region(!odd);
     TT_CHECK(nb < Reducer::kLookBB, -3, "look buffer too small");
-    hipLaunchKernelGGL(k_fcg_update, dim3(nb), dim3(BS), 0, s, x, p, r, q, n, red.part(PB_PQ), red.nblk[PB_PQ],
-                       red.part(old), red.nblk[old], red.scal.p, red.part(now), red.look_dev, first ? 1 : 0);
+    auto launch = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3(nb), dim3(BS), 0, s, x, p, r, q, n, red.part(PB_PQ), red.nblk[PB_PQ],
+                           red.part(old), red.nblk[old], red.scal.p, red.part(now), red.look_dev, first ? 1 : 0, dinv,
+                           red.part(PB_DOTS));
+    };
+    if (dinv) {
+        launch(k_fcg_update<true>);
+        red.nblk[PB_DOTS] = nb;
+        red.nv[PB_DOTS] = 2;
+    } else {
+        launch(k_fcg_update<false>);
+    }
     red.nblk[now] = nb;
     red.nv[now] = 1;
     TT_HIP(hipGetLastError());
 }
 
-__global__ void k_fcg_direction(const double* __restrict__ z, const double* __restrict__ pold,
-                                double* __restrict__ pnew, long n, const double* __restrict__ dots, int dots_nblk,
-                                double* scal, int first) {
-    const double beta = fcg_beta(dots, dots_nblk, scal, first);
-    for (long i = blockIdx.x * (long)blockDim.x + threadIdx.x; i < n; i += (long)gridDim.x * blockDim.x)
-        pnew[i] = first ? z[i] : fma(beta, pold[i], z[i]);
+// ------------------------------------------------------------------ PDE filter operator (PDEFilter.cc)
+// On the node grid of a box the Helmholtz matrix is a sum of products of 1-D matrices (stiffness K = [-1 c -1] / h, mass
+// M = [1 2c 1] h / 6 per direction, c = the 1 or 2 elements at the node), R^2 (Kx My Mz + Mx Ky Mz + Mx My Kz) +
+// Mx My Mz.  A block owns 32 x 8 node columns and marches up its planes: a plane (with one halo node) is staged in LDS,
+// each thread forms A = My Mx u and B = (R^2 (Kx My + Mx Ky) + Mx My) u of its column from the 9 neighbours, and the
+// row sum is Mz B + R^2 Kz A over three planes.  The staged value is the solution (the residual) or the CG direction
+// formed on the fly.  At 128x64x64 a CG iteration's two kernels (this one and k_fcg_update) replace seven (48 us:
+// Jacobi, dots, beta, direction, an apply that gathered 64 products per node, alpha, update).
+constexpr int FX = 32, FY = 8, FHX = FX + 2, FHY = FY + 2;
+template <bool CG>  // CG: u = p = D^-1 r + beta p_old (written), y = q = A p, partials of p.q; else y = rhs - A u
+__global__ __launch_bounds__(256) void k_filter_op(GridArgs g, FilterOp f, int tx, int ty, int tz,
+                                                   const double* __restrict__ a0, const double* __restrict__ dinv,
+                                                   const double* __restrict__ a1, double* __restrict__ pnew,
+                                                   double* __restrict__ y, double* part0, double* part1, double* part2,
+                                                   const double* dots, int dots_nblk, double* scal, int first) {
+    __shared__ double su[2][FHX * FHY];
+    const int tid = threadIdx.x, lx = tid & 31, ly = tid >> 5;
+    const int tile = blockIdx.x, tzi = tile / (tx * ty), tr = tile - tzi * tx * ty, tyi = tr / tx, txi = tr - tyi * tx;
+    const int i0 = txi * FX, j0 = tyi * FY;
+    const int k0 = (int)((long)tzi * g.nz / tz), k1 = (int)((long)(tzi + 1) * g.nz / tz);
+    const int i = i0 + lx, j = j0 + ly;
+    const bool own = i < g.nx && j < g.ny;
+    double beta = 0.0;
+    if constexpr (CG) beta = fcg_beta(dots, dots_nblk, scal, first);
+    // 1-D rows of the thread's node (a neighbour outside the grid has weight 0 at a valid index)
+    auto row = [](int n, int nn, double h, double (&m)[3], double (&k)[3]) {
+        const double l = n > 0 ? 1.0 : 0.0, r = n < nn - 1 ? 1.0 : 0.0, c = l + r;
+        m[0] = l * (h / 6.0); m[1] = c * (h / 3.0); m[2] = r * (h / 6.0);
+        k[0] = -l / h; k[1] = c / h; k[2] = -r / h;
+    };
+    double mx[3], kx[3], my[3], ky[3];
+    row(i, g.nx, f.h[0], mx, kx);
+    row(j, g.ny, f.h[1], my, ky);
+    // staging: two of the 340 box nodes per thread
+    int so[2];
+    bool sv[2];
+#pragma unroll
+    for (int q = 0; q < 2; q++) {
+        const int v = tid + q * 256, sy = v / FHX, sx = v - sy * FHX;
+        sv[q] = v < FHX * FHY;
+        so[q] = min(max(i0 - 1 + sx, 0), g.nx - 1) + g.nx * min(max(j0 - 1 + sy, 0), g.ny - 1);
+    }
+    const int plane = g.nx * g.ny;
+    double v0[2], v1[2], v2[2];
+    auto load = [&](int k) {
+        const size_t b = (size_t)min(max(k, 0), g.nz - 1) * plane;
+#pragma unroll
+        for (int q = 0; q < 2; q++) {
+            v0[q] = a0[b + so[q]];
+            if constexpr (CG) {
+                v1[q] = dinv[b + so[q]];
+                v2[q] = first ? 0.0 : a1[b + so[q]];
+            }
+        }
+    };
+    auto commit = [&](int b) {
+#pragma unroll
+        for (int q = 0; q < 2; q++) {
+            double x = v0[q];
+            if constexpr (CG) {
+                x = v1[q] * v0[q];
+                if (!first) x = fma(beta, v2[q], x);
+            }
+            if (sv[q]) su[b][tid + q * 256] = x;
+        }
+    };
+    double A[3] = {0, 0, 0}, B[3] = {0, 0, 0}, uo[2] = {0, 0}, acc[3] = {0, 0, 0};
+    load(k0 - 1);
+    commit(0);
+    __syncthreads();
+    for (int k = k0 - 1; k <= k1; k++) {  // plane k is staged in su[(k - k0 + 1) & 1]
+        const int sb = (k - k0 + 1) & 1;
+        if (k < k1) load(k + 1);
+        double As = 0.0, Bs = 0.0;
+        const double* u = &su[sb][ly * FHX + lx];
+#pragma unroll
+        for (int r = 0; r < 3; r++) {
+            const double ul = u[r * FHX], uc = u[r * FHX + 1], ur = u[r * FHX + 2];
+            const double um = fma(mx[0], ul, fma(mx[1], uc, mx[2] * ur)), uk = fma(kx[0], ul, fma(kx[1], uc, kx[2] * ur));
+            As = fma(my[r], um, As);
+            Bs = fma(my[r], fma(f.R2, uk, um), Bs);
+            Bs = fma(f.R2 * ky[r], um, Bs);
+        }
+        const double un = u[FHX + 1];
+        A[0] = A[1]; A[1] = A[2]; A[2] = As;
+        B[0] = B[1]; B[1] = B[2]; B[2] = Bs;
+        const int kk = k - 1;  // the plane whose three neighbours are now known
+        if (kk >= k0 && own) {
+            double mz[3], kz[3];
+            row(kk, g.nz, f.h[2], mz, kz);
+            double s = 0.0;
+#pragma unroll
+            for (int d = 0; d < 3; d++) s = fma(mz[d], B[d], fma(f.R2 * kz[d], A[d], s));
+            const size_t n = (size_t)kk * plane + i + (size_t)g.nx * j;
+            if constexpr (CG) {
+                y[n] = s;
+                pnew[n] = uo[0];
+                acc[0] = fma(uo[0], s, acc[0]);
+            } else {
+                const double b = a1[n], r = b - s;
+                y[n] = r;
+                acc[0] = fma(r, r, acc[0]);
+                acc[1] = fma(dinv[n] * r, r, acc[1]);
+                acc[2] = fma(b, b, acc[2]);
+            }
+        }
+        uo[0] = un;
+        if (k < k1) commit(sb ^ 1);
+        __syncthreads();
+    }
+    __shared__ double sh[16 * 3];
+    block_sum<3>(acc, sh);
+    if (tid == 0) {
+        part0[tile] = acc[0];
+        if constexpr (!CG) {
+            part1[2 * tile] = acc[1];
+            part1[2 * tile + 1] = 0.0;
+            if (part2) part2[tile] = acc[2];
+        }
+    }
 }
-void launch_fcg_direction(const double* z, const double* p_old, double* p_new, long n, Reducer& red, bool first,
-                          hipStream_t s) {
-    hipLaunchKernelGGL(k_fcg_direction, dim3(rb_blocks(n)), dim3(BS), 0, s, z, p_old, p_new, n, red.part(PB_DOTS),
+// tiles: about 4 blocks per CU, at least one plane each
+static inline dim3 filter_tiles(const Grid& g) {
+    const int tx = (g.nx + FX - 1) / FX, ty = (g.ny + FY - 1) / FY;
+    return dim3(tx, ty, std::min(g.nz, std::max(1, 1024 / (tx * ty))));
+}
+void launch_filter_residual(const Grid& g, const FilterOp& f, const double* U, const double* rhs, const double* dinv,
+                            double* r, Reducer& red, bool bb, hipStream_t s) {
+    const dim3 t = filter_tiles(g);
+    const int nb = t.x * t.y * t.z;
+    TT_CHECK(nb <= red.maxblocks, -3, "reducer too small");
+    hipLaunchKernelGGL(k_filter_op<false>, dim3(nb), dim3(256), 0, s, gargs(g), f, (int)t.x, (int)t.y, (int)t.z, U, dinv,
+                       rhs, (double*)nullptr, r, red.part(PB_MISC2), red.part(PB_DOTS),
+                       bb ? red.part(PB_MISC) : (double*)nullptr, (const double*)nullptr, 0, (double*)nullptr, 0);
+    TT_HIP(hipGetLastError());
+    for (int region : {(int)PB_MISC2, (int)PB_DOTS, (int)PB_MISC})
+        if (region != PB_MISC || bb) {
+            red.nblk[region] = nb;
+            red.nv[region] = region == PB_DOTS ? 2 : 1;
+        }
+}
+void launch_filter_direction(const Grid& g, const FilterOp& f, const double* r, const double* dinv, const double* p_old,
+                             double* p_new, double* q, Reducer& red, bool first, hipStream_t s) {
+    const dim3 t = filter_tiles(g);
+    const int nb = t.x * t.y * t.z;
+    TT_CHECK(nb <= red.maxblocks, -3, "reducer too small");
+    hipLaunchKernelGGL(k_filter_op<true>, dim3(nb), dim3(256), 0, s, gargs(g), f, (int)t.x, (int)t.y, (int)t.z, r, dinv,
+                       p_old, p_new, q, red.part(PB_PQ), (double*)nullptr, (double*)nullptr, red.part(PB_DOTS),
                        red.nblk[PB_DOTS], red.scal.p, first ? 1 : 0);
     TT_HIP(hipGetLastError());
+    red.nblk[PB_PQ] = nb;
+    red.nv[PB_PQ] = 1;
 }
 
 __global__ void k_jacobi(const double* __restrict__ dinv, const double* __restrict__ r, double* __restrict__ z,

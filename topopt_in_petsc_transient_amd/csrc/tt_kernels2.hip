@@ -244,52 +244,6 @@ void launch_sens(const SensArgs& a, Reducer& red, double* fx_out, hipStream_t st
 }
 
 // ------------------------------------------------------------------ PDE filter (PDEFilter.cc)
-// y_n = sum_{e at n} sum_b KF[a][b] U_{node(e,b)}  (constant-coefficient scalar hex8 operator)
-__global__ void k_filter_apply(GA g, const double* __restrict__ KF, const double* __restrict__ u,
-                               double* __restrict__ y, double* partials, unsigned* counter, double* out) {
-    const long n = blockIdx.x * (long)blockDim.x + threadIdx.x;
-    const long nn = (long)g.nx * g.ny * g.nz;
-    double acc[1] = {0.0};
-    if (n < nn) {
-        int i, j, k;
-        grid_ijk((unsigned)n, g.nx, g.ny, i, j, k);
-        double s = 0.0;
-#pragma unroll
-        for (int ez = 0; ez < 2; ez++)
-#pragma unroll
-            for (int ey = 0; ey < 2; ey++)
-#pragma unroll
-                for (int ex = 0; ex < 2; ex++) {
-                    const int ei = i - 1 + ex, ej = j - 1 + ey, ek = k - 1 + ez;
-                    if (ei < 0 || ej < 0 || ek < 0 || ei >= g.ex || ej >= g.ey || ek >= g.ez) continue;
-                    const int a = (1 - ez) * 4 + ((1 - ey) == 0 ? ((1 - ex) == 0 ? 0 : 1) : ((1 - ex) == 1 ? 2 : 3));
-#pragma unroll
-                    for (int b = 0; b < 8; b++) {
-                        const int bx = ((b & 3) == 1 || (b & 3) == 2), by = (b & 3) >= 2, bz = b >> 2;
-                        const long m = (ei + bx) + (long)g.nx * ((ej + by) + (long)g.ny * (ek + bz));
-                        s = fma(KF[a * 8 + b], u[m], s);
-                    }
-                }
-        y[n] = s;
-        acc[0] = s * u[n];
-    }
-    if (partials) rfinish<1>(acc, partials, counter, out);
-}
-void launch_filter_apply(const Grid& g, const double* kf, const double* u, double* y, Reducer* red, int dot_slot,
-                         hipStream_t s) {
-    const int nb = nblk(g.nn);
-    if (red) {
-        TT_CHECK(nb <= red->maxblocks, -3, "reducer too small for filter apply");
-        hipLaunchKernelGGL(k_filter_apply, dim3(nb), dim3(BS2), 0, s, ga(g), kf, u, y, red->part(dot_slot),
-                           (unsigned*)nullptr, (double*)nullptr);
-        set_region(*red, dot_slot, nb, 1);
-    } else {
-        hipLaunchKernelGGL(k_filter_apply, dim3(nb), dim3(BS2), 0, s, ga(g), kf, u, y, (double*)nullptr,
-                           (unsigned*)nullptr, (double*)nullptr);
-    }
-    TT_HIP(hipGetLastError());
-}
-
 // rhs_n = scale * sum_{e at n} x_e / 8   (T x, PDEFilter.cc:580-588, scaled by the element volume at :208)
 __global__ void k_filter_T(GA g, const double* __restrict__ x, double scale, double* __restrict__ rhs) {
     const long n = blockIdx.x * (long)blockDim.x + threadIdx.x;
