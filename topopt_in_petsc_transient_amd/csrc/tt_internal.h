@@ -235,7 +235,10 @@ struct OpLevel {
 // packing of a full symmetric matrix, and x = A b with per-tile partials (nt (nt + 1) / 2 x 64 each).
 long sym_packed_size(int n);
 void launch_sym_pack(const double* A, int n, double* P, hipStream_t s);
-void launch_sym_solve(const double* P, const double* b, double* x, int n, double* prow, double* pcol, hipStream_t s);
+// Up to order kDenseMvMax the full matrix A is used instead.
+constexpr int kDenseMvMax = 1536;
+void launch_sym_solve(const double* A, const double* P, const double* b, double* x, int n, double* prow, double* pcol,
+                      hipStream_t s);
 // Dense N (cK K + cM M) N + I - N of a (coarsest) level from its FP64 element coefficients, on the device
 // (row-major n x n, n = g.nd; cleared first).
 void launch_dense_coarse(const Grid& g, const double* kf, const double* mf, double cK, double cM, const double* KE,
@@ -297,9 +300,10 @@ void launch_cheb_last(const OpLevel& L, double cK, double cM, const void* b, con
 // bc = R rf (fine precision fp64; an FP32 fine level may write an FP64 coarse vector, out64)
 void launch_restrict(const Grid& fine, const Grid& coarse, const void* rf, const uint8_t* cmask, void* bc,
                      bool fp64, bool out64, hipStream_t s);
-// xf += P xc (fine precision fp64; an FP32 fine level may read an FP64 coarse vector, in64)
-void launch_prolong_add(const Grid& fine, const Grid& coarse, const void* xc, const uint8_t* fmask, void* xf,
-                        bool fp64, bool in64, hipStream_t s);
+// xf += sum_l P_l xc[l]: the corrections of the n coarser levels coarse[0..n-1] (each 2:1 from the one before, the first
+// from `fine`), in the fine precision except that an FP32 fine level may read an FP64 last one (last64)
+void launch_prolong_chain(const Grid& fine, int n, const Grid* const* coarse, const void* const* xc,
+                          const uint8_t* fmask, void* xf, bool fp64, bool last64, hipStream_t s);
 void launch_coarsen_coef(const Grid& fine, const Grid& coarse, const double* kf_f, const double* mf_f, double* kf_c,
                          double* mf_c, hipStream_t s);
 void launch_convert_coef(const double* src, void* dst, long n, int kind, hipStream_t s);

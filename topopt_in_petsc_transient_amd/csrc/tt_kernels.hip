@@ -990,55 +990,68 @@ void launch_restrict(const Grid& fine, const Grid& coarse, const void* rf, const
     TT_HIP(hipGetLastError());
 }
 
-// xf += P xc on free dofs.  Each fine node interpolates from 1, 2, 4 or 8 coarse nodes; the
-// unrolled 2 x 2 x 2 loop gives a second node of a direction weight 0 (at a valid index) where the
-// fine index is even, so the sum is the same as over the contributing nodes only.
-template <typename Tf, typename Tc>
-__global__ void k_prolong_add(GridArgs f, GridArgs c, const Tc* __restrict__ xc, const uint8_t* __restrict__ fmask,
-                              Tf* __restrict__ xf) {
+// xf += P_1 x_1 + P_2 x_2 + ... on free dofs: the corrections of one or several coarser levels, each interpolated to the
+// fine nodes directly.  Nested trilinear interpolation is trilinear on the coarser cells, and a level's clamped dofs lie
+// on faces and edges whose coarse nodes are clamped (zero) too, so a chain of prolongations through the levels between,
+// x_1 += P x_2 and then xf += P x_1, is this sum: one kernel per V-cycle instead of one per level where the
+// intermediate levels do not smooth after the correction.  Level l's node of fine node i is i >> l with weight
+// (1 - f), f = (i mod 2^l) / 2^l, and its successor with f (at a valid index when f = 0).  At 128x64x64 (4 levels) 7.0 +
+// 4.0 + 3.4 us for the three kernels before.
+struct ProlongChain {
+    const void* x[7];
+    int nx[7], ny[7];
+    int n;
+};
+template <typename Tf, typename Tx>
+__device__ __forceinline__ void prolong_level(const Tx* __restrict__ x, int nx, int ny, int l, int i, int j, int k,
+                                              Tf (&s)[3]) {
+    const Tf inv = (Tf)1 / (Tf)(1 << l);
+    const int fi = i & ((1 << l) - 1), fj = j & ((1 << l) - 1), fk = k & ((1 << l) - 1);
+    const Tf wi = (Tf)fi * inv, wj = (Tf)fj * inv, wk = (Tf)fk * inv;
+    const int di = fi ? 3 : 0, dj = fj ? 3 * nx : 0, dk = fk ? 3 * nx * ny : 0;
+    const Tx* p = x + 3 * ((size_t)(i >> l) + (size_t)nx * ((j >> l) + (size_t)ny * (k >> l)));
+#pragma unroll
+    for (int q = 0; q < 8; q++) {
+        const Tf w = ((q & 1) ? wi : (Tf)1 - wi) * ((q & 2) ? wj : (Tf)1 - wj) * ((q & 4) ? wk : (Tf)1 - wk);
+        const Tx* pq = p + ((q & 1) ? di : 0) + ((q & 2) ? dj : 0) + ((q & 4) ? dk : 0);
+#pragma unroll
+        for (int c = 0; c < 3; c++) s[c] = fma(w, (Tf)pq[c], s[c]);
+    }
+}
+template <typename Tf, typename Tl>  // Tl: the last (coarsest) level's type
+__global__ void k_prolong_chain(GridArgs f, ProlongChain pc, const uint8_t* __restrict__ fmask, Tf* __restrict__ xf) {
     const long n = blockIdx.x * (long)blockDim.x + threadIdx.x;
     if (n >= (long)f.nx * f.ny * f.nz) return;
     int i, j, k;
     grid_ijk((unsigned)n, f.nx, f.ny, i, j, k);
-    const int I0 = i >> 1, J0 = j >> 1, K0 = k >> 1;
-    const int oi = i & 1, oj = j & 1, ok = k & 1;
-    Tf s0 = 0, s1 = 0, s2 = 0;
-#pragma unroll
-    for (int kk = 0; kk < 2; kk++) {
-        const Tf wk = ok ? (Tf)0.5 : (kk ? (Tf)0 : (Tf)1);
-        const int K = K0 + (kk & ok);
-#pragma unroll
-        for (int jj = 0; jj < 2; jj++) {
-            const Tf wj = oj ? wk * (Tf)0.5 : (jj ? (Tf)0 : wk);
-            const int J = J0 + (jj & oj);
-#pragma unroll
-            for (int ii = 0; ii < 2; ii++) {
-                const Tf w = oi ? wj * (Tf)0.5 : (ii ? (Tf)0 : wj);
-                const int I = I0 + (ii & oi);
-                const long m = I + (long)c.nx * (J + (long)c.ny * K);
-                s0 = fma(w, (Tf)xc[3 * m], s0);
-                s1 = fma(w, (Tf)xc[3 * m + 1], s1);
-                s2 = fma(w, (Tf)xc[3 * m + 2], s2);
-            }
-        }
-    }
     const uint8_t cl = fmask[n];
-    if (!(cl & 1)) xf[3 * n] += s0;
-    if (!(cl & 2)) xf[3 * n + 1] += s1;
-    if (!(cl & 4)) xf[3 * n + 2] += s2;
+    Tf x[3], s[3] = {0, 0, 0};
+#pragma unroll
+    for (int c = 0; c < 3; c++) x[c] = xf[3 * n + c];
+    for (int l = 0; l + 1 < pc.n; l++)
+        prolong_level<Tf, Tf>((const Tf*)pc.x[l], pc.nx[l], pc.ny[l], l + 1, i, j, k, s);
+    prolong_level<Tf, Tl>((const Tl*)pc.x[pc.n - 1], pc.nx[pc.n - 1], pc.ny[pc.n - 1], pc.n, i, j, k, s);
+#pragma unroll
+    for (int c = 0; c < 3; c++)
+        if (!((cl >> c) & 1)) xf[3 * n + c] = x[c] + s[c];
 }
-void launch_prolong_add(const Grid& fine, const Grid& coarse, const void* xc, const uint8_t* fmask, void* xf,
-                        bool fp64, bool in64, hipStream_t s) {
+void launch_prolong_chain(const Grid& fine, int n, const Grid* const* coarse, const void* const* xc,
+                          const uint8_t* fmask, void* xf, bool fp64, bool last64, hipStream_t s) {
+    TT_CHECK(n >= 1 && n <= 7, -3, "launch_prolong_chain: 1..7 levels");
+    ProlongChain pc{};
+    pc.n = n;
+    for (int l = 0; l < n; l++) {
+        pc.x[l] = xc[l];
+        pc.nx[l] = coarse[l]->nx;
+        pc.ny[l] = coarse[l]->ny;
+    }
     const dim3 gr(nblocks(fine.nn)), bl(BS);
     if (fp64)
-        hipLaunchKernelGGL((k_prolong_add<double, double>), gr, bl, 0, s, gargs(fine), gargs(coarse),
-                           (const double*)xc, fmask, (double*)xf);
-    else if (in64)
-        hipLaunchKernelGGL((k_prolong_add<float, double>), gr, bl, 0, s, gargs(fine), gargs(coarse),
-                           (const double*)xc, fmask, (float*)xf);
+        hipLaunchKernelGGL((k_prolong_chain<double, double>), gr, bl, 0, s, gargs(fine), pc, fmask, (double*)xf);
+    else if (last64)
+        hipLaunchKernelGGL((k_prolong_chain<float, double>), gr, bl, 0, s, gargs(fine), pc, fmask, (float*)xf);
     else
-        hipLaunchKernelGGL((k_prolong_add<float, float>), gr, bl, 0, s, gargs(fine), gargs(coarse),
-                           (const float*)xc, fmask, (float*)xf);
+        hipLaunchKernelGGL((k_prolong_chain<float, float>), gr, bl, 0, s, gargs(fine), pc, fmask, (float*)xf);
     TT_HIP(hipGetLastError());
 }
 
@@ -1260,80 +1273,109 @@ void launch_sym_pack(const double* A, int n, double* P, hipStream_t s) {
     hipLaunchKernelGGL(k_sym_pack, dim3(nt, nt), dim3(256), 0, s, A, n, P);
     TT_HIP(hipGetLastError());
 }
-// per tile: row sums A_IJ x_J and (off the diagonal) column sums A_IJ^T x_I, written as FP64
-// partials.  Each thread first loads its 16 tile values (16-byte loads, all in flight), then the
-// tile goes through LDS once.
-template <typename PT>
-__global__ __launch_bounds__(256) void k_sym_tiles(const PT* __restrict__ P, const double* __restrict__ x, int n,
+// per tile: row sums A_IJ x_J and (off the diagonal) column sums A_IJ^T x_I, written as FP64 partials.  Each thread
+// holds 8 rows (tid / 32 + 8 k) x 2 columns of the tile in registers (16-byte loads, all in flight): its columns' sums go
+// through LDS over the 8 row groups, its rows' over the 32 lanes of the half wave by halving exchanges (9 instead of
+// 40 shuffles).  HBM bound: 68 MB at 4,131 dofs, see k_sym_sum.
+__global__ __launch_bounds__(256) void k_sym_tiles(const double* __restrict__ P, const double* __restrict__ x, int n,
                                                    double* __restrict__ prow, double* __restrict__ pcol) {
-    __shared__ double tile[ST][ST + 1];
-    __shared__ double xs[2][ST];
-    __shared__ double red[4][ST];
+    __shared__ double cs[8][ST];
     const int id = blockIdx.x;
     int I = (int)((sqrt(8.0 * id + 1.0) - 1.0) * 0.5);  // I (I + 1) / 2 <= id < (I + 1)(I + 2) / 2
     while ((I + 1) * (I + 2) / 2 <= id) I++;
     while (I * (I + 1) / 2 > id) I--;
     const int J = id - I * (I + 1) / 2;
-    constexpr int VW = 16 / sizeof(PT), NL = ST * ST / (256 * VW);  // values per load, loads per thread
-    using V = typename std::conditional<VW == 2, double2, float4>::type;
-    const V* T2 = reinterpret_cast<const V*>(P + (size_t)id * ST * ST);
-    const int tid = threadIdx.x;
-    V v[NL];
+    const double2* T2 = reinterpret_cast<const double2*>(P + (size_t)id * ST * ST);
+    const int tid = threadIdx.x, rg = tid >> 5, c = 2 * (tid & 31);
+    double2 v[8];
 #pragma unroll
-    for (int k = 0; k < NL; k++) v[k] = T2[tid + 256 * k];
+    for (int k = 0; k < 8; k++) v[k] = T2[tid + 256 * k];
+    const int j = J * ST + c, i = I * ST + rg;
+    const double x0 = j < n ? x[j] : 0.0, x1 = j + 1 < n ? x[j + 1] : 0.0;
+    double xi[8], rs[8], c0 = 0.0, c1 = 0.0;
+#pragma unroll
+    for (int k = 0; k < 8; k++) xi[k] = i + 8 * k < n ? x[i + 8 * k] : 0.0;
+#pragma unroll
+    for (int k = 0; k < 8; k++) {
+        rs[k] = fma(v[k].x, x0, v[k].y * x1);
+        c0 = fma(v[k].x, xi[k], c0);
+        c1 = fma(v[k].y, xi[k], c1);
+    }
+    cs[rg][c] = c0;
+    cs[rg][c + 1] = c1;
+    // after the exchange over lane bit 4, 3, 2 a lane keeps 4, 2, 1 of its rows
+    int row = rg;
+#pragma unroll
+    for (int b = 0; b < 3; b++) {
+        const int h = 4 >> b, bit = 16 >> b;
+        const bool up = (tid & bit) != 0;
+        row += up ? 8 * h : 0;
+#pragma unroll
+        for (int m = 0; m < 4; m++)
+            if (m < h) {
+                const double keep = up ? rs[m + h] : rs[m], send = up ? rs[m] : rs[m + h];
+                rs[m] = keep + __shfl_xor(send, bit, 64);
+            }
+    }
+    rs[0] += __shfl_xor(rs[0], 2, 64);
+    rs[0] += __shfl_xor(rs[0], 1, 64);
+    if ((tid & 3) == 0) prow[(size_t)id * ST + row] = rs[0];
+    __syncthreads();
     if (tid < ST) {
-        const int j = J * ST + tid, i = I * ST + tid;
-        xs[0][tid] = j < n ? x[j] : 0.0;
-        xs[1][tid] = i < n ? x[i] : 0.0;
-    }
+        double s = 0.0;
 #pragma unroll
-    for (int k = 0; k < NL; k++) {
-        const int e = VW * (tid + 256 * k);
-        const PT* pv = reinterpret_cast<const PT*>(&v[k]);
-#pragma unroll
-        for (int q = 0; q < VW; q++) tile[e / ST][e % ST + q] = (double)pv[q];
+        for (int q = 0; q < 8; q++) s += cs[q][tid];
+        pcol[(size_t)id * ST + tid] = I == J ? 0.0 : s;
     }
-    __syncthreads();
-    const int part = tid >> 6, k = tid & 63;  // 4 x 64 threads: rows (parts 0, 1) and columns (parts 2, 3)
-    double sacc = 0.0;
-    if (part < 2) {
-#pragma unroll 8
-        for (int c = part * 32; c < part * 32 + 32; c++) sacc = fma(tile[k][c], xs[0][c], sacc);
-    } else {
-#pragma unroll 8
-        for (int r = (part - 2) * 32; r < (part - 2) * 32 + 32; r++) sacc = fma(tile[r][k], xs[1][r], sacc);
-    }
-    red[part][k] = sacc;
-    __syncthreads();
-    if (tid < ST) prow[(size_t)id * ST + tid] = red[0][tid] + red[1][tid];
-    else if (tid < 2 * ST) pcol[(size_t)id * ST + (tid - ST)] = I == J ? 0.0 : red[2][tid - ST] + red[3][tid - ST];
 }
-// y_i = sum_{J <= I} prow(I, J) + sum_{K > I} pcol(K, I): one block of 256 threads per tile row I,
-// 4 threads per output summing every 4th partial, combined in a fixed order
-__global__ __launch_bounds__(256) void k_sym_sum(const double* __restrict__ prow, const double* __restrict__ pcol,
-                                                 int n, int nt, double* __restrict__ y) {
-    __shared__ double red[4][ST];
+// y_i = sum_{J <= I} prow(I, J) + sum_{K > I} pcol(K, I): one block per tile row I, 16 threads per output summing every
+// 16th partial (their loads in flight together), combined in a fixed order
+__global__ __launch_bounds__(1024) void k_sym_sum(const double* __restrict__ prow, const double* __restrict__ pcol,
+                                                  int n, int nt, double* __restrict__ y) {
+    __shared__ double red[16][ST];
     const int I = blockIdx.x, q = threadIdx.x >> 6, r = threadIdx.x & 63;
     double s = 0.0;
-    for (int m = q; m < nt; m += 4) {  // m <= I: tile (I, m) rows; m > I: tile (m, I) columns
-        s += m <= I ? prow[((size_t)I * (I + 1) / 2 + m) * ST + r] : pcol[((size_t)m * (m + 1) / 2 + I) * ST + r];
+#pragma unroll 8
+    for (int m = q; m < nt; m += 16) {  // m <= I: tile (I, m) rows; m > I: tile (m, I) columns
+        const double* p = m <= I ? prow + ((size_t)I * (I + 1) / 2 + m) * ST : pcol + ((size_t)m * (m + 1) / 2 + I) * ST;
+        s += p[r];
     }
     red[q][r] = s;
     __syncthreads();
     const int i = I * ST + threadIdx.x;
-    if (threadIdx.x < ST && i < n) y[i] = (red[0][threadIdx.x] + red[1][threadIdx.x]) + (red[2][threadIdx.x] + red[3][threadIdx.x]);
+    if (threadIdx.x < ST && i < n) {
+        double t = 0.0;
+#pragma unroll
+        for (int g = 0; g < 16; g++) t += red[g][threadIdx.x];
+        y[i] = t;
+    }
 }
-template <typename PT>
-static void sym_solve(const PT* P, const double* b, double* x, int n, double* prow, double* pcol, hipStream_t s) {
-    const int nt = sym_tiles(n);
-    hipLaunchKernelGGL(k_sym_tiles<PT>, dim3(nt * (nt + 1) / 2), dim3(256), 0, s, P, b, n, prow, pcol);
-    TT_HIP(hipGetLastError());
-    hipLaunchKernelGGL(k_sym_sum, dim3(nt), dim3(256), 0, s, prow, pcol, n, nt, x);
-    TT_HIP(hipGetLastError());
+// y = A x with the full matrix, one wave per row: for small orders, where the matrix sits in L2 and the second launch of
+// the packed form is what counts
+__global__ __launch_bounds__(256) void k_dense_mv(const double* __restrict__ A, const double* __restrict__ x, int n,
+                                                  double* __restrict__ y) {
+    const int row = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+    if (row >= n) return;
+    const double* a = A + (size_t)row * n;
+    double s = 0.0;
+#pragma unroll 8
+    for (int j = lane; j < n; j += 64) s = fma(a[j], x[j], s);
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off, 64);
+    if (lane == 0) y[row] = s;
 }
-void launch_sym_solve(const double* P, const double* b, double* x, int n, double* prow, double* pcol,
+void launch_sym_solve(const double* A, const double* P, const double* b, double* x, int n, double* prow, double* pcol,
                       hipStream_t s) {
-    sym_solve(P, b, x, n, prow, pcol, s);
+    if (n <= kDenseMvMax) {
+        hipLaunchKernelGGL(k_dense_mv, dim3((n + 3) / 4), dim3(256), 0, s, A, b, n, x);
+        TT_HIP(hipGetLastError());
+        return;
+    }
+    const int nt = sym_tiles(n);
+    hipLaunchKernelGGL(k_sym_tiles, dim3(nt * (nt + 1) / 2), dim3(256), 0, s, P, b, n, prow, pcol);
+    TT_HIP(hipGetLastError());
+    hipLaunchKernelGGL(k_sym_sum, dim3(nt), dim3(1024), 0, s, prow, pcol, n, nt, x);
+    TT_HIP(hipGetLastError());
 }
 
 // ------------------------------------------------------------------ reductions / Krylov

@@ -327,13 +327,13 @@ void Multigrid::coarse_solve(bool direct64) {
         b64 = cb.p;
         x64 = cx.p;
         if (direct64) {
-            launch_sym_solve(AinvP.p, b64, x64, nc, sprow.p, spcol.p, s);
+            launch_sym_solve(Ainv.p, AinvP.p, b64, x64, nc, sprow.p, spcol.p, s);
             return;
         }
         launch_copy(lc.b.p, cb.p, nc, false, true, s);
     }
     if (dense) {
-        launch_sym_solve(AinvP.p, b64, x64, nc, sprow.p, spcol.p, s);
+        launch_sym_solve(Ainv.p, AinvP.p, b64, x64, nc, sprow.p, spcol.p, s);
     } else {
         OpLevel op = coarse_op64();
         const double theta = 0.5 * (clmax + clmin), delta = 0.5 * (clmax - clmin), sigma = theta / delta;
@@ -413,7 +413,22 @@ void Multigrid::vcycle(int l, const double* r64, double* z64, const double* q64,
     const bool direct64 = l + 2 == nl && dense && !lc.fp64;
     launch_restrict(lv.g, lc.g, lv.r.p, lc.mask.p, direct64 ? (void*)cb.p : lc.b.p, f64, direct64, s);
     vcycle(l + 1);
-    launch_prolong_add(lv.g, lc.g, direct64 ? (const void*)cx.p : lc.x.p, lv.mask.p, lv.x.p, f64, direct64, s);
+    // An intermediate level that does not smooth after its correction leaves it to the finest level's prolongation,
+    // which interpolates the corrections of all coarser levels in one pass.
+    const bool chain = coarse_post == 0;
+    if (l == 0 || !chain) {
+        const Grid* gc[8];
+        const void* xc[8];
+        int n = 0;
+        bool last64 = false;
+        for (int c = l + 1; c < nl && (n == 0 || chain); c++, n++) {
+            const bool d64 = c == nl - 1 && dense && !L[c]->fp64;  // the coarsest solve's FP64 vector
+            gc[n] = &L[c]->g;
+            xc[n] = d64 ? (const void*)cx.p : L[c]->x.p;
+            last64 = d64;
+        }
+        launch_prolong_chain(lv.g, n, gc, xc, lv.mask.p, lv.x.p, f64, last64, s);
+    }
     // post-smoothing
     rho0 = 1.0 / sigma;
     for (int k = 0; k < npost; k++) {
