@@ -71,7 +71,12 @@ static int plan(int ex, int ey, int ez) {
     int bad = 0;
     for (int d = 0; d < 2; d++) {
         const ColPlan p = make_col_plan(g, d != 0);
+        if (p.cx == 0) {  // the one-shot kernel's 4 x 4 x 4 tiles
+            bad += p.tx != (ex + 4) / 4 || p.ty != (ey + 4) / 4 || p.tz != (ez + 4) / 4 || g.nn > kBoxNodes;
+            continue;
+        }
         const int cy = p.by + 1;
+        bad += g.nn <= kBoxNodes;
         bad += p.bx < 1 || p.by < 1 || p.cx != p.bx + 1 || p.cx * cy > 256 || 3 * (p.cx + 1) * (cy + 1) > 1024;
         bad += p.tx * p.bx < g.nx || (p.tx - 1) * p.bx >= g.nx || p.ty * p.by < g.ny || (p.ty - 1) * p.by >= g.ny;
         bad += p.tz < 1 || p.tz > g.nz;
@@ -102,8 +107,8 @@ static int plan(int ex, int ey, int ez) {
 int main() {
     int bad = 0;
     const int ext[] = {1, 2, 3, 7, 8, 15, 16, 17, 31, 64, 97};
-    for (int x : ext) for (int y : ext) for (int z : ext) if (x * y * z <= 40000) bad += plan(x, y, z);
-    bad += plan(128, 64, 64) + plan(300, 1, 1) + plan(1, 300, 2) + plan(2, 1, 700);
+    for (int x : ext) for (int y : ext) for (int z : ext) if (x * y * z <= 150000) bad += plan(x, y, z);
+    bad += plan(128, 64, 64) + plan(30000, 1, 1) + plan(1, 11000, 2) + plan(2, 1, 9000) + plan(300, 11, 12);
     bad += modes(0.1, 0.1, 0.1, 0.3) + modes(1, 1, 1, 0.0) + modes(0.01, 0.2, 3.0, 0.45) + modes(2, 0.3, 0.3, -0.4);
     printf("bad %d\n", bad);
     return bad != 0;

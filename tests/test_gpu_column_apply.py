@@ -1,6 +1,7 @@
-"""The column operator kernel (csrc/tt_apply_cols.inc) against the oracle where its tiling can go wrong: grids of one
-element, single rows and planes, extents at and around the tile edges, long thin boxes of one tile and of many, with
-both boundary masks (clamped dofs inside and at the edges of tiles).
+"""The operator kernels (csrc/tt_apply_box.inc for small grids, csrc/tt_apply_cols.inc for the others) against the oracle
+where their tilings can go wrong: grids of one element, single rows and planes, extents at and around the tile edges,
+long thin boxes, the sizes on both sides of the rule between the two kernels, with both boundary masks (clamped dofs
+inside and at the edges of tiles).
 
 Tolerance: a result is a sum of at most 8 element contributions, each reached through about 25 rounded operations from
 the inputs (3 + 3 levels of sums, the block products, the coefficients), and the element products of random inputs do
@@ -17,7 +18,9 @@ from topopt_in_petsc_transient_amd import capi
 pytestmark = pytest.mark.gpu
 
 GRIDS = [(1, 1, 1), (2, 1, 3), (7, 5, 3), (15, 15, 2), (16, 8, 9), (17, 31, 1), (3, 70, 2), (130, 2, 2), (2, 3, 150),
-         (61, 43, 5)]
+         (61, 43, 5),
+         # above 40,000 nodes: the column kernel
+         (130, 20, 15), (17, 47, 50), (300, 11, 12), (3, 3, 3000), (2, 4000, 3), (3999, 2, 3), (31, 31, 39), (15, 49, 49)]
 
 
 @pytest.mark.parametrize("nel", GRIDS)

@@ -93,7 +93,7 @@ Context::Context(const tt_params& p) : prm(p) {
     TT_HIP(hipMemcpy(mask.p, m.data(), nn, hipMemcpyHostToDevice));
     split.build(g, m);
     // (an apply writes one partial per block; coarser levels have fewer nodes and no more blocks)
-    const long apply_blocks = 8 * ((std::max(split.s32.plan.ntiles(), split.s64.plan.ntiles()) + 7) / 8);
+    const long apply_blocks = std::max(split.s32.plan.blocks(), split.s64.plan.blocks());
     red.init((int)std::max<long>({apply_blocks, (nel + 255) / 256, (nn + 255) / 256, 2048}));
     F.alloc(nd);
     TT_HIP(hipMemcpy(F.p, Fhost.data(), nd * 8, hipMemcpyHostToDevice));
@@ -559,7 +559,7 @@ int tt_time_fcg_apply(tt_ctx* ctx, int nrep, double* ms) {
     tt::launch_fill_hash(C.kz.p, nd, 0x51ED270B27A1F00Dull, true, C.stream);
     tt::launch_fill_hash(C.kp0.p, nd, 0x2F1C3A5B4D6E7F81ull, true, C.stream);
     tt::launch_fill_hash(C.kq2.p, nd, 0x7C3B1A9E5D2F4681ull, true, C.stream);
-    const int nparts = 8 * ((C.split.s64.plan.ntiles() + 7) / 8);
+    const int nparts = C.split.s64.plan.blocks();
     double* dots = C.red.part(tt::PB_DOTS);
     tt::launch_fill(dots, 0.0, 2 * nparts, true, C.stream);
     tt::launch_fill(dots, 1.0, 1, true, C.stream);

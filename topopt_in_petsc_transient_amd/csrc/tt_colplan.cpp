@@ -11,11 +11,16 @@ namespace tt {
 // us per plane with 1, 2, 3 blocks per CU): FP32 0.96, 1.19, 1.6; FP64 1.27, 1.87, and no third block (registers).  The
 // columns of a tile (cx x cy <= 256 threads, one halo row and column) and the planes per block trade halo work
 // against blocks in flight: the split with the least modelled time is taken.
+// Grids of up to kBoxNodes nodes take the one-shot kernel: at 1,377 nodes (16x8x8) an FP64 apply takes 3.5 us there against
+// 5.6 us in columns, at 30,625 (48x24x24) 4.5 against 5.8 (flexible-CG apply 6.8 against 8.5, FP32 3.8 against 5.0); at
+// 70,785 (64x32x32) 6.9 against 7.1, and the flexible-CG apply 13.4 against 10.1.
+constexpr long kBoxNodes = 40000;
 ColPlan make_col_plan(const Grid& g, bool fp64) {
     constexpr double cus = 256.0;
     const int resident = fp64 ? 2 : 3;                // blocks per CU
     const double lat = fp64 ? 1.27 : 1.0, iss = fp64 ? 0.93 : 0.54;  // us per plane: alone; per block sharing the CU
     auto plane = [&](int r) { return std::max(lat, iss * r); };
+    if (g.nn <= kBoxNodes) return ColPlan{0, 4, 4, (g.nx + 3) / 4, (g.ny + 3) / 4, (g.nz + 3) / 4};
     ColPlan best{};
     double cost = 1e300;
     for (int cx = std::min(3, g.nx + 1); cx <= std::min(64, g.nx + 1); cx++) {
@@ -79,6 +84,7 @@ void ColSplitStore::build(const Grid& g, const std::vector<uint8_t>& mask) {
     for (int d = 0; d < 2; d++) {
         ColSplit& s = d ? s64 : s32;
         s.plan = make_col_plan(g, d != 0);
+        if (s.plan.cx == 0) continue;  // (the one-shot kernel reads the mask itself)
         std::vector<uint8_t> f;
         col_bc_flags(g, s.plan, mask, f);
         flags[d].alloc(f.size());

@@ -110,11 +110,14 @@ void hex8_modes(const double* ke, const double* m8, ModeConst<double>& mc);
 // the same in device memory, in both precisions
 void upload_modes(const double* ke, const double* m8, DBuf<ModeConst<double>>& d64, DBuf<ModeConst<float>>& d32);
 // The tile split of one grid for the column kernels (tt_apply_cols.inc): columns of elements per tile row
-// (bx + 1) and owned node columns per tile in x and y; tiles (the nz node planes are split evenly over tz).
+// (bx + 1) and owned node columns per tile in x and y; tiles (the nz node planes are split evenly over tz).  cx = 0: a
+// small grid, for the one-shot kernel (tt_apply_box.inc), whose tiles are 4 x 4 x 4 nodes.
 struct ColPlan {
     int cx, bx, by;
     int tx, ty, tz;
     int ntiles() const { return tx * ty * tz; }
+    // blocks of a launch (column kernel: rounded up to a multiple of 8 for the XCD-aware tile order)
+    int blocks() const { return cx ? 8 * ((ntiles() + 7) / 8) : ntiles(); }
 };
 ColPlan make_col_plan(const Grid& g, bool fp64);
 // Per tile of a split: 1 if the tile's staged node box (one halo layer) holds a node with a nonzero mask.

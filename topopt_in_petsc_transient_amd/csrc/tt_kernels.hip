@@ -254,6 +254,7 @@ struct StageThree {  // wK = sum_i cK_i in_i, wM = sum_i cM_i in_i (FP64)
 };
 
 #include "tt_apply_cols.inc"
+#include "tt_apply_box.inc"
 
 // ---- epilogues.  A node's three dofs are b + i .. b + i + 2, b uniform over the block (its node plane's first dof, or
 // 0).  fetch() loads the per-node operands an epilogue reads (its Pre) for one owned node, ahead of the element
@@ -574,10 +575,11 @@ struct EpiRHS {  // R = N.(fs F + yK + yM)
 // the solve is frozen, when gamma_old may be 0.  (One block for it alone took 4.4 us per iteration; summing ~500
 // partials in every block hides behind the other blocks' work.)
 __device__ __forceinline__ double fcg_beta(const double* part, int nblk, double* scal, int first) {
+    const double done = scal[SC_DONE], al = scal[SC_ALPHA], old = scal[SC_GAMMA_OLD];  // (in flight with the partials)
     double d[2];
     sum_partials<2>(part, nblk, d);
     if (blockIdx.x == 0 && threadIdx.x == 0) scal[SC_GAMMA] = d[0];
-    return (first || scal[SC_DONE] != 0.0) ? 0.0 : -scal[SC_ALPHA] * d[1] / scal[SC_GAMMA_OLD];
+    return (first || done != 0.0) ? 0.0 : -al * d[1] / old;
 }
 
 // Flexible-CG direction and its product, with z staged (A z from the contraction): p = z + beta p_old,
@@ -630,8 +632,15 @@ template <typename T, typename CT, bool MASKIN, class Stage, class Epi>
 static int launch_cols_ct(const OpLevel& L, double cK, double cM, const Stage& st, const Epi& epi, hipStream_t s) {
     const ColSplit& cs = sizeof(T) == 8 ? L.split64 : L.split32;
     const ColPlan& p = cs.plan;
+    const ModeConst<T>* mc = sizeof(T) == 8 ? (const ModeConst<T>*)L.modes64 : (const ModeConst<T>*)L.modes32;
+    if (p.cx == 0) {  // a small grid
+        const int tx = (L.g.nx + 3) / 4, ty = (L.g.ny + 3) / 4, tz = (L.g.nz + 3) / 4;
+        hipLaunchKernelGGL((k_apply_box<T, CT, MASKIN, Stage, Epi>), dim3(tx * ty * tz), dim3(128), 0, s, gargs(L.g), tx,
+                           ty, mc, (const CT*)L.kf, (const CT*)L.mf, (T)cK, (T)cM, L.mask, st, epi);
+        TT_HIP(hipGetLastError());
+        return tx * ty * tz;
+    }
     const int nb = 8 * ((p.ntiles() + 7) / 8);
-    const ModeConst<T>* mc = std::is_same<T, double>::value ? (const ModeConst<T>*)L.modes64 : (const ModeConst<T>*)L.modes32;
     hipLaunchKernelGGL((k_apply_cols<T, CT, MASKIN, Stage, Epi>), dim3(nb), dim3(256), 0, s, gargs(L.g), p, mc,
                        (const CT*)L.kf, (const CT*)L.mf, (T)cK, (T)cM, L.mask, cs.bc, st, epi);
     TT_HIP(hipGetLastError());
@@ -649,8 +658,8 @@ static int run_apply(const OpLevel& L, double cK, double cM, const Stage& st, co
 
 // the blocks of an apply launch on this level must fit the reducer's partial regions
 static inline void check_partials(const OpLevel& L, const Reducer& red) {
-    const int nt = std::max(L.split64.plan.ntiles(), L.split32.plan.ntiles());
-    TT_CHECK(8 * ((nt + 7) / 8) <= red.maxblocks, -3, "reducer too small");
+    const int nt = std::max(L.split64.plan.blocks(), L.split32.plan.blocks());
+    TT_CHECK(nt <= red.maxblocks, -3, "reducer too small");
 }
 
 void launch_apply_bc(const OpLevel& L, double cK, double cM, const void* u, void* y, bool fp64, hipStream_t s,
@@ -1002,38 +1011,57 @@ struct ProlongChain {
     int nx[7], ny[7];
     int n;
 };
+// adds level l's correction at fine nodes (i, j, k) and (i + 1, j, k), i even: both lie in one cell of every coarser level
 template <typename Tf, typename Tx>
 __device__ __forceinline__ void prolong_level(const Tx* __restrict__ x, int nx, int ny, int l, int i, int j, int k,
-                                              Tf (&s)[3]) {
+                                              Tf (&s0)[3], Tf (&s1)[3]) {
     const Tf inv = (Tf)1 / (Tf)(1 << l);
     const int fi = i & ((1 << l) - 1), fj = j & ((1 << l) - 1), fk = k & ((1 << l) - 1);
-    const Tf wi = (Tf)fi * inv, wj = (Tf)fj * inv, wk = (Tf)fk * inv;
-    const int di = fi ? 3 : 0, dj = fj ? 3 * nx : 0, dk = fk ? 3 * nx * ny : 0;
+    const Tf w0 = (Tf)fi * inv, w1 = (Tf)(fi + 1) * inv, wj = (Tf)fj * inv, wk = (Tf)fk * inv;
+    const int di = (i >> l) + 1 < nx ? 3 : 0, dj = fj ? 3 * nx : 0, dk = fk ? 3 * nx * ny : 0;
     const Tx* p = x + 3 * ((size_t)(i >> l) + (size_t)nx * ((j >> l) + (size_t)ny * (k >> l)));
+    Tf a[3] = {0, 0, 0}, b[3] = {0, 0, 0};  // the cell's low-x and high-x edges at (j, k)
 #pragma unroll
-    for (int q = 0; q < 8; q++) {
-        const Tf w = ((q & 1) ? wi : (Tf)1 - wi) * ((q & 2) ? wj : (Tf)1 - wj) * ((q & 4) ? wk : (Tf)1 - wk);
-        const Tx* pq = p + ((q & 1) ? di : 0) + ((q & 2) ? dj : 0) + ((q & 4) ? dk : 0);
+    for (int q = 0; q < 4; q++) {
+        const Tf w = ((q & 1) ? wj : (Tf)1 - wj) * ((q & 2) ? wk : (Tf)1 - wk);
+        const Tx* pq = p + ((q & 1) ? dj : 0) + ((q & 2) ? dk : 0);
 #pragma unroll
-        for (int c = 0; c < 3; c++) s[c] = fma(w, (Tf)pq[c], s[c]);
+        for (int c = 0; c < 3; c++) {
+            a[c] = fma(w, (Tf)pq[c], a[c]);
+            b[c] = fma(w, (Tf)pq[di + c], b[c]);
+        }
+    }
+#pragma unroll
+    for (int c = 0; c < 3; c++) {
+        s0[c] = fma((Tf)1 - w0, a[c], fma(w0, b[c], s0[c]));
+        s1[c] = fma((Tf)1 - w1, a[c], fma(w1, b[c], s1[c]));
     }
 }
-template <typename Tf, typename Tl>  // Tl: the last (coarsest) level's type
+template <typename Tf, typename Tl>  // Tl: the last (coarsest) level's type; one thread per pair of nodes in x
 __global__ void k_prolong_chain(GridArgs f, ProlongChain pc, const uint8_t* __restrict__ fmask, Tf* __restrict__ xf) {
-    const long n = blockIdx.x * (long)blockDim.x + threadIdx.x;
-    if (n >= (long)f.nx * f.ny * f.nz) return;
+    const unsigned px = (unsigned)(f.nx + 1) >> 1;
+    const long t = blockIdx.x * (long)blockDim.x + threadIdx.x;
+    if (t >= (long)px * f.ny * f.nz) return;
     int i, j, k;
-    grid_ijk((unsigned)n, f.nx, f.ny, i, j, k);
-    const uint8_t cl = fmask[n];
-    Tf x[3], s[3] = {0, 0, 0};
+    grid_ijk((unsigned)t, px, f.ny, i, j, k);
+    i *= 2;
+    const long n = i + (long)f.nx * (j + (long)f.ny * k);
+    const bool two = i + 1 < f.nx;
+    const uint8_t cl0 = fmask[n], cl1 = two ? fmask[n + 1] : (uint8_t)7;
+    Tf x[6], s0[3] = {0, 0, 0}, s1[3] = {0, 0, 0};
 #pragma unroll
     for (int c = 0; c < 3; c++) x[c] = xf[3 * n + c];
-    for (int l = 0; l + 1 < pc.n; l++)
-        prolong_level<Tf, Tf>((const Tf*)pc.x[l], pc.nx[l], pc.ny[l], l + 1, i, j, k, s);
-    prolong_level<Tf, Tl>((const Tl*)pc.x[pc.n - 1], pc.nx[pc.n - 1], pc.ny[pc.n - 1], pc.n, i, j, k, s);
+    if (two)
 #pragma unroll
-    for (int c = 0; c < 3; c++)
-        if (!((cl >> c) & 1)) xf[3 * n + c] = x[c] + s[c];
+        for (int c = 3; c < 6; c++) x[c] = xf[3 * n + c];
+    for (int l = 0; l + 1 < pc.n; l++)
+        prolong_level<Tf, Tf>((const Tf*)pc.x[l], pc.nx[l], pc.ny[l], l + 1, i, j, k, s0, s1);
+    prolong_level<Tf, Tl>((const Tl*)pc.x[pc.n - 1], pc.nx[pc.n - 1], pc.ny[pc.n - 1], pc.n, i, j, k, s0, s1);
+#pragma unroll
+    for (int c = 0; c < 3; c++) {
+        if (!((cl0 >> c) & 1)) xf[3 * n + c] = x[c] + s0[c];
+        if (!((cl1 >> c) & 1)) xf[3 * n + 3 + c] = x[3 + c] + s1[c];
+    }
 }
 void launch_prolong_chain(const Grid& fine, int n, const Grid* const* coarse, const void* const* xc,
                           const uint8_t* fmask, void* xf, bool fp64, bool last64, hipStream_t s) {
@@ -1045,7 +1073,7 @@ void launch_prolong_chain(const Grid& fine, int n, const Grid* const* coarse, co
         pc.nx[l] = coarse[l]->nx;
         pc.ny[l] = coarse[l]->ny;
     }
-    const dim3 gr(nblocks(fine.nn)), bl(BS);
+    const dim3 gr(nblocks((long)((fine.nx + 1) / 2) * fine.ny * fine.nz)), bl(BS);
     if (fp64)
         hipLaunchKernelGGL((k_prolong_chain<double, double>), gr, bl, 0, s, gargs(fine), pc, fmask, (double*)xf);
     else if (last64)
@@ -1636,11 +1664,12 @@ __global__ __launch_bounds__(BS) void k_fcg_update(double* __restrict__ x, const
         r0 = r[i0];
         q0 = q[i0];
     }
+    const double s_zero = scal[SC_ZERO], s_done = scal[SC_DONE], tol2 = scal[SC_TOL2], gam = scal[SC_GAMMA];
     double pq[1], rr[1] = {0.0};
     sum_partials<1>(pq_part, pq_nblk, pq);
     if (!first) sum_partials<1>(rr_old, rr_nblk, rr);
-    const bool zero = scal[SC_ZERO] != 0.0, done = scal[SC_DONE] != 0.0 || (!first && rr[0] <= scal[SC_TOL2]);
-    const double gam = scal[SC_GAMMA], al = done ? 0.0 : gam / pq[0];
+    const bool zero = s_zero != 0.0, done = s_done != 0.0 || (!first && rr[0] <= tol2);
+    const double al = done ? 0.0 : gam / pq[0];
     constexpr int NA = JAC ? 3 : 1;
     double acc[NA];
 #pragma unroll
