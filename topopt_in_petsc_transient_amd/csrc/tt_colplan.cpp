@@ -7,27 +7,34 @@
 namespace tt {
 
 // Tile split of one grid.  A block's planes pass one after the other, so its time is (planes + 2) times the time of a
-// plane, which is bound by latency while few blocks share a CU and by issue beyond.  Measured on 128x64x64 (256 CUs;
-// us per plane with 1, 2, 3 blocks per CU): FP32 0.96, 1.19, 1.6; FP64 1.27, 1.87, and no third block (registers).  The
-// columns of a tile (cx x cy <= 256 threads, one halo row and column) and the planes per block trade halo work
-// against blocks in flight: the split with the least modelled time is taken.
+// plane: a latency that grows slowly with the blocks sharing a CU, plus the cache lines the tile's rows touch (a narrow
+// tile reads more halo).  The constants are fitted to 170 splits on each of 8 grids between 97x51x43 and 320x160x160
+// elements (FP64 to the plain and the flexible-CG apply alike; rms error 6 and 9 %).  The columns of a tile (cx x cy <=
+// 256 threads, one halo row and column) and the planes per block trade halo work against blocks in flight: the split
+// with the least modelled time is taken.  Against a model with a plane bound by issue alone (FP64 apply, FP32 apply,
+// flexible-CG apply; us): 192x96x96 40.6 -> 39.4, 26.7 -> 22.6, 62 -> 57; 320x160x160 171 -> 163, 95 -> 78, 305 -> 283;
+// 40x40x300 17.7 -> 17.1, 12.3 -> 11.3, 23.4 -> 22.2; 128x64x64 and smaller as they were.
 // Grids of up to kBoxNodes nodes take the one-shot kernel: at 1,377 nodes (16x8x8) an FP64 apply takes 3.5 us there against
 // 5.6 us in columns, at 30,625 (48x24x24) 4.5 against 5.8 (flexible-CG apply 6.8 against 8.5, FP32 3.8 against 5.0); at
 // 70,785 (64x32x32) 6.9 against 7.1, and the flexible-CG apply 13.4 against 10.1.
 constexpr long kBoxNodes = 40000;
 ColPlan make_col_plan(const Grid& g, bool fp64) {
     constexpr double cus = 256.0;
-    const int resident = fp64 ? 2 : 3;                // blocks per CU
-    const double lat = fp64 ? 1.27 : 1.0, iss = fp64 ? 0.93 : 0.54;  // us per plane: alone; per block sharing the CU
-    auto plane = [&](int r) { return std::max(lat, iss * r); };
+    const int resident = fp64 ? 2 : 3;  // blocks per CU
+    // us per plane with r blocks on the CU, and per r and 100 lines of 128 bytes touched
+    const double base[3] = {fp64 ? 1.4 : 0.83, fp64 ? 1.95 : 1.03, 1.25}, lines = fp64 ? 0.17 : 0.013;
+    const double tail = fp64 ? 0.3 : 0.35;  // of a full CU's plane: blocks of the last round left alone
     if (g.nn <= kBoxNodes) return ColPlan{0, 4, 4, (g.nx + 3) / 4, (g.ny + 3) / 4, (g.nz + 3) / 4};
     ColPlan best{};
     double cost = 1e300;
-    for (int cx = std::min(3, g.nx + 1); cx <= std::min(64, g.nx + 1); cx++) {
+    for (int cx = std::min(3, g.nx + 1); cx <= std::min(34, g.nx + 1); cx++) {
         const int bx = cx - 1, tx = (g.nx + bx - 1) / bx;
         const int cymax = std::min({256 / cx, 1024 / (3 * (cx + 1)) - 1, g.ny + 1});
         for (int cy = std::min(3, cymax); cy <= cymax; cy++) {
             const int by = cy - 1, ty = (g.ny + by - 1) / by;
+            const double row = (std::min(cx, g.nx) + 1) * 3.0 * (fp64 ? 8 : 4) / 128.0 + 1.0;
+            const double touched = lines * row * (std::min(cy, g.ny) + 1) / 100.0;
+            auto plane = [&](int r) { return base[r - 1] + r * touched; };
             for (int nk = 1, last = 0; nk <= g.nz; nk++) {
                 const int tz = (g.nz + nk - 1) / nk;
                 if (tz == last) continue;
@@ -35,8 +42,7 @@ ColPlan make_col_plan(const Grid& g, bool fp64) {
                 const double nt = (double)tx * ty * tz, per = nt / cus;
                 const int r = (int)std::ceil(per);
                 // (between splits of one modelled time, the one with fewer blocks)
-                const double c = 1e-4 * nt + (r <= resident ? (nk + 2) * plane(r)
-                                                            : (nk + 2) * plane(resident) * (0.5 + per / resident));
+                const double c = 1e-4 * nt + (nk + 2) * (r <= resident ? plane(r) : plane(resident) * (tail + per / resident));
                 if (c < cost) {
                     cost = c;
                     best = ColPlan{cx, bx, by, tx, ty, tz};
