@@ -78,7 +78,7 @@ struct Multigrid {
 
    private:
     void vcycle(int l, const double* r64 = nullptr, double* z64 = nullptr, const double* q64 = nullptr,
-                bool first = false);
+                bool first = false, const double* b_in = nullptr, double* x_out = nullptr);
     void coarse_solve(bool direct64);
     double power_lmax(int l, int iters);
     void assemble_coarse_inverse();
