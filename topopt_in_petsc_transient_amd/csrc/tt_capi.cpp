@@ -143,7 +143,7 @@ Context::Context(const tt_params& p) : prm(p) {
         b->alloc(nd);
     TT_HIP(hipMemsetAsync(lamT.p, 0, nd * 8, stream));
     TT_HIP(hipMemsetAsync(nu0.p, 0, nd * 8, stream));
-    fxs.alloc((size_t)(p.nsteps + 1) * ((nel + 255) / 256));  // per-step objective partials
+    fxs.alloc((size_t)(p.nsteps + 1) * sens_blocks(g));  // per-step objective partials
 
     // state storage: every state, or s binomial slots + the t = 0 state
     const int T = p.nsteps;

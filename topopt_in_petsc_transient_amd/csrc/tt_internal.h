@@ -379,11 +379,10 @@ void launch_adjoint0_rhs(const double* Kl, const double* Ml, const double* hdddu
 void launch_hdiag(const double* w, const double* cnt, double dt, double* h, long nn, hipStream_t s);
 void launch_region_count(const Grid& g, const double* P, double* cnt, hipStream_t s);
 
-// sensitivities and objective (per time step); accumulates into df and red.scal[slot] (objective)
+// sensitivities and objective (per time step); accumulates into df, objective partials per block
 struct SensArgs {
     Grid g;
-    const double* KE;  // 576
-    const double* M8;  // 64
+    const ModeConst<double>* modes;
     const double *kf, *mf, *dkf, *dmf, *P;
     const double *lam, *u, *v, *a, *ub, *vb, *ab;
     double wK[4];  // coefficients of (u, ub, vb, ab) in w_K
@@ -393,7 +392,8 @@ struct SensArgs {
     int mode;      // 0: general step (lambda), 1: t = 0 step (nu0 with dK u0 + dC v0 + dM a0)
     double* df;
 };
-void launch_sens(const SensArgs& a, Reducer& red, double* fx_out, hipStream_t s);
+long sens_blocks(const Grid& g);  // objective partials written to fx_out
+void launch_sens(const SensArgs& a, double* fx_out, hipStream_t s);
 
 // PDE filter (scalar Helmholtz on nodes)
 // The filter's operator R^2 (Kx My Mz + Mx Ky Mz + Mx My Kz) + Mx My Mz by its 1-D factors.

@@ -255,6 +255,7 @@ struct StageThree {  // wK = sum_i cK_i in_i, wM = sum_i cM_i in_i (FP64)
 
 #include "tt_apply_cols.inc"
 #include "tt_apply_box.inc"
+#include "tt_sens.inc"
 
 // ---- epilogues.  A node's three dofs are b + i .. b + i + 2, b uniform over the block (its node plane's first dof, or
 // 0).  fetch() loads the per-node operands an epilogue reads (its Pre) for one owned node, ahead of the element

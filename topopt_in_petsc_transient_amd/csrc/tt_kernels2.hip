@@ -1,5 +1,4 @@
-// HIP kernels for gfx950: element sensitivities and objective, PDE (Helmholtz)
-// filter, Heaviside projection, and the element-wise parts of MMA.
+// HIP kernels for gfx950: transfers of the PDE (Helmholtz) filter, Heaviside projection, and the element-wise parts of MMA.
 #include "../../include/topopt_gpu.h"
 #include "tt_internal.h"
 
@@ -73,174 +72,6 @@ __device__ __forceinline__ void elem_nodes(const GA& g, long e, long (&nd)[8]) {
     nd[5] = n0 + 1 + sz;
     nd[6] = n0 + 1 + sy + sz;
     nd[7] = n0 + sy + sz;
-}
-
-// ------------------------------------------------------------------ sensitivities
-// Per element and time step (ComputeSensitivitiesElementLoopn, LinearElasticity.cc:1911-2077):
-//   df_e += P_e*dfx0 + lambda_e^T (dA u_t + dB1 u_{t-1} + dB2 v_{t-1} + dB3 a_{t-1})
-// which factorises into dkfac * lambda^T KE w_K + dmfac * lambda^T ME w_M with
-// w_K, w_M linear combinations of (u_t, u_{t-1}, v_{t-1}, a_{t-1}) given by wK/wM.
-// mode 1 is the t = 0 loop (ComputeSensitivitiesElementLoop0, :2080-2204) with
-// the slots (u0, v0, a0): w_K = u0 + dbeta v0, w_M = dalpha v0 + a0.
-struct SensDev {
-    GA g;
-    const double* KE;
-    const double* M8;
-    const double *kf, *mf, *dkf, *dmf, *P;
-    const double *lam, *u, *v, *a, *s1, *s2, *s3;
-    double wK[4], wM[4];
-    double dt, al, be;
-    int objective;
-    double* df;
-};
-
-// On the matrix cores (v_mfma_f64_16x16x4f64).  A wave takes batches of 16
-// consecutive elements, one per MFMA column, and forms per batch
-//     KE w_K and ME w_M, plus the objective's element products: KE u (objectives 3, 5), ME v (4-6),
-//     KE v (6)   (each: 2 row tiles x 6 k-steps of 24 x 24 by 24 x 16).
-// The element's 24 dofs are taken in the order sens_dof(k): lane group q owns the two x-adjacent
-// corners of one element edge (corners 0-1, 3-2, 4-5, 7-6), whose 6 dofs are consecutive in memory
-// (3 wide loads per vector instead of 6 scattered ones), as k = 4 t + q, t = 0..5.  Operand layout:
-// lane j + 16 q holds the B value of k row q of k-step t, i.e. sens_dof(4 t + q) of element j, and
-// receives D rows 4 v + q of each row tile (measured on gfx950), i.e. k = 16 R + 4 v + q: the same
-// six dofs.  The A fragments hold KE and ME with rows and columns in the same order, so every lane
-// loads just its six values of each input vector, and lambda^T KE w_K, lambda^T ME w_M and the
-// objective's quadratic forms (u^T u, v^T v, a^T a for objectives 0-2) are sums over the four lane
-// groups (two shuffles, in a fixed order).  The element matrices stay in registers as A fragments.
-// Measured at 128x64x64 (objective 3): 72 us per launch (148 VGPRs, 3 waves per SIMD), against 82 us
-// (204 VGPRs) with the dofs = q (mod 4) in lane group q, which takes 6 scattered 8-byte loads per vector,
-// and 64-bit element index arithmetic (75 us with the contiguous loads alone).  sens_dof is in
-// tt_internal.h.
-typedef double sens_d4 __attribute__((ext_vector_type(4)));
-__device__ __forceinline__ double lane_group_sum(double x) {
-    x += __shfl_xor(x, 16, 64);
-    return x + __shfl_xor(x, 32, 64);
-}
-template <int OBJ>
-__global__ __launch_bounds__(256) void k_sens_mfma(SensDev s, double* partials) {
-    constexpr bool KU = OBJ == 3 || OBJ == 5, MV = OBJ >= 4, KV = OBJ == 6;
-    constexpr bool LV = OBJ == 1 || OBJ >= 4, LA = OBJ == 2;  // v or a of state t needed
-    const int lane = threadIdx.x & 63, j = lane & 15, q = lane >> 4, wave = threadIdx.x >> 6;
-    const long nel = (long)s.g.ex * s.g.ey * s.g.ez;
-    // A fragments: lane j + 16 q holds row j, k column q of each 16 x 4 block (rows 24..31 zero)
-    double aK[2][6], aM[2][6];
-#pragma unroll
-    for (int R = 0; R < 2; R++)
-#pragma unroll
-        for (int t = 0; t < 6; t++) {
-            const int r = 16 * R + j, rd = sens_dof(r < 24 ? r : 23), cd = sens_dof(4 * t + q);
-            const double k = s.KE[rd * 24 + cd], m = s.M8[(rd / 3) * 8 + cd / 3];
-            aK[R][t] = r < 24 ? k : 0.0;
-            aM[R][t] = (r < 24 && rd % 3 == cd % 3) ? m : 0.0;
-        }
-    const long sy = s.g.nx, sz = (long)s.g.nx * s.g.ny;
-    const double hdt = 0.5 * s.dt;
-    double h[1] = {0.0};
-#pragma unroll 1
-    for (int b = 0; b < 4; b++) {
-        const long e = (long)blockIdx.x * 256 + (wave * 4 + b) * 16 + j;
-        const bool valid = e < nel;
-        const long ec = valid ? e : nel - 1;
-        // element -> (i, jj, kk) in 32-bit unsigned arithmetic (two divisions; element and node
-        // indices fit in 32 bits, as everywhere in the apply kernels)
-        const unsigned eu = (unsigned)ec, exu = (unsigned)s.g.ex, eyu = (unsigned)s.g.ey;
-        const unsigned row = eu / exu, kk = row / eyu, i = eu - row * exu, jj = row - kk * eyu;
-        const long n0 = (long)i + sy * (long)jj + sz * (long)kk;
-        // the low-x node of the lane group's edge: dofs sens_dof(4 t + q), t = 0..5, at x0 + t
-        const long x0 = 3 * (n0 + sy * (q & 1) + sz * (q >> 1));
-        double lam[6], u[6], wk[6], wm[6], w2[6];
-#pragma unroll
-        for (int t = 0; t < 6; t++) {
-            const long x = x0 + t;
-            const double uu = s.u[x], x1 = s.s1[x], x2 = s.s2[x], x3 = s.s3[x];
-            lam[t] = s.lam[x];
-            u[t] = uu;
-            wk[t] = fma(s.wK[3], x3, fma(s.wK[2], x2, fma(s.wK[1], x1, s.wK[0] * uu)));
-            wm[t] = fma(s.wM[3], x3, fma(s.wM[2], x2, fma(s.wM[1], x1, s.wM[0] * uu)));
-            w2[t] = LV ? s.v[x] : LA ? s.a[x] : 0.0;  // the state-t vector of the objective
-        }
-        sens_d4 accK[2], accM[2], accU[2], accVM[2], accVK[2];
-#pragma unroll
-        for (int R = 0; R < 2; R++) accK[R] = accM[R] = accU[R] = accVM[R] = accVK[R] = sens_d4{0.0, 0.0, 0.0, 0.0};
-#pragma unroll
-        for (int t = 0; t < 6; t++)
-#pragma unroll
-            for (int R = 0; R < 2; R++) {
-                accK[R] = __builtin_amdgcn_mfma_f64_16x16x4f64(aK[R][t], wk[t], accK[R], 0, 0, 0);
-                accM[R] = __builtin_amdgcn_mfma_f64_16x16x4f64(aM[R][t], wm[t], accM[R], 0, 0, 0);
-                if (KU) accU[R] = __builtin_amdgcn_mfma_f64_16x16x4f64(aK[R][t], u[t], accU[R], 0, 0, 0);
-                if (MV) accVM[R] = __builtin_amdgcn_mfma_f64_16x16x4f64(aM[R][t], w2[t], accVM[R], 0, 0, 0);
-                if (KV) accVK[R] = __builtin_amdgcn_mfma_f64_16x16x4f64(aK[R][t], w2[t], accVK[R], 0, 0, 0);
-            }
-        // D row 4 v + q of row tile R is k = 4 (4 R + v) + q: the lane's value t = 4 R + v (t < 6)
-        double tK = 0.0, tM = 0.0, fU = 0.0, fVM = 0.0, fVK = 0.0;
-#pragma unroll
-        for (int t = 0; t < 6; t++) {
-            const int R = t >> 2, v = t & 3;
-            tK = fma(accK[R][v], lam[t], tK);
-            tM = fma(accM[R][v], lam[t], tM);
-            if (KU) fU = fma(accU[R][v], u[t], fU);
-            if (OBJ == 0) fU = fma(u[t], u[t], fU);
-            if (OBJ == 1 || OBJ == 2) fU = fma(w2[t], w2[t], fU);
-            if (MV) fVM = fma(accVM[R][v], w2[t], fVM);
-            if (KV) fVK = fma(accVK[R][v], w2[t], fVK);
-        }
-        tK = lane_group_sum(tK);
-        tM = lane_group_sum(tM);
-        fU = lane_group_sum(fU);
-        if (MV) fVM = lane_group_sum(fVM);
-        if (KV) fVK = lane_group_sum(fVK);
-        if (valid && q == 0) {
-            const double dkf = s.dkf[e], dmf = s.dmf[e], kf = s.kf[e], mf = s.mf[e], P = s.P[e];
-            // objective terms of state t (EvaluateObjective / EvaluateObjectiveGradient, :1416-1514)
-            double h0 = 0.0, dfx0 = 0.0;
-            if (OBJ <= 2) h0 = hdt * fU;
-            if (OBJ == 3) { h0 = hdt * (kf * fU); dfx0 = hdt * (dkf * fU); }
-            if (OBJ == 4) { h0 = hdt * (mf * fVM); dfx0 = hdt * (dmf * fVM); }
-            if (OBJ == 5) { h0 = hdt * (kf * fU + mf * fVM); dfx0 = hdt * (dkf * fU + dmf * fVM); }
-            if (OBJ == 6) {
-                h0 = hdt * (s.al * mf * fVM + s.be * kf * fVK);
-                dfx0 = hdt * (s.al * dmf * fVM + s.be * dkf * fVK);
-            }
-            s.df[e] += P * dfx0 + (dkf * tK + dmf * tM);
-            h[0] += h0 * P;
-        }
-    }
-    rfinish<1>(h, partials, nullptr, nullptr);
-}
-
-void launch_sens(const SensArgs& a, Reducer& red, double* fx_out, hipStream_t st) {
-    SensDev s;
-    s.g = ga(a.g);
-    s.KE = a.KE;
-    s.M8 = a.M8;
-    s.kf = a.kf; s.mf = a.mf; s.dkf = a.dkf; s.dmf = a.dmf; s.P = a.P;
-    s.lam = a.lam;
-    s.v = a.v;
-    s.a = a.a;
-    s.dt = a.dt; s.al = a.dalpha; s.be = a.dbeta;
-    s.objective = a.objective;
-    s.df = a.df;
-    if (a.mode == 0) {
-        s.u = a.u; s.s1 = a.ub; s.s2 = a.vb; s.s3 = a.ab;
-    } else {
-        s.u = a.u; s.s1 = a.v; s.s2 = a.a; s.s3 = a.a;
-    }
-    for (int k = 0; k < 4; k++) { s.wK[k] = a.wK[k]; s.wM[k] = a.wM[k]; }
-    // fx_out receives one partial objective value per block (nblk(nel) of them)
-    const int nb = nblk(a.g.nel);
-    (void)red;
-    static_assert(BS2 == 256, "k_sens_mfma: one block per 256 elements");
-    switch (a.objective) {
-    case 0: hipLaunchKernelGGL(k_sens_mfma<0>, dim3(nb), dim3(256), 0, st, s, fx_out); break;
-    case 1: hipLaunchKernelGGL(k_sens_mfma<1>, dim3(nb), dim3(256), 0, st, s, fx_out); break;
-    case 2: hipLaunchKernelGGL(k_sens_mfma<2>, dim3(nb), dim3(256), 0, st, s, fx_out); break;
-    case 3: hipLaunchKernelGGL(k_sens_mfma<3>, dim3(nb), dim3(256), 0, st, s, fx_out); break;
-    case 4: hipLaunchKernelGGL(k_sens_mfma<4>, dim3(nb), dim3(256), 0, st, s, fx_out); break;
-    case 5: hipLaunchKernelGGL(k_sens_mfma<5>, dim3(nb), dim3(256), 0, st, s, fx_out); break;
-    default: hipLaunchKernelGGL(k_sens_mfma<6>, dim3(nb), dim3(256), 0, st, s, fx_out); break;
-    }
-    TT_HIP(hipGetLastError());
 }
 
 // ------------------------------------------------------------------ PDE filter (PDEFilter.cc)

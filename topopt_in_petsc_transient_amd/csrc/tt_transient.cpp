@@ -357,7 +357,7 @@ void Context::objective_gradient(double* fx_host, double* dfdx_dev) {
     const double al = prm.dalpha, be = prm.dbeta;
     const int obj = prm.objective;
     const double coef[8] = {a[0], a[1], a[2], a[3], a[4], a[5], al, be};
-    const long nbs = (g.nel + 255) / 256;  // objective partials per time step (one per sensitivity block)
+    const long nbs = sens_blocks(g);  // objective partials per time step
     launch_fill(df.p, 0.0, g.nel, true, stream);
     launch_fill(hdu.p, 0.0, nd, true, stream);
     launch_fill(hddu.p, 0.0, nd, true, stream);
@@ -387,8 +387,7 @@ void Context::objective_gradient(double* fx_host, double* dfdx_dev) {
     auto sens = [&](int mode, const double* lamv, const double* st, const double* stb, int t) {
         SensArgs sa;
         sa.g = g;
-        sa.KE = KE64d.p;
-        sa.M8 = M864d.p;
+        sa.modes = modes64.p;
         sa.kf = kf.p; sa.mf = mf.p; sa.dkf = dkf.p; sa.dmf = dmf.p; sa.P = P.p;
         sa.lam = lamv;
         sa.u = st; sa.v = st + nd; sa.a = st + 2 * nd;
@@ -410,7 +409,7 @@ void Context::objective_gradient(double* fx_host, double* dfdx_dev) {
         sa.objective = obj;
         sa.mode = mode;
         sa.df = df.p;
-        launch_sens(sa, red, fxs.p + (size_t)t * nbs, stream);
+        launch_sens(sa, fxs.p + (size_t)t * nbs, stream);
     };
 
     // one backward step at t: needs state t and state t-1
