@@ -40,7 +40,8 @@ def test_sensitivities(nel, objective):
     assert rel(df, df_ref) < 1e-8
 
 
-@pytest.mark.parametrize("nel", [(1, 1, 1), (31, 7, 2), (32, 8, 1), (30, 6, 3), (2, 17, 40), (70, 3, 5), (3, 2, 300)])
+@pytest.mark.parametrize("nel", [(1, 1, 1), (31, 7, 2), (32, 8, 1), (30, 6, 3), (2, 17, 40), (70, 3, 5), (3, 2, 300),
+                                 (1, 20000, 1)])
 def test_filter(nel):
     print("filter", nel, flush=True)
     po, pg = problem(*nel, nsteps=2, lx=0.05 * nel[0], ly=0.07 * nel[1], lz=0.04 * nel[2], nlvls=1, rmin=0.11)
@@ -69,6 +70,20 @@ def test_levels_and_coarsest_solve(nel, nlvls, precision):
     c.close()
     assert rel(u, ref[4, 0]) < 1e-8 and rel(v, ref[4, 1]) < 1e-8
     assert iters <= 5 * 40  # the preconditioner works at every depth
+
+
+def test_long_thin_levels():
+    """The coarser grid (1 x 1 x 9,500 elements) has more blocks and reduction partials than the finest."""
+    po, pg = problem(2, 2, 19000, nsteps=2, dt=0.001, pulse_steps=2, nlvls=2, lx=0.2, ly=0.2, lz=1900.0)
+    x = random_density(O.nel(po), seed=12)
+    ref = O.forward(po, x)
+    c = capi.Context(pg)
+    c.set_density(x)
+    c.complete_initial_state()
+    c.forward()
+    u, v, a = c.get_state(2)
+    c.close()
+    assert rel(u, ref[2, 0]) < 1e-8 and rel(v, ref[2, 1]) < 1e-8
 
 
 def test_basis_solves_over_many_krylov_vectors():

@@ -92,9 +92,14 @@ Context::Context(const tt_params& p) : prm(p) {
     mask.alloc(nn);
     TT_HIP(hipMemcpy(mask.p, m.data(), nn, hipMemcpyHostToDevice));
     split.build(g, m);
-    // (an apply writes one partial per block; coarser levels have fewer nodes and no more blocks)
-    const long apply_blocks = std::max(split.s32.plan.blocks(), split.s64.plan.blocks());
-    red.init((int)std::max<long>({apply_blocks, (nel + 255) / 256, (nn + 255) / 256, 2048}));
+    // an apply writes one partial per block, on every level (a long thin coarser grid can have more blocks than the
+    // finest one), and so does the filter's operator
+    long op_blocks = filter_blocks(g);
+    for (int l = 0; l < std::min(p.nlvls, 8) && (p.nelx >> l) && (p.nely >> l) && (p.nelz >> l); l++) {
+        const Grid gl = make_grid(p.nelx >> l, p.nely >> l, p.nelz >> l, 1.0, 1.0, 1.0);
+        for (bool fp64 : {false, true}) op_blocks = std::max<long>(op_blocks, make_col_plan(gl, fp64).blocks());
+    }
+    red.init((int)std::max<long>({op_blocks, (nel + 255) / 256, (nn + 255) / 256, 2048}));
     F.alloc(nd);
     TT_HIP(hipMemcpy(F.p, Fhost.data(), nd * 8, hipMemcpyHostToDevice));
     std::vector<double> Ph(nel);

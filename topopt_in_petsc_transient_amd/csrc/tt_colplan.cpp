@@ -35,10 +35,8 @@ ColPlan make_col_plan(const Grid& g, bool fp64) {
             const double row = (std::min(cx, g.nx) + 1) * 3.0 * (fp64 ? 8 : 4) / 128.0 + 1.0;
             const double touched = lines * row * (std::min(cy, g.ny) + 1) / 100.0;
             auto plane = [&](int r) { return base[r - 1] + r * touched; };
-            for (int nk = 1, last = 0; nk <= g.nz; nk++) {
+            for (int nk = 1;;) {  // planes per block: the fewest that give each number of blocks in z
                 const int tz = (g.nz + nk - 1) / nk;
-                if (tz == last) continue;
-                last = tz;
                 const double nt = (double)tx * ty * tz, per = nt / cus;
                 const int r = (int)std::ceil(per);
                 // (between splits of one modelled time, the one with fewer blocks)
@@ -47,6 +45,8 @@ ColPlan make_col_plan(const Grid& g, bool fp64) {
                     cost = c;
                     best = ColPlan{cx, bx, by, tx, ty, tz};
                 }
+                if (tz == 1) break;
+                nk = (g.nz + tz - 2) / (tz - 1);
             }
         }
     }

@@ -181,7 +181,7 @@ enum {
 // Elasticity operator on one level.  Coefficient storage CT is double, float or BF16.
 enum CoefKind { COEF_F64 = 0, COEF_F32 = 1, COEF_BF16 = 2 };
 
-// Batch tables of the node tiles of one grid (see tt_apply_mfma.inc): per tile position (bits 0/1: the
+// Batch tables of the node tiles of one grid (tt_tables.cpp; the library's kernels do not use them): per tile position (bits 0/1: the
 // first / last tile in x, bits 2/3 in y, bits 4/5 in z) the offset and batch count of its table in
 // `codes`.  A tile's table holds the elements that exist and touch one of its nodes: the first tile in
 // a direction has no elements on its low side, and the last tile owns fewer nodes than a full tile
@@ -196,7 +196,7 @@ __host__ __device__ inline void grid_ijk(unsigned n, unsigned nx, unsigned ny, i
     j = (int)(row - kk * ny);
     k = (int)kk;
 }
-// The sensitivity kernel's element dof order: k = 4 t + q (t = 0..5) is dof 3 a + c of corner
+// Element dof order by edges (no kernel uses it): k = 4 t + q (t = 0..5) is dof 3 a + c of corner
 // a = sens_corner(q, t >= 3), component c = t mod 3.  Lane group q owns the two x-adjacent corners of one
 // element edge (corners 0-1, 3-2, 4-5, 7-6), whose six dofs are consecutive in memory from the edge's
 // low-x node.
@@ -401,6 +401,7 @@ struct FilterOp {
     double h[3], R2;
 };
 // r = rhs - A U, partials of r.r (PB_MISC2), of z.r with z = D^-1 r (PB_DOTS) and, with bb, of rhs.rhs (PB_MISC)
+long filter_blocks(const Grid& g);  // partials written by the two launches below
 void launch_filter_residual(const Grid& g, const FilterOp& f, const double* U, const double* rhs, const double* dinv,
                             double* r, Reducer& red, bool bb, hipStream_t s);
 // Jacobi-preconditioned CG direction and product: p = z + beta p_old with z = D^-1 r, q = A p, partials of p.q

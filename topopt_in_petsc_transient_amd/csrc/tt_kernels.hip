@@ -2,12 +2,11 @@
 // Krylov vector kernels and deterministic reductions.
 //
 // The operator y = sum_e (cK*kfac_e*KE + cM*mfac_e*ME) u_e of the reference's
-// assembled AIJ matrices (LinearElasticity.cc:2502-2619) is applied node by
-// node: each thread owns one node and gathers the contributions of its (up to)
-// eight elements from an LDS tile holding the node box (8x8x4 owned + halo 1)
-// and the element coefficients.  No scatter, no atomics: results are
-// bit-reproducible.  Epilogue functors fuse the Krylov / Chebyshev vector work
-// into the same pass.
+// assembled AIJ matrices (LinearElasticity.cc:2502-2619) is applied element by
+// element in the element's symmetry-adapted basis (tt_apply_cols.inc; small
+// grids tt_apply_box.inc), with the corner values added per node in a fixed
+// order: no atomics, results are bit-reproducible.  Epilogue functors fuse the
+// Krylov / Chebyshev vector work into the same pass.
 #include <algorithm>
 #include <cmath>
 #include <cstring>
@@ -1868,6 +1867,10 @@ __global__ __launch_bounds__(256) void k_filter_op(GridArgs g, FilterOp f, int t
 static inline dim3 filter_tiles(const Grid& g) {
     const int tx = (g.nx + FX - 1) / FX, ty = (g.ny + FY - 1) / FY;
     return dim3(tx, ty, std::min(g.nz, std::max(1, 1024 / (tx * ty))));
+}
+long filter_blocks(const Grid& g) {
+    const dim3 t = filter_tiles(g);
+    return (long)t.x * t.y * t.z;
 }
 void launch_filter_residual(const Grid& g, const FilterOp& f, const double* U, const double* rhs, const double* dinv,
                             double* r, Reducer& red, bool bb, hipStream_t s) {
