@@ -32,17 +32,14 @@ sys.path.insert(0, ROOT)
 METRIC = "Newmark steps/s + adjoint-gradient time, 128x64x64 hex8, mixed vs FP64 GPU"
 PEAK_HBM = 8.0e12          # MI355X HBM3E, B/s
 PEAK_FP64 = 78.6e12        # MI355X dense FP64 (vector and matrix), flop/s
-PEAK_FP32 = 157.3e12       # MI355X dense FP32 matrix, flop/s
-PEAK_FP16 = 2.5e15         # MI355X dense FP16 matrix, flop/s
-# matrix instructions of one FP32 A apply at 128x64x64, as rocprofv3 counts them (SQ_INSTS_MFMA summed
-# over the dispatch): 520,058 v_mfma_f32_16x16x32_f16 of 16,384 flops each (2,601 tiles of 8x8x4 nodes;
-# the tables per tile position leave out elements outside the grid and edge-tile elements that touch
-# none of the tile's nodes)
-MFMA_EXEC_A32 = 520058 * 16384
+PEAK_FP32 = 157.3e12       # MI355X dense FP32, flop/s
+# arithmetic of one element's (cK K + cM M) u in the symmetry-adapted basis: sums and differences of the corner values
+# and back 144, the blocks 136, adding the 24 corner values 24
+ELEM_FLOPS = 304
 # HBM bytes per launch (FETCH_SIZE + WRITE_SIZE, rocprofv3 --pmc, FETCH scaled by 1.99922, the factor the
 # counters read for a device copy of 64 MiB; WRITE by 1.0)
-TRAFFIC_A32 = 20985242     # FP32 A apply: FETCH 7050.6 KiB, WRITE 6397.7 KiB
-TRAFFIC_FCG64 = 84492971   # FP64 flexible-CG apply: FETCH 28375.6 KiB, WRITE 25783.6 KiB
+TRAFFIC_A32 = 23220798     # FP32 A apply: FETCH 8127.2 KiB, WRITE 6428.5 KiB
+TRAFFIC_FCG64 = 89953651   # FP64 flexible-CG apply: FETCH 30946.0 KiB, WRITE 25977.5 KiB
 NEL = (128, 64, 64)
 DT = 0.005
 NLVLS = 4      # multigrid levels of the 128x64x64 workload (coarsest 16x8x8 elements, 4,131 dofs)
@@ -99,8 +96,8 @@ def op_microbench(capi, torch, nrep):
         err = float(torch.linalg.norm(y32.double() - ref) / torch.linalg.norm(ref))
         ms64 = ctx.time_op_apply(which, u64, y64, 0, nrep)
         ms32 = ctx.time_op_apply(which, u32, y32, 1, nrep)
-        # algorithmic flops: K dense 24x24 per element; M as (8x8 scalar) x I3 per element
-        fl = 2 * nel * ((576 if which != capi.TT_OP_M else 0) + (192 if which != capi.TT_OP_K else 0))
+        # arithmetic by the element modes (the mass matrix is diagonal there)
+        fl = nel * (192 if which == capi.TT_OP_M else ELEM_FLOPS)
         b64 = 2 * nd * 8 + 2 * nel * 8
         b32 = 2 * nd * 4 + 2 * nel * 4
         out[name] = {
@@ -205,7 +202,7 @@ def step_roofline_ms(precision, iters, cheb=2):
         return max(flops / peak, nbytes / PEAK_HBM)
 
     nel0, nn0, nd0 = lvl(0)
-    c = 2 * 1152  # flops per element of the stacked [K; M] contraction
+    c = ELEM_FLOPS
     step = t(c * nel0, 8 * (5 * nd0 + 2 * nel0) + nn0, PEAK_FP64)  # right-hand side
     step += t(c * nel0, 8 * (3 * nd0 + 2 * nel0) + nn0, PEAK_FP64)  # initial residual
     step += t(4 * nd0, 8 * 3 * nd0, PEAK_FP64)  # b.b, r.r
@@ -230,14 +227,14 @@ def step_roofline_ms(precision, iters, cheb=2):
 def gradient_roofline_s(precision, forward_steps, adjoint_steps, iters):
     """Roofline time of the adjoint gradient: forward steps (first sweep and revolve recomputation)
     plus adjoint steps, each a solve of the same operator plus the split K / M apply of the previous
-    multiplier, the adjoint vector combination and the sensitivity contraction (two stacked GEMMs,
-    4 x 1152 flops per element, reading 7 dof vectors)."""
+    multiplier, the adjoint vector combination and the sensitivities (four sets of modes and their products,
+    500 flops per element, reading 5 dof vectors and 7 element arrays)."""
     ex, ey, ez = NEL
     nel = ex * ey * ez
     nd = 3 * (ex + 1) * (ey + 1) * (ez + 1)
-    extra = (max(2 * 1152 * nel / PEAK_FP64, 8 * (3 * nd + 2 * nel) / PEAK_HBM)  # split apply
+    extra = (max(ELEM_FLOPS * nel / PEAK_FP64, 8 * (3 * nd + 2 * nel) / PEAK_HBM)  # split apply
              + 8 * 10 * nd / PEAK_HBM  # adjoint combination
-             + max(4 * 1152 * nel / PEAK_FP64, 8 * (7 * nd + 2 * nel) / PEAK_HBM))  # sensitivities
+             + max(500 * nel / PEAK_FP64, 8 * (5 * nd + 7 * nel) / PEAK_HBM))  # sensitivities
     step = step_roofline_ms(precision, iters) * 1e-3
     return forward_steps * step + adjoint_steps * (step + extra)
 
@@ -368,36 +365,29 @@ def main():
         cpu = cpu_baseline(x, args.cpu_steps)
 
     # roofline of the dominant kernel of the step: the FP64 flexible-CG apply of every Krylov iteration
-    # (z staged, A z contracted, p = z + beta p_old and q = A z + beta q_old = A p formed at the owned
-    # nodes, p.q partials), the largest single kernel of the mixed step.  Algorithmic work per launch: the
-    # stacked [K; M] 48x24 element contraction, 2 x 1152 flops per element; its algorithmic bytes: z, p_old,
-    # q_old read, p, q written (FP64), kfac, mfac, mask.
-    fl = 2 * 1152 * ops["A"]["nel"]
+    # (z staged, A z by the element modes, p = z + beta p_old and q = A z + beta q_old = A p formed at the owned
+    # nodes, p.q partials), the largest single kernel of the mixed step.  Algorithmic bytes per launch: z, p_old,
+    # q_old read, p, q written (FP64), kfac, mfac, mask; its arithmetic takes a fifth of their time.
     nd0, nel0 = ops["A"]["nd"], ops["A"]["nel"]
     fcg_ms = ops["fcg_fp64_ms"]
-    ach = fl / (fcg_ms * 1e-3) / 1e12
-    roof = {"bound": "mfma", "achieved": ach, "peak": PEAK_FP64 / 1e12, "unit": "TFLOP/s",
-            "frac": ach / (PEAK_FP64 / 1e12), "traffic": TRAFFIC_FCG64,
-            "kernel": "k_apply_tiles<double,double,4,true,StageOne<double>,EpiFcg> (flexible-CG apply: z staged, p = "
-                      "z + beta p_old, q = A z + beta q_old = A p, p.q partials; FP64, 128x64x64, 8x8x4-node tiles, "
-                      "v_mfma_f64_16x16x4f64)",
-            "kernel_ms": fcg_ms, "flops_per_launch": fl,
-            "algorithmic_bytes_per_launch": 8 * (5 * nd0 + 2 * nel0) + nd0 // 3}
-    # second entry: the FP32 Newmark-operator apply of the V-cycle smoothers (FP16-split matrix cores)
+    by = 8 * (5 * nd0 + 2 * nel0) + nd0 // 3
+    ach = by / (fcg_ms * 1e-3) / 1e12
+    roof = {"bound": "hbm", "achieved": ach, "peak": PEAK_HBM / 1e12, "unit": "TB/s",
+            "frac": ach / (PEAK_HBM / 1e12), "traffic": TRAFFIC_FCG64,
+            "kernel": "k_apply_cols<double,double,true,StageOne<double>,EpiFcg> (flexible-CG apply: z staged, p = "
+                      "z + beta p_old, q = A z + beta q_old = A p, p.q partials; FP64, 128x64x64, element columns)",
+            "kernel_ms": fcg_ms, "flops_per_launch": ELEM_FLOPS * nel0,
+            "algorithmic_bytes_per_launch": by}
+    # second entry: the FP32 Newmark-operator apply of the V-cycle smoothers
     a32 = ops["A"]
-    ach32 = fl / (a32["fp32_ms"] * 1e-3) / 1e12
+    by32 = 4 * (2 * nd0 + 2 * nel0) + nd0 // 3
+    ach32 = by32 / (a32["fp32_ms"] * 1e-3) / 1e12
     roof["fp32_apply"] = {
-        "bound": "mfma", "achieved": ach32, "peak": PEAK_FP32 / 1e12, "unit": "TFLOP/s",
-        "frac": ach32 / (PEAK_FP32 / 1e12), "traffic": TRAFFIC_A32,
-        "kernel": "k_apply_tiles<float,float,4,EpiBC> (A u = (1+a2 beta) K u + (a5+a2 alpha) M u, FP32, "
-                  "128x64x64, 8x8x4-node tiles, FP16-split v_mfma_f32_16x16x32_f16)",
-        "kernel_ms": a32["fp32_ms"], "flops_per_launch": fl,
-        # the FP32-accurate contraction runs as three FP16 products on the matrix cores: executed
-        # matrix-instruction work per launch (the counted v_mfma_f32_16x16x32_f16, 16,384 flops each)
-        # against the FP16 dense peak
-        "matrix_pipe": {"instr": "v_mfma_f32_16x16x32_f16", "executed_flops_per_launch": MFMA_EXEC_A32,
-                        "achieved": MFMA_EXEC_A32 / (a32["fp32_ms"] * 1e-3) / 1e12, "peak": PEAK_FP16 / 1e12,
-                        "unit": "TFLOP/s", "frac": MFMA_EXEC_A32 / (a32["fp32_ms"] * 1e-3) / PEAK_FP16}}
+        "bound": "hbm", "achieved": ach32, "peak": PEAK_HBM / 1e12, "unit": "TB/s",
+        "frac": ach32 / (PEAK_HBM / 1e12), "traffic": TRAFFIC_A32,
+        "kernel": "k_apply_cols<float,float,true,StageOne<float>,EpiBC> (A u = (1+a2 beta) K u + (a5+a2 alpha) M u, "
+                  "FP32, 128x64x64, element columns)",
+        "kernel_ms": a32["fp32_ms"], "flops_per_launch": ELEM_FLOPS * nel0, "algorithmic_bytes_per_launch": by32}
     # whole-step and whole-gradient rooflines (algorithmic work x measured iterations, against the
     # measured times)
     steps_roof = {}
