@@ -52,9 +52,9 @@ def test_filter(nel):
     assert rel(out, O.pde_filter(po, 0.11, x)) < 1e-10
 
 
-# coarsest grids: 1,911, 336, 81, 3,993 and 192 dofs
+# coarsest grids: 1,911, 336, 81, 3,993, 192 and 1,176 dofs; the last finest grid has 136,857 nodes (the wider prolongation)
 @pytest.mark.parametrize("nel,nlvls", [((24, 12, 12), 2), ((24, 12, 12), 3), ((16, 16, 16), 4), ((20, 20, 20), 2),
-                                       ((12, 12, 12), 3)])
+                                       ((12, 12, 12), 3), ((56, 48, 48), 4)])
 @pytest.mark.parametrize("precision", [capi.TT_PREC_FP64, capi.TT_PREC_MIXED])
 def test_levels_and_coarsest_solve(nel, nlvls, precision):
     print("levels", nel, nlvls, precision, flush=True)

@@ -1018,59 +1018,79 @@ void launch_restrict(const Grid& fine, const Grid& coarse, const void* rf, const
 // 4.0 + 3.4 us for the three kernels before.
 struct ProlongChain {
     const void* x[7];
-    int nx[7], ny[7];
+    int nx[7], ny[7], nz[7];
     int n;
 };
-// adds level l's correction at fine nodes (i, j, k) and (i + 1, j, k), i even: both lie in one cell of every coarser level
-template <typename Tf, typename Tx>
-__device__ __forceinline__ void prolong_level(const Tx* __restrict__ x, int nx, int ny, int l, int i, int j, int k,
-                                              Tf (&s0)[3], Tf (&s1)[3]) {
+// adds level l's correction at the fine nodes (i, j + b, k + d), b < 2, d < NZ (s[b + 2 d]), j (and k with NZ = 2) even: all
+// lie in one cell of every coarser level
+template <int NZ, typename Tf, typename Tx>
+__device__ __forceinline__ void prolong_level(const Tx* __restrict__ x, int nx, int ny, int nz, int l, int i, int j, int k,
+                                              Tf (&s)[2 * NZ][3]) {
     const Tf inv = (Tf)1 / (Tf)(1 << l);
     const int fi = i & ((1 << l) - 1), fj = j & ((1 << l) - 1), fk = k & ((1 << l) - 1);
-    const Tf w0 = (Tf)fi * inv, w1 = (Tf)(fi + 1) * inv, wj = (Tf)fj * inv, wk = (Tf)fk * inv;
-    const int di = (i >> l) + 1 < nx ? 3 : 0, dj = fj ? 3 * nx : 0, dk = fk ? 3 * nx * ny : 0;
+    const Tf wi = (Tf)fi * inv;
+    const int di = fi ? 3 : 0, dj = (j >> l) + 1 < ny ? 3 * nx : 0;
+    const int dk = (NZ == 2 ? (k >> l) + 1 < nz : fk != 0) ? 3 * nx * ny : 0;
     const Tx* p = x + 3 * ((size_t)(i >> l) + (size_t)nx * ((j >> l) + (size_t)ny * (k >> l)));
-    Tf a[3] = {0, 0, 0}, b[3] = {0, 0, 0};  // the cell's low-x and high-x edges at (j, k)
+    Tf v[2][2][3];  // the cell's edges in x at i: [z][y]
 #pragma unroll
     for (int q = 0; q < 4; q++) {
-        const Tf w = ((q & 1) ? wj : (Tf)1 - wj) * ((q & 2) ? wk : (Tf)1 - wk);
         const Tx* pq = p + ((q & 1) ? dj : 0) + ((q & 2) ? dk : 0);
 #pragma unroll
+        for (int c = 0; c < 3; c++) v[q >> 1][q & 1][c] = fma((Tf)1 - wi, (Tf)pq[c], wi * (Tf)pq[di + c]);
+    }
+#pragma unroll
+    for (int b = 0; b < 2; b++) {
+        const Tf wj = (Tf)(fj + b) * inv;
+#pragma unroll
         for (int c = 0; c < 3; c++) {
-            a[c] = fma(w, (Tf)pq[c], a[c]);
-            b[c] = fma(w, (Tf)pq[di + c], b[c]);
+            const Tf lo = fma((Tf)1 - wj, v[0][0][c], wj * v[0][1][c]), hi = fma((Tf)1 - wj, v[1][0][c], wj * v[1][1][c]);
+#pragma unroll
+            for (int d = 0; d < NZ; d++) {
+                const Tf wk = (Tf)(fk + d) * inv;
+                s[b + 2 * d][c] = fma((Tf)1 - wk, lo, fma(wk, hi, s[b + 2 * d][c]));
+            }
         }
     }
-#pragma unroll
-    for (int c = 0; c < 3; c++) {
-        s0[c] = fma((Tf)1 - w0, a[c], fma(w0, b[c], s0[c]));
-        s1[c] = fma((Tf)1 - w1, a[c], fma(w1, b[c], s1[c]));
-    }
 }
-template <typename Tf, typename Tl>  // Tl: the last (coarsest) level's type; one thread per pair of nodes in x
+// Tl: the last (coarsest) level's type; one thread per two nodes in y (and NZ in z), the lanes of a wave along x, so that
+// the fine vector is read and written in order and neighbouring lanes share the coarse loads: the kernel is bound by
+// its memory instructions.  128x64x64, 3 coarser levels: 11.8 us (FP32) and 16.4 us (FP64) with two nodes in x per
+// thread, 10.4 and 15.0 with NZ = 1, 8.5 and 13.4 with NZ = 2.  NZ = 2 takes grids above kChainNodes: at 70,785 nodes
+// (64x32x32) NZ = 1 and 2 take 5.6 and 5.6 us (FP32), 6.1 and 7.2 (FP64), at 1,377 (16x8x8) 3.6 and 4.0, at 232,897
+// (96x48x48, FP32) 6.5 and 5.9.
+constexpr long kChainNodes = 131072;
+template <int NZ, typename Tf, typename Tl>
 __global__ void k_prolong_chain(GridArgs f, ProlongChain pc, const uint8_t* __restrict__ fmask, Tf* __restrict__ xf) {
-    const unsigned px = (unsigned)(f.nx + 1) >> 1;
+    const unsigned py = (unsigned)(f.ny + 1) >> 1, pz = (unsigned)(f.nz + NZ - 1) / NZ;
     const long t = blockIdx.x * (long)blockDim.x + threadIdx.x;
-    if (t >= (long)px * f.ny * f.nz) return;
+    if (t >= (long)f.nx * py * pz) return;
     int i, j, k;
-    grid_ijk((unsigned)t, px, f.ny, i, j, k);
-    i *= 2;
+    grid_ijk((unsigned)t, f.nx, py, i, j, k);
+    j *= 2;
+    k *= NZ;
+    // (a node beyond the grid is read as the one before it and not written)
+    const long oy = j + 1 < f.ny ? f.nx : 0, oz = NZ == 2 && k + 1 < f.nz ? (long)f.nx * f.ny : 0;
     const long n = i + (long)f.nx * (j + (long)f.ny * k);
-    const bool two = i + 1 < f.nx;
-    const uint8_t cl0 = fmask[n], cl1 = two ? fmask[n + 1] : (uint8_t)7;
-    Tf x[6], s0[3] = {0, 0, 0}, s1[3] = {0, 0, 0};
+    uint8_t cl[2 * NZ];
+    Tf x[2 * NZ][3], s[2 * NZ][3] = {};
 #pragma unroll
-    for (int c = 0; c < 3; c++) x[c] = xf[3 * n + c];
-    if (two)
+    for (int q = 0; q < 2 * NZ; q++) {
+        const long m = n + ((q & 1) ? oy : 0) + ((q & 2) ? oz : 0);
+        cl[q] = ((q & 1) && !oy) || ((q & 2) && !oz) ? (uint8_t)7 : fmask[m];
 #pragma unroll
-        for (int c = 3; c < 6; c++) x[c] = xf[3 * n + c];
+        for (int c = 0; c < 3; c++) x[q][c] = xf[3 * m + c];
+    }
     for (int l = 0; l + 1 < pc.n; l++)
-        prolong_level<Tf, Tf>((const Tf*)pc.x[l], pc.nx[l], pc.ny[l], l + 1, i, j, k, s0, s1);
-    prolong_level<Tf, Tl>((const Tl*)pc.x[pc.n - 1], pc.nx[pc.n - 1], pc.ny[pc.n - 1], pc.n, i, j, k, s0, s1);
+        prolong_level<NZ, Tf, Tf>((const Tf*)pc.x[l], pc.nx[l], pc.ny[l], pc.nz[l], l + 1, i, j, k, s);
+    const int l = pc.n - 1;
+    prolong_level<NZ, Tf, Tl>((const Tl*)pc.x[l], pc.nx[l], pc.ny[l], pc.nz[l], l + 1, i, j, k, s);
 #pragma unroll
-    for (int c = 0; c < 3; c++) {
-        if (!((cl0 >> c) & 1)) xf[3 * n + c] = x[c] + s0[c];
-        if (!((cl1 >> c) & 1)) xf[3 * n + 3 + c] = x[3 + c] + s1[c];
+    for (int q = 0; q < 2 * NZ; q++) {
+        const long m = n + ((q & 1) ? oy : 0) + ((q & 2) ? oz : 0);
+#pragma unroll
+        for (int c = 0; c < 3; c++)
+            if (!((cl[q] >> c) & 1)) xf[3 * m + c] = x[q][c] + s[q][c];
     }
 }
 void launch_prolong_chain(const Grid& fine, int n, const Grid* const* coarse, const void* const* xc,
@@ -1082,14 +1102,23 @@ void launch_prolong_chain(const Grid& fine, int n, const Grid* const* coarse, co
         pc.x[l] = xc[l];
         pc.nx[l] = coarse[l]->nx;
         pc.ny[l] = coarse[l]->ny;
+        pc.nz[l] = coarse[l]->nz;
     }
-    const dim3 gr(nblocks((long)((fine.nx + 1) / 2) * fine.ny * fine.nz)), bl(BS);
-    if (fp64)
-        hipLaunchKernelGGL((k_prolong_chain<double, double>), gr, bl, 0, s, gargs(fine), pc, fmask, (double*)xf);
-    else if (last64)
-        hipLaunchKernelGGL((k_prolong_chain<float, double>), gr, bl, 0, s, gargs(fine), pc, fmask, (float*)xf);
-    else
-        hipLaunchKernelGGL((k_prolong_chain<float, float>), gr, bl, 0, s, gargs(fine), pc, fmask, (float*)xf);
+    auto launch = [&](auto kernel, int nz, auto* x) {
+        const long threads = (long)fine.nx * ((fine.ny + 1) / 2) * ((fine.nz + nz - 1) / nz);
+        hipLaunchKernelGGL(kernel, dim3(nblocks(threads)), dim3(BS), 0, s, gargs(fine), pc, fmask, x);
+    };
+    const bool big = fine.nn > kChainNodes;
+    if (fp64) {
+        if (big) launch(k_prolong_chain<2, double, double>, 2, (double*)xf);
+        else launch(k_prolong_chain<1, double, double>, 1, (double*)xf);
+    } else if (last64) {
+        if (big) launch(k_prolong_chain<2, float, double>, 2, (float*)xf);
+        else launch(k_prolong_chain<1, float, double>, 1, (float*)xf);
+    } else {
+        if (big) launch(k_prolong_chain<2, float, float>, 2, (float*)xf);
+        else launch(k_prolong_chain<1, float, float>, 1, (float*)xf);
+    }
     TT_HIP(hipGetLastError());
 }
 
