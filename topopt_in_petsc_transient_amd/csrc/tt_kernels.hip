@@ -949,7 +949,8 @@ void launch_cheb_first(const void* b, const void* dinv, double c1, void* x, long
 // The coarse output may be wider than the fine input (FP32 levels feeding an FP64 coarsest solve).
 // NC: components per thread.  A node per thread (3) where the coarse grid has enough nodes to fill the chip: one wide load
 // per neighbour; a dof per thread (1) below, where more and shorter chains of loads are what counts: at 225 coarse nodes
-// 2.8 instead of 4.6 us (FP64), at 35,937 4.7 instead of 3.9 us (FP32).
+// 2.8 instead of 4.6 us (FP64), at 35,937 4.7 instead of 3.9 us (FP32).  Blocks of one wave (3): the grid is about one wave
+// per SIMD, and 277 blocks of 256 left a second round on 21 CUs (70,785 coarse nodes: FP32 8.7 -> 6.1 us, FP64 9.0 -> 7.1).
 template <int NC, typename Tf, typename Tc>
 __global__ void k_restrict(GridArgs f, GridArgs c, const Tf* __restrict__ rf, const uint8_t* __restrict__ cmask,
                            Tc* __restrict__ bc) {
@@ -991,7 +992,7 @@ __global__ void k_restrict(GridArgs f, GridArgs c, const Tf* __restrict__ rf, co
 void launch_restrict(const Grid& fine, const Grid& coarse, const void* rf, const uint8_t* cmask, void* bc, bool fp64,
                      bool out64, hipStream_t s) {
     auto launch = [&](auto kernel, int nc, auto* src, auto* dst) {
-        const int bs = nc == 3 ? BS : 128;
+        const int bs = nc == 3 ? 64 : 128;
         hipLaunchKernelGGL(kernel, dim3(nblocks(3 / nc * coarse.nn, bs)), dim3(bs), 0, s, gargs(fine), gargs(coarse), src,
                            cmask, dst);
     };
@@ -1058,7 +1059,7 @@ __device__ __forceinline__ void prolong_level(const Tx* __restrict__ x, int nx, 
 // its memory instructions.  128x64x64, 3 coarser levels: 11.8 us (FP32) and 16.4 us (FP64) with two nodes in x per
 // thread, 10.4 and 15.0 with NZ = 1, 8.5 and 13.4 with NZ = 2.  NZ = 2 takes grids above kChainNodes: at 70,785 nodes
 // (64x32x32) NZ = 1 and 2 take 5.6 and 5.6 us (FP32), 6.1 and 7.2 (FP64), at 1,377 (16x8x8) 3.6 and 4.0, at 232,897
-// (96x48x48, FP32) 6.5 and 5.9.
+// (96x48x48, FP32) 6.5 and 5.9.  Blocks of one wave even out the CUs (9.1 -> 8.7 us on one box, 3.4 -> 3.1 at 16x8x8).
 constexpr long kChainNodes = 131072;
 template <int NZ, typename Tf, typename Tl>
 __global__ void k_prolong_chain(GridArgs f, ProlongChain pc, const uint8_t* __restrict__ fmask, Tf* __restrict__ xf) {
@@ -1106,7 +1107,7 @@ void launch_prolong_chain(const Grid& fine, int n, const Grid* const* coarse, co
     }
     auto launch = [&](auto kernel, int nz, auto* x) {
         const long threads = (long)fine.nx * ((fine.ny + 1) / 2) * ((fine.nz + nz - 1) / nz);
-        hipLaunchKernelGGL(kernel, dim3(nblocks(threads)), dim3(BS), 0, s, gargs(fine), pc, fmask, x);
+        hipLaunchKernelGGL(kernel, dim3(nblocks(threads, 64)), dim3(64), 0, s, gargs(fine), pc, fmask, x);
     };
     const bool big = fine.nn > kChainNodes;
     if (fp64) {
