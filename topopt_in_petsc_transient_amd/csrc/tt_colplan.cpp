@@ -60,18 +60,15 @@ void col_bc_flags(const Grid& g, const ColPlan& p, const std::vector<uint8_t>& m
         lo = std::max(0, (i + b - 1) / b - 1);
         hi = std::min(nt - 1, (i + 1) / b);
     };
-    std::vector<int> zlo(g.nz, 0), zhi(g.nz, 0);
-    for (int k = 0; k < g.nz; k++) {
-        int lo = -1, hi = -1;
-        for (int c = 0; c < p.tz; c++) {
-            const int k0 = (int)((long)c * g.nz / p.tz), k1 = (int)((long)(c + 1) * g.nz / p.tz);
-            if (k >= k0 - 1 && k <= k1) {
-                if (lo < 0) lo = c;
-                hi = c;
-            }
+    // the parts that stage node plane k: zlo[k] .. zhi[k] (one pass over the parts, which follow one another: a rod's
+    // grid has thousands of both)
+    std::vector<int> zlo(g.nz, p.tz), zhi(g.nz, -1);
+    for (int c = 0; c < p.tz; c++) {
+        const int k0 = (int)((long)c * g.nz / p.tz), k1 = (int)((long)(c + 1) * g.nz / p.tz);
+        for (int k = std::max(k0 - 1, 0); k <= std::min(k1, g.nz - 1); k++) {
+            zlo[k] = std::min(zlo[k], c);
+            zhi[k] = c;
         }
-        zlo[k] = lo;
-        zhi[k] = hi;
     }
     for (int k = 0; k < g.nz; k++)
         for (int j = 0; j < g.ny; j++)
