@@ -3,6 +3,8 @@ the CPU by small programs.
 
 * col_bc_flags takes time in proportion to the grid: a rod of 400,001 planes in 200,000 parts is done at once (formed
   part by part for every plane it takes minutes), with the flags of a direct test of every part's planes.
+* make_col_plan cuts a block's planes into strands where the cross-section's columns fit the block twice or more, as many
+  as its 256 threads and 1,024 staging slots hold, and into one otherwise.
 """
 import os
 import subprocess
@@ -40,6 +42,33 @@ int main() {
 }
 """
 
+STRANDS = r"""
+#include "tt_colplan.cpp"
+#include <cstdio>
+using namespace tt;
+int main() {
+    int bad = 0;
+    const int cs[][2] = {{1, 1}, {2, 2}, {3, 3}, {5, 5}, {7, 7}, {8, 8}, {9, 9}, {1, 7}, {7, 1}, {2, 20}, {20, 2}, {1, 39}, {3, 24},
+                         {10, 10}, {40, 20}, {128, 64}};
+    for (auto& c : cs)
+        for (long n : {45000, 70000, 900000})
+            for (int d = 0; d < 2; d++) {
+                const Grid g = make_grid(c[0], c[1], (int)(n / ((c[0] + 1) * (c[1] + 1))), 1, 1, 1);
+                const ColPlan p = make_col_plan(g, d != 0);
+                const int cols = p.cx * (p.by + 1), dofs = 3 * (p.bx + 2) * (p.by + 2);
+                int e = p.strands < 1 || p.strands * cols > 256 || p.strands * dofs > 1024 ||
+                        (p.strands > 1 && (p.tx * p.ty != 1 || p.bx != g.nx || p.by != g.ny));
+                // a tile of the whole cross-section is filled up; of a small one (half the threads idle) it is taken
+                if (p.tx * p.ty == 1) e += (p.strands + 1) * cols <= 256 && (p.strands + 1) * dofs <= 1024;
+                if (2 * (g.nx + 1) * (g.ny + 1) <= 170 && 6 * (g.nx + 2) * (g.ny + 2) <= 1024) e += p.strands < 2;
+                if (e) printf("%d x %d, %ld, %d: strands %d, %d columns, %d dofs\n", c[0], c[1], n, d, p.strands, cols, dofs);
+                bad += e;
+            }
+    printf("bad %d\n", bad);
+    return bad != 0;
+}
+"""
+
 
 def _run(tmp_path, name, prog, timeout):
     src = tmp_path / (name + ".cpp")
@@ -53,3 +82,7 @@ def _run(tmp_path, name, prog, timeout):
 
 def test_flags_of_a_rod(tmp_path):
     _run(tmp_path, "flags", FLAGS, 20)
+
+
+def test_strands_of_a_rod(tmp_path):
+    _run(tmp_path, "strands", STRANDS, 60)

@@ -33,17 +33,19 @@ ColPlan make_col_plan(const Grid& g, bool fp64) {
         for (int cy = std::min(3, cymax); cy <= cymax; cy++) {
             const int by = cy - 1, ty = (g.ny + by - 1) / by;
             const double row = (std::min(cx, g.nx) + 1) * 3.0 * (fp64 ? 8 : 4) / 128.0 + 1.0;
-            const double touched = lines * row * (std::min(cy, g.ny) + 1) / 100.0;
+            // a tile of the whole cross-section with room for more beside it: its planes in strands (ROD in tt_apply_cols.inc)
+            const int strands = tx * ty == 1 ? std::max(1, std::min(256 / (cx * cy), 1024 / (3 * (cx + 1) * (cy + 1)))) : 1;
+            const double touched = lines * strands * row * (std::min(cy, g.ny) + 1) / 100.0;
             auto plane = [&](int r) { return base[r - 1] + r * touched; };
             for (int nk = 1;;) {  // planes per block: the fewest that give each number of blocks in z
                 const int tz = (g.nz + nk - 1) / nk;
                 const double nt = (double)tx * ty * tz, per = nt / cus;
                 const int r = (int)std::ceil(per);
                 // (between splits of one modelled time, the one with fewer blocks)
-                const double c = 1e-4 * nt + (nk + 2) * (r <= resident ? plane(r) : plane(resident) * (tail + per / resident));
+                const double c = 1e-4 * nt + ((nk + strands - 1) / strands + 2) * (r <= resident ? plane(r) : plane(resident) * (tail + per / resident));
                 if (c < cost) {
                     cost = c;
-                    best = ColPlan{cx, bx, by, tx, ty, tz};
+                    best = ColPlan{cx, bx, by, tx, ty, tz, strands};
                 }
                 if (tz == 1) break;
                 nk = (g.nz + tz - 2) / (tz - 1);

@@ -115,6 +115,7 @@ void upload_modes(const double* ke, const double* m8, DBuf<ModeConst<double>>& d
 struct ColPlan {
     int cx, bx, by;
     int tx, ty, tz;
+    int strands = 1;  // parts of a block's planes that march side by side (a rod's tile: its whole cross-section)
     int ntiles() const { return tx * ty * tz; }
     // blocks of a launch (column kernel: rounded up to a multiple of 8 for the XCD-aware tile order)
     int blocks() const { return cx ? 8 * ((ntiles() + 7) / 8) : ntiles(); }

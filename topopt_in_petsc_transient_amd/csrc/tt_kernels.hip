@@ -642,8 +642,12 @@ static int launch_cols_ct(const OpLevel& L, double cK, double cM, const Stage& s
         return tx * ty * tz;
     }
     const int nb = 8 * ((p.ntiles() + 7) / 8);
-    hipLaunchKernelGGL((k_apply_cols<T, CT, MASKIN, Stage, Epi>), dim3(nb), dim3(256), 0, s, gargs(L.g), p, mc,
-                       (const CT*)L.kf, (const CT*)L.mf, (T)cK, (T)cM, L.mask, cs.bc, st, epi);
+    auto launch = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3(nb), dim3(256), 0, s, gargs(L.g), p, mc, (const CT*)L.kf, (const CT*)L.mf, (T)cK,
+                           (T)cM, L.mask, cs.bc, st, epi);
+    };
+    if (p.strands > 1) launch(k_apply_cols<T, CT, MASKIN, true, Stage, Epi>);
+    else launch(k_apply_cols<T, CT, MASKIN, false, Stage, Epi>);
     TT_HIP(hipGetLastError());
     return nb;
 }
