@@ -1779,23 +1779,36 @@ void launch_fcg_update(double* x, const double* p, double* r, const double* q, l
 // ------------------------------------------------------------------ PDE filter operator (PDEFilter.cc)
 // On the node grid of a box the Helmholtz matrix is a sum of products of 1-D matrices (stiffness K = [-1 c -1] / h, mass
 // M = [1 2c 1] h / 6 per direction, c = the 1 or 2 elements at the node), R^2 (Kx My Mz + Mx Ky Mz + Mx My Kz) +
-// Mx My Mz.  A block owns 32 x 8 node columns and marches up its planes: a plane (with one halo node) is staged in LDS,
+// Mx My Mz.  A block owns BX x BY node columns (32 x 8, narrower where the grid is) and marches up its planes: a plane (with one halo node) is staged in LDS,
 // each thread forms A = My Mx u and B = (R^2 (Kx My + Mx Ky) + Mx My) u of its column from the 9 neighbours, and the
 // row sum is Mz B + R^2 Kz A over three planes.  The staged value is the solution (the residual) or the CG direction
 // formed on the fly.  At 128x64x64 a CG iteration's two kernels (this one and k_fcg_update) replace seven (48 us:
 // Jacobi, dots, beta, direction, an apply that gathered 64 products per node, alpha, update).
-constexpr int FX = 32, FY = 8, FHX = FX + 2, FHY = FY + 2;
-template <bool CG>  // CG: u = p = D^-1 r + beta p_old (written), y = q = A p, partials of p.q; else y = rhs - A u
+// A cross-section of up to 8 x 8 nodes takes S = 4 or 16 parts of a block's planes side by side (strands, as the operator's
+// columns).  Whole filter calls on device arrays, us, the node-by-node operator of seven kernels an iteration that the march
+// replaced, 32 x 8 tiles alone, and tiles by the grid: 1x1x20000 elements 696 -> 963 -> 585, 3x3x30000 1173 -> 1384 -> 705,
+// 3x30000x3 1107 -> 1498 -> 695, 1x500x500 1182 -> 1651 -> 733, 1x1000x1000 3247 -> 5084 -> 1501 (129 x 65 x 65 nodes: the
+// same tiles as before).
+template <int LBX, int LBY>
+struct FilterTile {
+    static constexpr int BX = 1 << LBX, BY = 1 << LBY, S = 256 >> (LBX + LBY), HX = BX + 2, BOX = HX * (BY + 2),
+                         Q = (S * BOX + 255) / 256;  // staged nodes per strand and per thread
+};
+template <bool CG, int LBX, int LBY>  // CG: u = p = D^-1 r + beta p_old (written), y = q = A p, partials of p.q; else y = rhs - A u
 __global__ __launch_bounds__(256) void k_filter_op(GridArgs g, FilterOp f, int tx, int ty, int tz,
                                                    const double* __restrict__ a0, const double* __restrict__ dinv,
                                                    const double* __restrict__ a1, double* __restrict__ pnew,
                                                    double* __restrict__ y, double* part0, double* part1, double* part2,
                                                    const double* dots, int dots_nblk, double* scal, int first) {
-    __shared__ double su[2][FHX * FHY];
-    const int tid = threadIdx.x, lx = tid & 31, ly = tid >> 5;
+    typedef FilterTile<LBX, LBY> F;
+    constexpr int S = F::S, FHX = F::HX, Q = F::Q;
+    __shared__ double su[2][S * F::BOX];
+    const int tid = threadIdx.x, lx = tid & (F::BX - 1), ly = (tid >> LBX) & (F::BY - 1);
     const int tile = blockIdx.x, tzi = tile / (tx * ty), tr = tile - tzi * tx * ty, tyi = tr / tx, txi = tr - tyi * tx;
-    const int i0 = txi * FX, j0 = tyi * FY;
-    const int k0 = (int)((long)tzi * g.nz / tz), k1 = (int)((long)(tzi + 1) * g.nz / tz);
+    const int i0 = txi * F::BX, j0 = tyi * F::BY;
+    const int k0 = (int)((long)tzi * g.nz / tz), nk = (int)((long)(tzi + 1) * g.nz / tz) - k0;
+    // a strand's planes, and the thread's: koff above the march's, below kend
+    const int np = (nk + S - 1) / S, koff = (S > 1 ? tid >> (LBX + LBY) : 0) * np, kend = k0 + min(koff + np, nk);
     const int i = i0 + lx, j = j0 + ly;
     const bool own = i < g.nx && j < g.ny;
     double beta = 0.0;
@@ -1809,21 +1822,23 @@ __global__ __launch_bounds__(256) void k_filter_op(GridArgs g, FilterOp f, int t
     double mx[3], kx[3], my[3], ky[3];
     row(i, g.nx, f.h[0], mx, kx);
     row(j, g.ny, f.h[1], my, ky);
-    // staging: two of the 340 box nodes per thread
-    int so[2];
-    bool sv[2];
+    // staging: Q of the box nodes per thread
+    int so[Q], sk[Q];
+    bool sv[Q];
 #pragma unroll
-    for (int q = 0; q < 2; q++) {
-        const int v = tid + q * 256, sy = v / FHX, sx = v - sy * FHX;
-        sv[q] = v < FHX * FHY;
+    for (int q = 0; q < Q; q++) {
+        const int v = tid + q * 256, st = S > 1 ? min(v / F::BOX, S - 1) : 0, w = v - st * F::BOX, sy = w / FHX,
+                  sx = w - sy * FHX;
+        sv[q] = v < S * F::BOX;
+        sk[q] = st * np;
         so[q] = min(max(i0 - 1 + sx, 0), g.nx - 1) + g.nx * min(max(j0 - 1 + sy, 0), g.ny - 1);
     }
     const int plane = g.nx * g.ny;
-    double v0[2], v1[2], v2[2];
+    double v0[Q], v1[Q], v2[Q];
     auto load = [&](int k) {
-        const size_t b = (size_t)min(max(k, 0), g.nz - 1) * plane;
 #pragma unroll
-        for (int q = 0; q < 2; q++) {
+        for (int q = 0; q < Q; q++) {
+            const size_t b = (size_t)min(max(S > 1 ? k + sk[q] : k, 0), g.nz - 1) * plane;
             v0[q] = a0[b + so[q]];
             if constexpr (CG) {
                 v1[q] = dinv[b + so[q]];
@@ -1833,7 +1848,7 @@ __global__ __launch_bounds__(256) void k_filter_op(GridArgs g, FilterOp f, int t
     };
     auto commit = [&](int b) {
 #pragma unroll
-        for (int q = 0; q < 2; q++) {
+        for (int q = 0; q < Q; q++) {
             double x = v0[q];
             if constexpr (CG) {
                 x = v1[q] * v0[q];
@@ -1846,11 +1861,11 @@ __global__ __launch_bounds__(256) void k_filter_op(GridArgs g, FilterOp f, int t
     load(k0 - 1);
     commit(0);
     __syncthreads();
-    for (int k = k0 - 1; k <= k1; k++) {  // plane k is staged in su[(k - k0 + 1) & 1]
+    for (int k = k0 - 1; k <= k0 + np; k++) {  // plane k is staged in su[(k - k0 + 1) & 1]
         const int sb = (k - k0 + 1) & 1;
-        if (k < k1) load(k + 1);
+        if (k < k0 + np) load(k + 1);
         double As = 0.0, Bs = 0.0;
-        const double* u = &su[sb][ly * FHX + lx];
+        const double* u = &su[sb][(S > 1 ? (tid >> (LBX + LBY)) * F::BOX : 0) + ly * FHX + lx];
 #pragma unroll
         for (int r = 0; r < 3; r++) {
             const double ul = u[r * FHX], uc = u[r * FHX + 1], ur = u[r * FHX + 2];
@@ -1862,8 +1877,8 @@ __global__ __launch_bounds__(256) void k_filter_op(GridArgs g, FilterOp f, int t
         const double un = u[FHX + 1];
         A[0] = A[1]; A[1] = A[2]; A[2] = As;
         B[0] = B[1]; B[1] = B[2]; B[2] = Bs;
-        const int kk = k - 1;  // the plane whose three neighbours are now known
-        if (kk >= k0 && own) {
+        const int kk = k - 1 + koff;  // the plane whose three neighbours are now known
+        if (k > k0 && kk < kend && own) {
             double mz[3], kz[3];
             row(kk, g.nz, f.h[2], mz, kz);
             double s = 0.0;
@@ -1883,7 +1898,7 @@ __global__ __launch_bounds__(256) void k_filter_op(GridArgs g, FilterOp f, int t
             }
         }
         uo[0] = un;
-        if (k < k1) commit(sb ^ 1);
+        if (k < k0 + np) commit(sb ^ 1);
         __syncthreads();
     }
     __shared__ double sh[16 * 3];
@@ -1897,24 +1912,42 @@ __global__ __launch_bounds__(256) void k_filter_op(GridArgs g, FilterOp f, int t
         }
     }
 }
-// tiles: about 4 blocks per CU, at least one plane each
-static inline dim3 filter_tiles(const Grid& g) {
-    const int tx = (g.nx + FX - 1) / FX, ty = (g.ny + FY - 1) / FY;
-    return dim3(tx, ty, std::min(g.nz, std::max(1, 1024 / (tx * ty))));
+// tiles: about 4 blocks per CU, at least one plane (of each strand)
+struct FilterPlan {
+    int lbx, lby, tx, ty, tz;
+    int blocks() const { return tx * ty * tz; }
+};
+static inline FilterPlan filter_plan(const Grid& g) {
+    FilterPlan p{5, 3, 0, 0, 0};
+    while (p.lbx > 2 && (1 << (p.lbx - 1)) >= g.nx) p.lbx--;
+    p.lby = 8 - p.lbx;
+    if (g.nx <= 8 && g.ny <= 8) p.lbx = p.lby = g.nx <= 4 && g.ny <= 4 ? 2 : 3;
+    const int s = 256 >> (p.lbx + p.lby);
+    p.tx = (g.nx + (1 << p.lbx) - 1) >> p.lbx;
+    p.ty = (g.ny + (1 << p.lby) - 1) >> p.lby;
+    p.tz = std::min((g.nz + s - 1) / s, std::max(1, 1024 / (p.tx * p.ty)));
+    return p;
 }
-long filter_blocks(const Grid& g) {
-    const dim3 t = filter_tiles(g);
-    return (long)t.x * t.y * t.z;
+long filter_blocks(const Grid& g) { return filter_plan(g).blocks(); }
+template <bool CG, class... Args>
+static void filter_op(const Grid& g, const FilterPlan& p, hipStream_t s, const FilterOp& f, Args... args) {
+    auto launch = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3(p.blocks()), dim3(256), 0, s, gargs(g), f, p.tx, p.ty, p.tz, args...);
+    };
+    if (p.lbx + p.lby < 8) p.lbx == 2 ? launch(k_filter_op<CG, 2, 2>) : launch(k_filter_op<CG, 3, 3>);
+    else if (p.lbx == 5) launch(k_filter_op<CG, 5, 3>);
+    else if (p.lbx == 4) launch(k_filter_op<CG, 4, 4>);
+    else if (p.lbx == 3) launch(k_filter_op<CG, 3, 5>);
+    else launch(k_filter_op<CG, 2, 6>);
+    TT_HIP(hipGetLastError());
 }
 void launch_filter_residual(const Grid& g, const FilterOp& f, const double* U, const double* rhs, const double* dinv,
                             double* r, Reducer& red, bool bb, hipStream_t s) {
-    const dim3 t = filter_tiles(g);
-    const int nb = t.x * t.y * t.z;
+    const FilterPlan p = filter_plan(g);
+    const int nb = p.blocks();
     TT_CHECK(nb <= red.maxblocks, -3, "reducer too small");
-    hipLaunchKernelGGL(k_filter_op<false>, dim3(nb), dim3(256), 0, s, gargs(g), f, (int)t.x, (int)t.y, (int)t.z, U, dinv,
-                       rhs, (double*)nullptr, r, red.part(PB_MISC2), red.part(PB_DOTS),
-                       bb ? red.part(PB_MISC) : (double*)nullptr, (const double*)nullptr, 0, (double*)nullptr, 0);
-    TT_HIP(hipGetLastError());
+    filter_op<false>(g, p, s, f, U, dinv, rhs, (double*)nullptr, r, red.part(PB_MISC2), red.part(PB_DOTS),
+                     bb ? red.part(PB_MISC) : (double*)nullptr, (const double*)nullptr, 0, (double*)nullptr, 0);
     for (int region : {(int)PB_MISC2, (int)PB_DOTS, (int)PB_MISC})
         if (region != PB_MISC || bb) {
             red.nblk[region] = nb;
@@ -1923,13 +1956,11 @@ void launch_filter_residual(const Grid& g, const FilterOp& f, const double* U, c
 }
 void launch_filter_direction(const Grid& g, const FilterOp& f, const double* r, const double* dinv, const double* p_old,
                              double* p_new, double* q, Reducer& red, bool first, hipStream_t s) {
-    const dim3 t = filter_tiles(g);
-    const int nb = t.x * t.y * t.z;
+    const FilterPlan p = filter_plan(g);
+    const int nb = p.blocks();
     TT_CHECK(nb <= red.maxblocks, -3, "reducer too small");
-    hipLaunchKernelGGL(k_filter_op<true>, dim3(nb), dim3(256), 0, s, gargs(g), f, (int)t.x, (int)t.y, (int)t.z, r, dinv,
-                       p_old, p_new, q, red.part(PB_PQ), (double*)nullptr, (double*)nullptr, red.part(PB_DOTS),
-                       red.nblk[PB_DOTS], red.scal.p, first ? 1 : 0);
-    TT_HIP(hipGetLastError());
+    filter_op<true>(g, p, s, f, r, dinv, p_old, p_new, q, red.part(PB_PQ), (double*)nullptr, (double*)nullptr,
+                    (const double*)red.part(PB_DOTS), red.nblk[PB_DOTS], red.scal.p, first ? 1 : 0);
     red.nblk[PB_PQ] = nb;
     red.nv[PB_PQ] = 1;
 }
