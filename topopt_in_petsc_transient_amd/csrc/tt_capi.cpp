@@ -29,9 +29,9 @@ static void check_params(const tt_params& p) {
              "omega0 must be nonzero: the basis vectors after the first are solves with 2 omega0 M Q");
     long nn = (long)(p.nelx + 1) * (p.nely + 1) * (p.nelz + 1);
     TT_CHECK(3 * nn < (1L << 31), TT_ERR_ARG, "too many dofs for 32-bit indexing");
-    // the kernels address FP64 dof vectors through 32-bit byte offsets and form node indices with
-    // 24-bit multiplies over one y-z cross-section
+    // the kernels address FP64 dof vectors through 32-bit byte offsets
     TT_CHECK(3 * nn * 8 < (1L << 32), TT_ERR_ARG, "too many dofs for 32-bit byte offsets (nodes must be < 178,956,970)");
+    // (no kernel's index arithmetic needs this one; flatter grids have never been run, and stay refused)
     TT_CHECK((long)(p.nely + 1) * (p.nelz + 1) < (1L << 24), TT_ERR_ARG, "y-z cross-section above 2^24 nodes");
 }
 
