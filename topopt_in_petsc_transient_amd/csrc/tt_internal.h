@@ -165,16 +165,12 @@ enum {
     SC_GAMMA = 0,   // z.r of current iteration
     SC_GAMMA_OLD,   // z.r of previous iteration
     SC_ALPHA,       // step length of the last update
-    SC_RR,          // r.r
-    SC_TMP0,
-    SC_TMP1,
     SC_TMP2,
     SC_TMP3,
     SC_DONE,        // flexible CG: 1 once the recursive residual met the tolerance (x is then frozen)
     SC_TOL2,        // flexible CG: (rtol ||b||)^2
     SC_ZERO,        // flexible CG: 1 if b = 0 (the solution is x = 0)
     SC_ITERS,       // flexible CG: iterations that moved x in this solve
-    SC_FX0,         // objective accumulators start here
     SC_COUNT = 32
 };
 
@@ -437,7 +433,6 @@ void launch_mma_movelimit(const double* x, double* xmin, double* xmax, long n, d
 void launch_mma_change(const double* x, double* xold, long n, Reducer& red, int slot, hipStream_t s);
 void launch_mma_kkt(const double* x, const double* df, const double* dg, const double* xmin, const double* xmax,
                     long n, double lam, Reducer& red, hipStream_t s);
-void launch_fill_scal(void* x, long n, double v, hipStream_t s);
 // x_i in [-1, 1) from a counter-based hash of (seed, i): deterministic, generated on the device
 void launch_fill_hash(void* x, long n, unsigned long long seed, bool fp64, hipStream_t s);
 // x = N.x (clamped dofs of the node mask set to 0)
@@ -445,9 +440,6 @@ void launch_mask_dofs(double* x, const uint8_t* mask, long nd, hipStream_t s);
 void launch_scale(double* x, long n, double a, hipStream_t s);
 // out = a*x + b*y (out may alias x or y)
 void launch_lincomb(double a, const double* x, double b, const double* y, double* out, long n, hipStream_t s);
-// out = a x + b y + c z
-void launch_lincomb3(double a, const double* x, double b, const double* y, double c, const double* z, double* out,
-                     long n, hipStream_t s);
 // out = sum_k c[k] v[k] over the m <= 8 vectors of e (polynomial extrapolation of a sequence)
 struct Extrap {
     const double* v[8];

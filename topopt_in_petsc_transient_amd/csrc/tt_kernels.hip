@@ -23,9 +23,6 @@ template <typename T>
 __device__ __forceinline__ T ld(const T* p, unsigned i) {
     return *reinterpret_cast<const T*>(reinterpret_cast<const char*>(p) + i * (unsigned)sizeof(T));
 }
-__device__ __forceinline__ double coef_ld(const double* p, unsigned i) { return ld(p, i); }
-__device__ __forceinline__ double coef_ld(const float* p, unsigned i) { return (double)ld(p, i); }
-__device__ __forceinline__ double coef_ld(const bf16_t* p, unsigned i) { return (double)__uint_as_float(((uint32_t)ld(p, i)) << 16); }
 __device__ __forceinline__ double coef_ld(const double* p, long i) { return p[i]; }
 __device__ __forceinline__ double coef_ld(const float* p, long i) { return (double)p[i]; }
 __device__ __forceinline__ double coef_ld(const bf16_t* p, long i) {
@@ -863,7 +860,6 @@ void launch_fill(void* x, double v, long n, bool fp64, hipStream_t s) {
     else hipLaunchKernelGGL(k_fill<float>, dim3(nblocks(n)), dim3(BS), 0, s, (float*)x, (float)v, n);
     TT_HIP(hipGetLastError());
 }
-void launch_fill_scal(void* x, long n, double v, hipStream_t s) { launch_fill(x, v, n, true, s); }
 
 // x_i uniform in [-1, 1) from a counter-based hash of (seed, i) (splitmix64 finaliser): a deterministic
 // start vector made on the device, with no host loop or copy
