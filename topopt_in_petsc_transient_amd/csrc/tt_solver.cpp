@@ -113,8 +113,8 @@ void Multigrid::build(Context* c, int nlvls, bool mixed_prec, int deg) {
     cx.alloc(nc);
     if (dense) {
         Ainv.alloc((size_t)nc * nc);
-        AinvP.alloc(sym_packed_size(nc));
-        {
+        if (nc > kDenseMvMax) {  // (up to that order the solves read the full matrix)
+            AinvP.alloc(sym_packed_size(nc));
             const long nt = (nc + 63) / 64, ntiles = nt * (nt + 1) / 2;
             sprow.alloc(ntiles * 64);
             spcol.alloc(ntiles * 64);
@@ -217,7 +217,7 @@ void Multigrid::assemble_coarse_inverse() {
     TT_HIP(hipStreamWaitEvent(s2, ev_asm, 0));
     TT_HIP(hipMemsetAsync(dinfo.p, 0, 2 * sizeof(int), s2));
     spd_inverse(Ainv.p, n, n, Winv.p);
-    launch_sym_pack(Ainv.p, n, AinvP.p, s2);
+    if (n > kDenseMvMax) launch_sym_pack(Ainv.p, n, AinvP.p, s2);
     TT_HIP(hipMemcpyAsync(info_host, dinfo.p, 2 * sizeof(int), hipMemcpyDeviceToHost, s2));
     TT_HIP(hipEventRecord(ev_inv, s2));
     inv_pending = true;
