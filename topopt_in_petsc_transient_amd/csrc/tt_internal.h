@@ -178,11 +178,6 @@ enum {
 // Elasticity operator on one level.  Coefficient storage CT is double, float or BF16.
 enum CoefKind { COEF_F64 = 0, COEF_F32 = 1, COEF_BF16 = 2 };
 
-// Batch tables of the node tiles of one grid (tt_tables.cpp; the library's kernels do not use them): per tile position (bits 0/1: the
-// first / last tile in x, bits 2/3 in y, bits 4/5 in z) the offset and batch count of its table in
-// `codes`.  A tile's table holds the elements that exist and touch one of its nodes: the first tile in
-// a direction has no elements on its low side, and the last tile owns fewer nodes than a full tile
-// when the grid's node count is not a multiple of the tile extent.
 // Element-local corner numbering of the reference (LinearElasticity.cc:3067-3074)
 __host__ __device__ constexpr int corner_id(int x, int y, int z) { return z * 4 + (y == 0 ? (x == 0 ? 0 : 1) : (x == 1 ? 2 : 3)); }
 // (i, j, k) of node or element n on an nx x ny x * grid, x fastest: two 32-bit unsigned divisions
@@ -193,7 +188,7 @@ __host__ __device__ inline void grid_ijk(unsigned n, unsigned nx, unsigned ny, i
     j = (int)(row - kk * ny);
     k = (int)kk;
 }
-// Element dof order by edges (no kernel uses it): k = 4 t + q (t = 0..5) is dof 3 a + c of corner
+// Element dof order by edges (no kernel uses it; it stays for the test of its invariants): k = 4 t + q (t = 0..5) is dof 3 a + c of corner
 // a = sens_corner(q, t >= 3), component c = t mod 3.  Lane group q owns the two x-adjacent corners of one
 // element edge (corners 0-1, 3-2, 4-5, 7-6), whose six dofs are consecutive in memory from the edge's
 // low-x node.
@@ -206,18 +201,6 @@ __host__ __device__ constexpr int sens_dof(int k) {  // k = 4 t + q -> element d
 __host__ __device__ constexpr int cx_of(int b) { return (b & 3) == 1 || (b & 3) == 2 ? 1 : 0; }
 __host__ __device__ constexpr int cy_of(int b) { return (b & 3) >= 2 ? 1 : 0; }
 __host__ __device__ constexpr int cz_of(int b) { return b >> 2; }
-
-struct BatchTab {
-    const int4* codes;
-    const int2* at;  // per position: (offset, batch count), in device memory (keeps the launch arguments small)
-};
-struct BatchTabStore {
-    DBuf<int4> buf;
-    DBuf<int2> at;
-    BatchTab t4{}, t2{};  // 8 x 8 x 4 and 8 x 8 x 2 node tiles
-};
-// tables of both tile depths for grid g, uploaded into st.buf
-void build_batch_tables(const Grid& g, BatchTabStore& st);
 
 struct OpLevel {
     Grid g;

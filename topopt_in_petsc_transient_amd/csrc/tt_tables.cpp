@@ -138,6 +138,8 @@ struct ClassBatches {
     }
 };
 
+// The tables of one tile depth, per tile position (bits 0/1: the first / last tile in x, bits 2/3 in y, bits 4/5 in z): offset
+// and batch count in `codes`.
 template <int TZ_>
 static void build_tab(const Grid& g, std::vector<int4>& codes, int2* at) {
     // owned extents of the last tile in each direction (a full extent when the node count divides)
@@ -155,19 +157,6 @@ static void build_tab(const Grid& g, std::vector<int4>& codes, int2* at) {
         at[c].x = (int)codes.size();
         at[c].y = ClassBatches<TZ_ + 1>::build(o, first, last, g.ex, g.ey, codes);
     }
-}
-
-void build_batch_tables(const Grid& g, BatchTabStore& st) {
-    std::vector<int4> codes;
-    std::vector<int2> at(128);
-    build_tab<4>(g, codes, at.data());
-    build_tab<2>(g, codes, at.data() + 64);
-    st.buf.alloc(codes.size());
-    st.at.alloc(at.size());
-    TT_HIP(hipMemcpy(st.buf.p, codes.data(), codes.size() * sizeof(int4), hipMemcpyHostToDevice));
-    TT_HIP(hipMemcpy(st.at.p, at.data(), at.size() * sizeof(int2), hipMemcpyHostToDevice));
-    st.t4 = BatchTab{st.buf.p, st.at.p};
-    st.t2 = BatchTab{st.buf.p, st.at.p + 64};
 }
 
 }  // namespace tt
