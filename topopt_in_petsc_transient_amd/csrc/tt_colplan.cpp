@@ -42,7 +42,7 @@ ColPlan make_col_plan(const Grid& g, bool fp64) {
                 const double nt = (double)tx * ty * tz, per = nt / cus;
                 const int r = (int)std::ceil(per);
                 // (between splits of one modelled time, the one with fewer blocks)
-                const double c = 1e-4 * nt + ((nk + strands - 1) / strands + 2) * (r <= resident ? plane(r) : plane(resident) * (tail + per / resident));
+                const double c = 1e-4 * nt + ((strands == 1 ? nk : (nk + strands - 1) / strands) + 2) * (r <= resident ? plane(r) : plane(resident) * (tail + per / resident));
                 if (c < cost) {
                     cost = c;
                     best = ColPlan{cx, bx, by, tx, ty, tz, strands};
