@@ -374,7 +374,7 @@ def main():
     ach = by / (fcg_ms * 1e-3) / 1e12
     roof = {"bound": "hbm", "achieved": ach, "peak": PEAK_HBM / 1e12, "unit": "TB/s",
             "frac": ach / (PEAK_HBM / 1e12), "traffic": TRAFFIC_FCG64,
-            "kernel": "k_apply_cols<double,double,true,StageOne<double>,EpiFcg> (flexible-CG apply: z staged, p = "
+            "kernel": "k_apply_cols<double,double,true,false,StageOne<double>,EpiFcg> (flexible-CG apply: z staged, p = "
                       "z + beta p_old, q = A z + beta q_old = A p, p.q partials; FP64, 128x64x64, element columns)",
             "kernel_ms": fcg_ms, "flops_per_launch": ELEM_FLOPS * nel0,
             "algorithmic_bytes_per_launch": by}
@@ -385,7 +385,7 @@ def main():
     roof["fp32_apply"] = {
         "bound": "hbm", "achieved": ach32, "peak": PEAK_HBM / 1e12, "unit": "TB/s",
         "frac": ach32 / (PEAK_HBM / 1e12), "traffic": TRAFFIC_A32,
-        "kernel": "k_apply_cols<float,float,true,StageOne<float>,EpiBC> (A u = (1+a2 beta) K u + (a5+a2 alpha) M u, "
+        "kernel": "k_apply_cols<float,float,true,false,StageOne<float>,EpiBC> (A u = (1+a2 beta) K u + (a5+a2 alpha) M u, "
                   "FP32, 128x64x64, element columns)",
         "kernel_ms": a32["fp32_ms"], "flops_per_launch": ELEM_FLOPS * nel0, "algorithmic_bytes_per_launch": by32}
     # whole-step and whole-gradient rooflines (algorithmic work x measured iterations, against the

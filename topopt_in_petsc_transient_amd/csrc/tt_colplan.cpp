@@ -16,11 +16,13 @@ namespace tt {
 // 40x40x300 17.7 -> 17.1, 12.3 -> 11.3, 23.4 -> 22.2; 128x64x64 and smaller as they were.
 // Grids of up to kBoxNodes nodes take the one-shot kernel: at 1,377 nodes (16x8x8) an FP64 apply takes 3.5 us there against
 // 5.6 us in columns, at 30,625 (48x24x24) 4.5 against 5.8 (flexible-CG apply 6.8 against 8.5, FP32 3.8 against 5.0); at
-// 70,785 (64x32x32) 6.9 against 7.1, and the flexible-CG apply 13.4 against 10.1.
+// 70,785 (64x32x32) 6.9 against 7.1, and the flexible-CG apply 13.4 against 10.1.  (Longer rods march in strands: at 60,016
+// nodes, 3x3x3750, one shot takes 4.8 us, flexible-CG apply 7.6, and strands 7.5 and 11.1; at 300,004, 1x1x75000, 50 and 226
+// against 19 and 26, every block summing all blocks' partials.)
 constexpr long kBoxNodes = 40000;
 ColPlan make_col_plan(const Grid& g, bool fp64) {
     constexpr double cus = 256.0;
-    const int resident = fp64 ? 2 : 3;  // blocks per CU
+    const int resident = fp64 ? 2 : 3;  // blocks per CU (2 in the first Chebyshev step from FP64, FP32's largest form)
     // us per plane with r blocks on the CU, and per r and 100 lines of 128 bytes touched
     const double base[3] = {fp64 ? 1.4 : 0.83, fp64 ? 1.95 : 1.03, 1.25}, lines = fp64 ? 0.17 : 0.013;
     const double tail = fp64 ? 0.3 : 0.35;  // of a full CU's plane: blocks of the last round left alone

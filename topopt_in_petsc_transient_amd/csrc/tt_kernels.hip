@@ -256,9 +256,9 @@ struct StageThree {  // wK = sum_i cK_i in_i, wM = sum_i cM_i in_i (FP64)
 // ---- epilogues.  A node's three dofs are b + i .. b + i + 2, b uniform over the block (its node plane's first dof, or
 // 0).  fetch() loads the per-node operands an epilogue reads (its Pre) for one owned node, ahead of the element
 // contraction.  put() then handles that node (inside the grid): cl are its clamped dofs, uo its input values (not
-// masked); it may add to the thread's reduction share.  prologue() runs
-// before the first put(), on every thread of a block that has a tile (block 0 always has one).  done() is called once by every thread of the block at the end
-// (reducing epilogues write their block partial there).
+// masked); it may add to the thread's reduction share.  prologue() runs before the first put(), on every thread of a block
+// that has a tile (block 0 always has one).  done() is called once by every thread of the block at the end (reducing
+// epilogues write their block partial there).
 // outputs: 2 where K and M results are taken apart (yK, yM), else yK is their sum; uses_input: whether put() reads uo.
 #define TT_NO_PRE                                                     \
     struct Pre {};                                                    \
@@ -1506,10 +1506,11 @@ void launch_axpy_multi(const Expand3& e, long n, hipStream_t s) {
 // Modified Gram-Schmidt in passes over groups of vectors.  One pass subtracts the current group (its coefficients from
 // the dots that the previous pass left) and forms the dots of the new w with the next group, or, after the last, with
 // its own group and itself.  With D_i = w.v_i at the group's start, the coefficients one after the other are
-// h_i = D_i - sum_{j < i} h_j (v_j.v_i): exactly those of subtracting v_0, v_1, ... in turn, with the stored dots
-// of the group's vectors.  HBM bound: (2 + group + next group) vectors a pass, against a dot product, a host round trip
-// and an update (5 vectors and ~28 us) per vector before: an Arnoldi step of 16 vectors at 128x64x64 takes 90
-// instead of 450 us.
+// h_i = D_i - sum_{j < i} h_j (v_j.v_i): those of subtracting v_0, v_1, ... in turn up to rounding (in exact arithmetic
+// the same; D_i is taken before the group's own vectors are subtracted), with the stored dots of the group's vectors.
+// Bound by memory: (2 + group + next group) vectors a pass, 30 us at 128x64x64 (7.8 TB/s, above the 6.5 of a copy: the last
+// level of cache holds part of them), against a dot product, a host round trip and an update (5 vectors and ~28 us) per
+// vector before: an Arnoldi step of 16 vectors takes 90 instead of 450 us.
 constexpr int MG = kMgsGroup, MB = kMgsBlocks, MT = 512;
 static_assert(MT / 64 == MG, "one wave sums one entry");
 // entry q of the MB partial rows, summed by wave q (fixed order), into d[q]; entry MG by wave 0
@@ -1686,8 +1687,8 @@ void launch_fcg_init(Reducer& red, int bb_region, int rr_region, double rtol2, b
 // <= (rtol ||b||)^2, SC_DONE is set and alpha is 0 for the rest of the solve, so x is frozen at the first iteration that
 // met the tolerance; a frozen solve keeps x and r as they are.  Block 0 writes the scalars: what other blocks read of
 // them gives the same decision before and after that write (SC_DONE is only ever set to what they find themselves).
-// HBM bound: 6 vectors, 14 us at 128x64x64 (with r_prev written as a 7th vector, which z.q_old makes unnecessary, and
-// a one-block kernel for alpha before it: 17 + 4.7 us).
+// HBM bound: 6 vectors, 16 us at 128x64x64 (4.9 TB/s; with r_prev written as a 7th vector, which z.q_old makes unnecessary,
+// and a one-block kernel for alpha before it: 17 + 4.7 us).
 template <bool JAC>
 __global__ __launch_bounds__(BS) void k_fcg_update(double* __restrict__ x, const double* __restrict__ p,
                                                    double* __restrict__ r, const double* __restrict__ q, long n,
