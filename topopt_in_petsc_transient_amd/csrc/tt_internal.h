@@ -112,9 +112,11 @@ void upload_modes(const double* ke, const double* m8, DBuf<ModeConst<double>>& d
 // The tile split of one grid for the column kernels (tt_apply_cols.inc): columns of elements per tile row
 // (bx + 1) and owned node columns per tile in x and y; tiles (the nz node planes are split evenly over tz).  cx = 0: a
 // small grid, for the one-shot kernel (tt_apply_box.inc), whose tiles are 4 x 4 x 4 nodes.
-struct ColPlan {
+struct ColTile {
     int cx, bx, by;
     int tx, ty, tz;
+};
+struct ColPlan : ColTile {
     int strands = 1;  // parts of a block's planes that march side by side (a rod's tile: its whole cross-section)
     int ntiles() const { return tx * ty * tz; }
     // blocks of a launch (column kernel: rounded up to a multiple of 8 for the XCD-aware tile order)

@@ -640,8 +640,8 @@ static int launch_cols_ct(const OpLevel& L, double cK, double cM, const Stage& s
     }
     const int nb = 8 * ((p.ntiles() + 7) / 8);
     auto launch = [&](auto kernel) {
-        hipLaunchKernelGGL(kernel, dim3(nb), dim3(256), 0, s, gargs(L.g), p, mc, (const CT*)L.kf, (const CT*)L.mf, (T)cK,
-                           (T)cM, L.mask, cs.bc, st, epi);
+        hipLaunchKernelGGL(kernel, dim3(nb), dim3(256), 0, s, gargs(L.g), (const ColTile&)p, mc, (const CT*)L.kf,
+                           (const CT*)L.mf, (T)cK, (T)cM, L.mask, cs.bc, st, epi, p.strands);
     };
     if (p.strands > 1) launch(k_apply_cols<T, CT, MASKIN, true, Stage, Epi>);
     else launch(k_apply_cols<T, CT, MASKIN, false, Stage, Epi>);
